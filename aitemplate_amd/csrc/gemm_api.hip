@@ -157,6 +157,38 @@ int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64
   return best;
 }
 
+// The heuristic's answer for a problem, kept per thread for the problems last seen: scoring every instance takes
+// 1.7 us of host time, as long as launching a small kernel, and a program calls with few distinct problems.  A
+// direct-mapped table: a problem that maps to an occupied entry takes its place.
+struct HeuristicKey {
+  const GemmAlgo* table;
+  int64_t batch, M, N, K, lda, ldb;
+  int32_t align_bytes, layout, has_workspace, cus;
+  bool operator==(const HeuristicKey& o) const {
+    return table == o.table && batch == o.batch && M == o.M && N == o.N && K == o.K && lda == o.lda && ldb == o.ldb &&
+        align_bytes == o.align_bytes && layout == o.layout && has_workspace == o.has_workspace && cus == o.cus;
+  }
+};
+int remembered_heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t lda,
+                         int64_t ldb, int align_bytes, int layout, bool has_workspace) {
+  constexpr int kEntries = 256;
+  struct Entry {
+    HeuristicKey key{};
+    int algo = -1;
+  };
+  static thread_local Entry entries[kEntries];
+  const HeuristicKey key{t.algos, batch, M, N, K, lda, ldb, align_bytes, layout, has_workspace ? 1 : 0, current_device_cus()};
+  uint64_t h = reinterpret_cast<uint64_t>(t.algos);
+  for (int64_t v : {batch, M, N, K, lda, ldb, (int64_t)(align_bytes * 8 + layout * 2 + key.has_workspace)})
+    h = (h ^ (uint64_t)v) * 0x9e3779b97f4a7c15ull;
+  Entry& e = entries[h >> 56];
+  if (!(e.key == key)) {
+    e.algo = heuristic(t, batch, M, N, K, lda, ldb, align_bytes, layout, has_workspace);
+    e.key = key;
+  }
+  return e.algo;
+}
+
 int run_gemm(int epilogue, int dtype, int algo, const GemmParams& p, hipStream_t stream) {
   const GemmAlgoTable t = gemm_table(epilogue, dtype);
   if (t.count == 0) return fail("aitamd_gemm: no kernels compiled for epilogue %d dtype %d", epilogue, dtype);
@@ -179,10 +211,10 @@ int run_gemm(int epilogue, int dtype, int algo, const GemmParams& p, hipStream_t
     if (a2 < align) align = a2;
   }
   if (algo < 0) {
-    algo = heuristic(t, p.batch, p.M, p.N, p.K, p.lda, p.ldb, align, p.layout, p.ws != nullptr && p.perm_on == 0);
+    algo = remembered_heuristic(t, p.batch, p.M, p.N, p.K, p.lda, p.ldb, align, p.layout, p.ws != nullptr && p.perm_on == 0);
     // (the heuristic prices stream-K on the grid it would get; a buffer too small for that falls back)
     if (algo >= 0 && t.algos[algo].workspace_bytes && t.algos[algo].workspace_bytes(p) > p.ws_bytes)
-      algo = heuristic(t, p.batch, p.M, p.N, p.K, p.lda, p.ldb, align, p.layout, false);
+      algo = remembered_heuristic(t, p.batch, p.M, p.N, p.K, p.lda, p.ldb, align, p.layout, false);
     if (algo < 0) return fail("aitamd_gemm: no instance supports M=%d N=%d K=%d", p.M, p.N, p.K);
   }
   if (algo >= t.count) return fail("aitamd_gemm: algo %d out of range (have %d)", algo, t.count);
