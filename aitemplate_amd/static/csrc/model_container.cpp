@@ -108,10 +108,10 @@ ModelBase* ModelContainer::GetAvailableModel() {
   }
 }
 
-void ModelContainer::ReturnModel(ModelBase* m, bool failed) {
+void ModelContainer::ReturnModel(ModelBase* m, bool idle) {
   {
     std::lock_guard<std::mutex> lk(pool_mutex_);
-    if (failed)
+    if (idle)
       available_.push_back(m);
     else
       pending_.push_back(m);
@@ -155,7 +155,11 @@ void ModelContainer::PrepareForRun(ModelBase* m, const AITData* inputs, size_t n
     }
     m->SetOutput(outputs[i].ptr, i);
   }
-  for (const auto& kv : unbound_ptrs_[0]) m->SetConstant(kv.first.c_str(), kv.second);
+  // (a lookup by name each: only after a binding has changed)
+  if (m->bound_constants_version != constants_version_) {
+    for (const auto& kv : unbound_ptrs_[0]) m->SetConstant(kv.first.c_str(), kv.second);
+    m->bound_constants_version = constants_version_;
+  }
 }
 
 void ModelContainer::Run(const AITData* inputs, size_t num_inputs, AITData* outputs, size_t num_outputs,
@@ -164,17 +168,18 @@ void ModelContainer::Run(const AITData* inputs, size_t num_inputs, AITData* outp
   ModelBase* m = GetAvailableModel();
   try {
     PrepareForRun(m, inputs, num_inputs, outputs, num_outputs);
-    m->Run(stream, graph_mode);
+    // a run that is waited for here needs no completion marker: the runtime is idle when it is given back
+    m->Run(stream, graph_mode, /*mark_finished=*/!sync);
+    if (output_shapes_out != nullptr) {
+      for (size_t i = 0; i < num_outputs; ++i)
+        if (output_shapes_out[i] != nullptr) m->GetOutputShape(i, output_shapes_out[i]);
+    }
+    if (sync) AIT_DEVICE_CHECK(hipStreamSynchronize(stream));
   } catch (...) {
-    ReturnModel(m, /*failed=*/true);
+    ReturnModel(m, /*idle=*/true);
     throw;
   }
-  if (output_shapes_out != nullptr) {
-    for (size_t i = 0; i < num_outputs; ++i)
-      if (output_shapes_out[i] != nullptr) m->GetOutputShape(i, output_shapes_out[i]);
-  }
-  ReturnModel(m, /*failed=*/false);
-  if (sync) AIT_DEVICE_CHECK(hipStreamSynchronize(stream));
+  ReturnModel(m, /*idle=*/sync);
 }
 
 void ModelContainer::RunWithOutputsOnHost(const AITData* inputs, size_t num_inputs, AITData* outputs,
@@ -254,12 +259,12 @@ float ModelContainer::BenchmarkImpl(const AITData* inputs, size_t num_inputs, AI
     AIT_DEVICE_CHECK(hipEventSynchronize(e1));
     AIT_DEVICE_CHECK(hipEventElapsedTime(&ms, e0, e1));
   } catch (...) {
-    ReturnModel(m, /*failed=*/true);
+    ReturnModel(m, /*idle=*/true);
     hipEventDestroy(e0);
     hipEventDestroy(e1);
     throw;
   }
-  ReturnModel(m, /*failed=*/false);
+  ReturnModel(m, /*idle=*/false);
   hipEventDestroy(e0);
   hipEventDestroy(e1);
   return count ? ms / count : 0.f;
@@ -365,6 +370,7 @@ void ModelContainer::SetConstant(const char* name, const AITData& tensor, bool u
     return;
   }
   unbound_ptrs_[use_inactive_set ? 1 : 0][c.name] = tensor.ptr;
+  ++constants_version_;
 }
 
 // Caller holds constants_mutex_ exclusively, so no Run() can start meanwhile.
@@ -407,6 +413,7 @@ void ModelContainer::SwapConstants() {
   std::unique_lock<std::shared_mutex> lk(constants_mutex_);
   // entries staged in the inactive set replace the active ones; unstaged names keep their binding
   for (auto& kv : unbound_ptrs_[1]) std::swap(unbound_ptrs_[0][kv.first], kv.second);
+  ++constants_version_;
   if (staged_blob_in_use_) {
     // the staged blob becomes the one every runtime reads; the old one is the next staging area
     WaitForAllModels();

@@ -104,6 +104,8 @@ class ModelBase {
   uint8_t* GetConstantsBlob() const { return constants_; }
   void SetConstantsBlob(uint8_t* base);
 
+  uint64_t bound_constants_version = 0;  // the container's set of constant bindings this runtime holds
+
  protected:
   // generated
   virtual void SetUpInputsOutputs() = 0;

@@ -69,7 +69,8 @@ class ModelContainer {
  private:
   ModelBase* GetAvailableModel();
   void ReclaimFinishedModels(std::unique_lock<std::mutex>& lk);
-  void ReturnModel(ModelBase* m, bool failed);
+  // `idle`: nothing of the runtime is in flight any more (it was waited for, or its run failed)
+  void ReturnModel(ModelBase* m, bool idle);
   void PrepareForRun(ModelBase* m, const AITData* inputs, size_t num_inputs, AITData* outputs, size_t num_outputs);
   const ConstantMeta& FindConstant(const char* name) const;
   void WaitForAllModels();
@@ -90,6 +91,7 @@ class ModelContainer {
   std::shared_mutex constants_mutex_;
   // unbound constants: [0] is the active set, [1] the set SwapConstants() activates
   std::unordered_map<std::string, const void*> unbound_ptrs_[2];
+  uint64_t constants_version_ = 1;  // of unbound_ptrs_[0]: a runtime whose bindings are older takes them over
 };
 
 }  // namespace ait
