@@ -92,17 +92,17 @@ struct AttnTile {
   static_assert(NG == 1 || (16 * OT + 2) * NW * 64 * 4 <= kLdsBytes, "the merge goes through the ring's memory");
 };
 
-// LDS transpose read: 4 x 16-bit per lane, gathered across the 16 lanes of a block
+// LDS transpose read: 4 x 16-bit per lane, gathered across the 16 lanes of a block (__restrict__: see tr_read16)
 template <class T>
 struct AttnVec;
 template <>
 struct AttnVec<f16> {
   typedef __fp16 raw4 __attribute__((__vector_size__(4 * sizeof(__fp16))));
-  static AITAMD_DEVICE f16x4 tr_read(const f16* p) {
+  static AITAMD_DEVICE f16x4 tr_read(const f16* __restrict__ p) {
     const raw4 r = __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) raw4*)p);
     return __builtin_bit_cast(f16x4, r);
   }
-  static AITAMD_DEVICE f16x4 tr_read(__attribute__((address_space(3))) const f16* p) {
+  static AITAMD_DEVICE f16x4 tr_read(__attribute__((address_space(3))) const f16* __restrict__ p) {
     const raw4 r = __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) raw4*)p);
     return __builtin_bit_cast(f16x4, r);
   }
@@ -110,11 +110,11 @@ struct AttnVec<f16> {
 template <>
 struct AttnVec<bf16> {
   typedef __bf16 raw4 __attribute__((__vector_size__(4 * sizeof(__bf16))));
-  static AITAMD_DEVICE bf16x4 tr_read(const bf16* p) {
+  static AITAMD_DEVICE bf16x4 tr_read(const bf16* __restrict__ p) {
     const raw4 r = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) raw4*)p);
     return __builtin_bit_cast(bf16x4, r);
   }
-  static AITAMD_DEVICE bf16x4 tr_read(__attribute__((address_space(3))) const bf16* p) {
+  static AITAMD_DEVICE bf16x4 tr_read(__attribute__((address_space(3))) const bf16* __restrict__ p) {
     const raw4 r = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) raw4*)p);
     return __builtin_bit_cast(bf16x4, r);
   }
