@@ -84,7 +84,8 @@ hipError_t launch_attention(const AttnParams& p, hipStream_t stream) {
                                    hipFuncAttributeMaxDynamicSharedMemorySize, Tile::kLdsBytes);
   });
   if (attr_err != hipSuccess) return attr_err;
-  const int64_t m_tiles = (p.M + Tile::BM - 1) / Tile::BM;
+  int64_t m_tiles = (p.M + Tile::BM - 1) / Tile::BM;
+  if (p.paired) m_tiles = (m_tiles + 1) / 2;
   dim3 grid((unsigned)m_tiles, (unsigned)(p.B < 65535 ? p.B : 65535), 1);
   hipLaunchKernelGGL(kernel, grid, dim3(Tile::NT), Tile::kLdsBytes, stream, p);
   return hipGetLastError();
@@ -206,6 +207,26 @@ int attention_entry(const char* who, int dtype, const void* q, const void* k, co
   // 128-row grid is too large for the rule above): 5-10 % faster on 4 x 16384^2, 8 x 8192^2, 16 x 4096^2, 32 x 2048^2;
   // no gain from 512 workgroups on
   if (mode == 0 && dma && groups_pay && (16 * ks + 32 * ot) <= 128 && ((M + 255) / 256) * B <= 256) mode = 2;
+  // Causal: a workgroup's work grows with its rows' position.  Pairs of query tiles, the last with the first and so on,
+  // are all the same length: taken by one workgroup each where they fill the chip twice over in 128-row form (two
+  // workgroups per CU) or once in the two-group form, and where there are enough tiles that an odd one in the middle
+  // is no matter.  Otherwise the longest go first, in 128-row workgroups (256 rows waste more above the diagonal).
+  // us, head dim 128, in order / longest first / pairs: 2 x 16 x 4096 237 / 210 / 177, 1 x 16 x 4096 - / 143 / 95,
+  // 16 x 16 x 1024 156 / 153 / 130; pairs of a three-tile sequence (64 x 12 x 384) 113 against 97, of 288 pairs (3 x 8 x
+  // 3000) 120 against 96.
+  if (causal && dma) {
+    const int64_t t = (M + 127) / 128, pairs = (t + 1) / 2 * B;
+    mode = groups_pay && t * B <= 256 ? 3 : 0;
+    if (B <= 65535 && (t % 2 == 0 || t >= 9)) {
+      if (pairs >= 512) {
+        p.paired = 1;
+        mode = 0;
+      } else if (groups_pay && t >= 8 && pairs >= 192 && pairs <= 256) {
+        p.paired = 1;
+        mode = 3;
+      }
+    }
+  }
   // aitamd_attention_set_variant(0|1|2|3) forces a variant where the shape allows it (a test and measurement knob)
   {
     const int m = forced_variant();

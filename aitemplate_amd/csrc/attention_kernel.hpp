@@ -56,6 +56,8 @@ struct AttnParams {
   const int32_t* q_len;
   // Non-zero: a NaN score counts as -inf (its key is left out of the row's softmax) instead of making the row NaN.
   int32_t nan_reset;
+  // Non-zero (causal): the grid has half the query tiles, and a workgroup takes the i-th from the end and then the i-th.
+  int32_t paired;
 };
 
 // NW_ waves (32 query rows each) share the K / V tiles; NS_ LDS stages.  The register-staged
@@ -203,22 +205,30 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
   const int h = lane >> 5;
   // Workgroup -> (query tile, batch entry).  The hardware deals consecutive workgroup ids round-robin over the
   // 8 XCDs, each with its own L2; dealt plainly, the workgroups of one batch entry land on all of them and every
-  // L2 fetches that entry's K and V.  When the grid divides evenly, XCD x takes the x-th eighth of the
-  // (batch entry, query tile) pairs instead, so the workgroups that stream the same K / V share one L2.
+  // L2 fetches that entry's K and V.  Instead XCD x works through the batch entries x, x + 8, x + 16, ... one after
+  // the other, so the workgroups that stream the same K / V share one L2.  (Eighths of consecutive entries share as
+  // well, but give whole XCDs the long or the short sequences where lengths follow the batch order: 64 x 12 x 384
+  // with lengths spread from all to a quarter of the keys ran in 53 us so, against 46.)  The up to seven entries
+  // that are left over go round the XCDs tile by tile.
+  // Causal: the longest rows first, so that the short ones fill the end of the launch.
   int bx = blockIdx.x, by = blockIdx.y;
-  {
-    const int total = gridDim.x * gridDim.y;
-    if ((int)gridDim.y == p.B && (total & 7) == 0) {
-      const int id = blockIdx.x + gridDim.x * blockIdx.y;
-      const int v = (id & 7) * (total >> 3) + (id >> 3);
-      by = v / (int)gridDim.x;
-      bx = v - by * (int)gridDim.x;
+  if ((int)gridDim.y == p.B) {
+    const int id = blockIdx.x + gridDim.x * blockIdx.y;
+    const int tiles = gridDim.x, even = p.B & ~(kNumXcd - 1);
+    if (id < even * tiles) {
+      const int slot = id / kNumXcd, entry = slot / tiles;
+      by = entry * kNumXcd + id % kNumXcd;
+      bx = slot - entry * tiles;
     }
+    if (p.causal) bx = tiles - 1 - bx;
   }
-  const int m0 = bx * Tile::BM;
-  const int q_row = m0 + wave * 32 + r32;  // this lane's query row
+  const int m_tiles = (p.M + Tile::BM - 1) / Tile::BM;
+  const int first_tile = p.paired ? m_tiles - 1 - ((int)gridDim.x - 1 - bx) : bx;
+  const int passes = p.paired && 2 * first_tile != m_tiles - 1 ? 2 : 1;
 
-  for (int b = by; b < p.B; b += gridDim.y) {
+  for (int b = by, pass = 0; b < p.B; pass = pass + 1 < passes ? pass + 1 : 0, b += pass == 0 ? gridDim.y : 0) {
+    const int m0 = (pass == 0 ? first_tile : m_tiles - 1 - first_tile) * Tile::BM;
+    const int q_row = m0 + wave * 32 + r32;  // this lane's query row
     const T* Qb = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.M * p.K;
     const T* Kb = reinterpret_cast<const T*>(p.k) + (int64_t)b * p.N * p.K;
     const T* Vb = reinterpret_cast<const T*>(p.v) + (int64_t)b * p.N * p.O;
@@ -686,6 +696,9 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
       }
     }
 
+    // the tiles issued past the last one: nothing may be landing when the workgroup ends or the stages are refilled
+    // (waited for ahead of the stores, which nobody waits for)
+    if constexpr (DMA) attn_wait_vmcnt<0>();
     // ---- normalise and store permuted: out[b / G][m][b % G][o]
     const float l_tot = sum_across_halves(l_run);
     const float inv = (l_tot > 0.0f && q_row < m_rows) ? 1.0f / l_tot : 0.0f;
@@ -710,8 +723,7 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
           }
         }
     }
-    if constexpr (DMA) attn_wait_vmcnt<0>();  // the zero-fill tiles issued past the last one
-    __syncthreads();  // LDS stage 0 is refilled by the next batch iteration
+    __builtin_amdgcn_s_barrier();  // every wave has left the stages that the next iteration refills
   }
 }
 

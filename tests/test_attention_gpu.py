@@ -291,3 +291,22 @@ def test_nan_key_and_lengths_at_head_dim_40(attn_variant):
         torch.testing.assert_close(got, want, atol=TOL, rtol=TOL)
         _check_mem_eff(3, 4, 150, 333, 40, 40, [333, 1, 200], causal=False)
         _check_mem_eff(3, 4, 150, 150, 40, 40, [150, 0, 77], causal=True, lens_q=[150, 10, 0])
+
+
+# causal workgroups in pairs of query tiles (an even and an odd number of tiles, both workgroup forms, the last rows cut
+# off), and the two cases on either side of the rule
+@pytest.mark.parametrize("batch,heads,S,d", [(43, 12, 256, 64), (43, 12, 200, 40), (16, 13, 1030, 64), (8, 8, 1024, 32),
+                                             (26, 8, 1100, 64), (43, 12, 300, 64), (2, 8, 1000, 64)])
+def test_causal_pairs_of_query_tiles(batch, heads, S, d):
+    print(f"case causal batch={batch} heads={heads} S={S} d={d}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v = (torch.randn(batch, heads, S, d, generator=g, device="cuda").half() for _ in range(3))
+    got = eager.mem_eff_attention(q, k, v, causal=True)
+    # every entry against torch on the first and the last batch, in fp32 on the CPU
+    for b in (0, batch - 1):
+        want = oracle.torch_mem_eff_attention(q[b:b + 1].cpu(), k[b:b + 1].cpu(), v[b:b + 1].cpu(), True).half().float()
+        torch.testing.assert_close(got[b:b + 1].cpu().float(), want, atol=2e-2, rtol=2e-2)
+    # and all of them against the unpaired rows of a shorter call: row m depends on keys 0 .. m alone
+    short = S // 3
+    part = eager.mem_eff_attention(q[:, :, :short].contiguous(), k[:, :, :short].contiguous(), v[:, :, :short].contiguous(), causal=True)
+    torch.testing.assert_close(got[:, :short].float(), part.float(), atol=2e-3, rtol=2e-2)
