@@ -134,6 +134,19 @@ AITAMD_DEVICE uint16_t buffer_load_2B(__amdgpu_buffer_rsrc_t r, uint32_t voffset
   return __builtin_amdgcn_raw_buffer_load_b16(r, voffset, 0, 0);
 }
 
+// A vector at an address of element alignment: one load or store (the gfx950 target reads and writes global memory
+// at any alignment)
+template <class V, class T>
+AITAMD_DEVICE V load_vec(const T* p) {
+  V v;
+  __builtin_memcpy(&v, p, sizeof(V));
+  return v;
+}
+template <class V, class T>
+AITAMD_DEVICE void store_vec(T* p, V v) {
+  __builtin_memcpy(p, &v, sizeof(V));
+}
+
 // Clamp a 64-bit byte count into the 32-bit num_records field.
 AITAMD_DEVICE uint32_t clamp_records(int64_t bytes) {
   return bytes <= 0 ? 0u : (bytes >= 0x7fffffffll ? 0x7fffffffu : (uint32_t)bytes);

@@ -62,35 +62,6 @@ int ptr_align(const void* p) {
   return a;
 }
 
-// Pick the instance that minimises an estimate of run time.  Work is dealt in
-// rounds of (256 CUs x workgroups per CU) tiles; a tile costs its MFMA work
-// (K plus a K-equivalent for prologue + epilogue) divided by a per-instance
-// efficiency taken from measured large-GEMM rates on MI355X.
-double instance_efficiency(const GemmAlgo& a) {
-  const int area = a.bm * a.bn;
-  if (a.direct_lds && a.kvec != 8) {
-    // dword-aligned rows: every 16-byte piece of a slab straddles two 16-byte lines of the L1 (measured rates)
-    GemmAlgo twin = a;
-    twin.kvec = 8;
-    return 0.9 * instance_efficiency(twin);
-  }
-  if (a.direct_lds) {
-    if (area >= 256 * 256) return a.direct_lds == 2 ? 1.03 : (a.threads == 512 ? 1.00 : 0.97);
-    if (area >= 256 * 192) return 0.88;
-    if (area >= 192 * 192) return 0.82;
-    if (area >= 256 * 128) return 0.86;
-    if (area >= 128 * 192) return 0.75;
-    if (area >= 128 * 128) return a.bk == 64 ? 0.70 : (a.wgs_per_cu >= 4 ? 0.72 : 0.80);
-    return area >= 64 * 64 ? 0.55 : 0.45;
-  }
-  // the register-staged instances are there for the alignments the 16-byte direct loads cannot take; where both
-  // qualify the direct-to-LDS instance of the same size is faster
-  const double narrow = a.kvec == 8 ? 1.0 : a.kvec / 10.0;
-  if (area >= 128 * 128) return 0.50 * narrow;
-  if (area >= 128 * 64) return 0.42 * narrow;
-  return 0.40 * narrow;
-}
-
 // workgroups per tile of a split-K instance on this problem (the launcher's rule, gemm_inst.hip)
 int split_factor(const GemmAlgo& a, int64_t batch, int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t tiles = ((M + a.bm - 1) / a.bm) * ((N + a.bn - 1) / a.bn) * (batch > 0 ? batch : 1);
@@ -98,57 +69,55 @@ int split_factor(const GemmAlgo& a, int64_t batch, int64_t M, int64_t N, int64_t
   return split_k_rule(tiles, k_tiles, cus);
 }
 
+// The instance with the smallest estimate of run time, from the measured figures that gemm_tiles.inc gives for each.
+// Work is dealt in rounds of (CUs x workgroups per CU) tiles.  A CU with n workgroups takes n times an instance's
+// slab time for a slab of each, but no less than the slab takes a workgroup that is alone there (it is then waiting
+// for memory); a tile adds its fill and its epilogue.  The time that memory takes for the operands and the result goes on
+// beside that: the longer of the two counts, and three tenths of the shorter.  Over 1000 problems the choice is 1.6 %
+// (odd K) to 4.5 % (batched products with both operands transposed) slower than the best instance on average; the
+// differences between runs of a launch of a few us are a good part of that.
 int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
               int align_bytes, int layout = 0, bool has_workspace = false) {
   int best = -1;
   double best_cost = 0;
   const int kNumCu = current_device_cus();  // what the launcher sizes grids and split factors with
+  const int64_t batches = batch > 0 ? batch : 1;
+  const double memory_us = 2.0 * (double)batches * (double)(M * K + N * K + M * N) / 5.5e6;
   for (int i = 0; i < t.count; ++i) {
     const GemmAlgo& a = t.algos[i];
     if (!algo_supported(a, M, N, K, lda, ldb, align_bytes, layout)) continue;
-    int64_t k_eff = K;  // depth of one workgroup's share of a tile
-    double fix_up = 0.0;
+    // (the dword-aligned twins of the direct-to-LDS tiles are for what the 16-byte ones cannot take)
+    if (a.kvec == 2 && (a.direct_lds & 5) != 0 && align_bytes >= 16 && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0) continue;
+    int64_t slabs = ((a.kvec == 2 && a.direct_lds != 8 ? K & ~7ll : K) + a.bk - 1) / a.bk;
+    int64_t tiles = ((M + a.bm - 1) / a.bm) * ((N + a.bn - 1) / a.bn) * batches;
+    double cost = a.cost.start;
     if (a.direct_lds == 4) {
       // split-K: usable with scratch memory, and worth a table entry of its own only where it does split (it is
-      // the plain instance otherwise).  Every workgroup multiplies K / s; the exchange of partial tiles through memory costs
-      // about 4.5 us whatever the tile (store, count, load: three trips to memory), some 1200 K-equivalents.
+      // the plain instance otherwise).  Every workgroup multiplies K / s; the exchange of partial tiles through
+      // memory is three trips to it (store, count, load) and s partial tiles to add.
       const int s_k = split_factor(a, batch, M, N, K, kNumCu);
       if (!has_workspace || s_k <= 1 || layout != 0) continue;
-      k_eff = (K + s_k - 1) / s_k;
-      fix_up = 1200.0 + 60.0 * s_k;
+      slabs = (slabs + s_k - 1) / s_k;
+      tiles *= s_k;
+      cost += 1.5 + (a.bm * a.bn >= 128 * 128 ? 0.65 : 0.33) * s_k;
     }
-    const int64_t tiles = ((M + a.bm - 1) / a.bm) * ((N + a.bn - 1) / a.bn) * (batch > 0 ? batch : 1) *
-        (a.direct_lds == 4 ? split_factor(a, batch, M, N, K, kNumCu) : 1);
     const int per_cu = a.wgs_per_cu > 0 ? a.wgs_per_cu : 1;
     const int64_t slots = (int64_t)kNumCu * per_cu;
     const int64_t rounds = (tiles + slots - 1) / slots;
-    // the last, partly filled round still runs its busiest CU at full length unless
-    // fewer than one tile per CU is left
     const int64_t last = tiles - (rounds - 1) * slots;
-    const int64_t busiest = last >= kNumCu ? (last + kNumCu - 1) / kNumCu : 1;  // workgroups on the busiest CU
-    double last_frac = (double)busiest / per_cu;
-    // a four-wave workgroup of a large tile alone on its CU (one wave per SIMD) multiplies at about 70 % of the rate
-    // that two interleaved waves per SIMD reach (the small tiles' efficiencies were measured in that state)
-    if (busiest == 1 && per_cu > 1 && a.threads == 256 && a.bm * a.bn >= 128 * 128) last_frac = 1.4 / per_cu;
+    const int64_t busiest = (last + kNumCu - 1) / kNumCu;  // workgroups on the busiest CU in the last round
+    // a tile wider or taller than the whole problem fetches only the rows that exist
+    const double live = (double)((M < a.bm ? M : a.bm) + (N < a.bn ? N : a.bn)) / (a.bm + a.bn);
+    const double fetch = a.cost.fetch * live;
+    const double slab = fetch > a.cost.mult ? fetch : a.cost.mult;
+    auto round_us = [&](double n) {
+      const double full = n * slab;
+      return (double)slabs * (full > a.cost.alone ? full : a.cost.alone) + n * a.cost.tile;
+    };
     // the persistent kernel splits the tiles of a last round that would leave half the CUs idle over two CUs each
-    if (a.direct_lds == 2 && rounds > 1 && 2 * last <= kNumCu) last_frac = 0.72;
-    // with one or two K-slabs per tile a CU is latency-bound: four resident workgroups hide each
-    // other's fill and store phases (measured on the B=768 M=N=384 K=64 batched shape)
-    // (the register-staged instances do not overlap a tile's fill with its neighbours' stores that way)
-    const double k_over = (K <= 128 && per_cu >= 4 && a.direct_lds) ? 200.0 : 320.0;
-    // a tile wider or taller than the whole problem multiplies its full area, but fetches, converts and stores only
-    // the part that exists
-    const double area = (double)a.bm * a.bn;
-    const double live = (double)(M < a.bm ? M : a.bm) * (double)(N < a.bn ? N : a.bn);
-    // a CU fetches operand bytes at no more than 64 per clock whatever the tile (measured: M=256 N=1024 at
-    // K = 64 ... 4096 costs 0.19 us per 64-deep slab of a 64x64 tile, from the L2 as from HBM), i.e. some 60
-    // multiply-adds of the matrix unit per fetched element (fitted on 18 shapes from 32x4096x4096 to 8192x1024x1024
-    // timed over every instance: the pick is within 17 % of the best everywhere, 3 % on average): small tiles are
-    // bound by that, not by their MFMAs, and a thin problem wants the tile with the smallest BM + BN per CU
-    const double fetch = 60.0 * (double)((M < a.bm ? M : a.bm) + (N < a.bn ? N : a.bn)) * (double)k_eff;
-    double mult = area * (double)k_eff / instance_efficiency(a);
-    if (fetch > mult) mult = fetch;
-    const double cost = ((double)(rounds - 1) + last_frac) * per_cu * (mult + live * (k_over + fix_up) / instance_efficiency(a));
+    const double last_frac = a.direct_lds == 2 && rounds > 1 && 2 * last <= kNumCu ? 0.72 : 1.0;
+    const double work = (double)(rounds - 1) * round_us(per_cu) + last_frac * round_us((double)busiest);
+    cost += work > memory_us ? work + 0.3 * memory_us : memory_us + 0.3 * work;
     if (best < 0 || cost < best_cost) {
       best = i;
       best_cost = cost;

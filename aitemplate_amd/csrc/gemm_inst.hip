@@ -9,6 +9,7 @@
 #include "gemm_host.hpp"
 #include "gemm_kernel_dma.hpp"
 #include "gemm_kernel_persist.hpp"
+#include "gemm_kernel_rows.hpp"
 
 #ifndef AITAMD_EPI
 #error "compile with -DAITAMD_EPI=<id>"
@@ -43,9 +44,7 @@ constexpr bool kLayoutsArePermuted = AITAMD_EPI == kEpiBias;  // the bias kernel
 
 constexpr int kShortK = 4;
 template <class Tile, bool PERM, int LAYOUT>
-struct KernelOf {
-  static constexpr auto value = gemm_rcr_kernel<Elem, Tile, Epi, PERM, LAYOUT>;
-};
+struct KernelOf;
 template <int BM, int BN, int BK, int WM, int WN, int NS, int OCC, int PIPE, int MT, int AUX, int MODE, bool PERM,
           int LAYOUT>
 struct KernelOf<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX, MODE>, PERM, LAYOUT> {
@@ -58,6 +57,10 @@ struct KernelOf<GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM, PAIR>, PERM, LA
   // (LAYOUT 4 is not an operand layout: it names the instantiation for tiles of fewer K-slabs than ring stages)
   static constexpr auto value =
       gemm_rcr_persist_kernel<Elem, GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM, PAIR>, Epi, PERM, LAYOUT == kShortK>;
+};
+template <int MT, int NW, int U, int ELEM, bool PERM, int LAYOUT>
+struct KernelOf<GemmTileRows<MT, NW, U, ELEM>, PERM, LAYOUT> {
+  static constexpr auto value = gemm_rcr_rows_kernel<Elem, GemmTileRows<MT, NW, U, ELEM>, Epi, PERM>;
 };
 // the slab-pair form of a persistent tile (the tile itself where it has none)
 template <class Tile>
@@ -75,16 +78,16 @@ template <class Tile>
 struct LayoutMask {
   static constexpr int value = 1;
 };
-// the element-wide loads take every layout: the instance of last resort for pitches and K that the
-// 16-byte loads cannot take
-template <int BM, int BN, int BK, int WM, int WN>
-struct LayoutMask<GemmTile<BM, BN, BK, WM, WN, 1>> {
-  static constexpr int value = kLayoutBits;
-};
 template <int BM, int BN, int BK, int WM, int WN, int NS, int OCC, int PIPE, int MT, int AUX>
 struct LayoutMask<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX, 0>> {
   static constexpr int value =
       GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX>::kTransposable ? kLayoutBits : 1;
+};
+// (the register-staged form takes every layout, pitch and K: the instances of last resort)
+template <int BM, int BN, int BK, int WM, int WN, int NS, int OCC, int PIPE, int MT, int AUX>
+struct LayoutMask<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX, 4>> {
+  static constexpr int value =
+      GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX, 4>::kTransposable ? kLayoutBits : 1;
 };
 // split-K form: rcr only
 template <class Tile>
@@ -248,14 +251,6 @@ hipError_t launch_tile(const GemmParams& p, hipStream_t stream) {
 // Workgroups one CU can hold: limited by LDS (160 KiB) and by the register file
 // (512 VGPRs per SIMD lane shared by the waves of a SIMD).
 constexpr int kLdsPerCu = 160 * 1024;
-constexpr int staged_wgs_per_cu(int bm, int bn, int nt, int lds) {
-  const int acc = bm * bn / nt;                       // fp32 accumulators per lane
-  const int regs = acc + 96;                          // plus staging / fragments / addresses
-  const int waves_per_simd = 512 / regs > 0 ? 512 / regs : 1;
-  const int by_regs = waves_per_simd * 4 / (nt / 64) > 0 ? waves_per_simd * 4 / (nt / 64) : 1;
-  const int by_lds = kLdsPerCu / lds > 0 ? kLdsPerCu / lds : 1;
-  return by_regs < by_lds ? by_regs : by_lds;
-}
 constexpr int dma_wgs_per_cu(int nt, int occ, int lds) {
   const int waves_per_wg_per_simd = nt / 64 / 4 > 0 ? nt / 64 / 4 : 1;
   const int by_regs = occ / waves_per_wg_per_simd > 0 ? occ / waves_per_wg_per_simd : 1;
@@ -263,63 +258,51 @@ constexpr int dma_wgs_per_cu(int nt, int occ, int lds) {
   return by_regs < by_lds ? by_regs : by_lds;
 }
 
-#define AITAMD_STR2(x) #x
-#define AITAMD_STR(x) AITAMD_STR2(x)
+// Table entry of a tile.  KIND: GemmAlgo::direct_lds; OCC: workgroups per CU of the persistent and few-rows kernels,
+// waves per SIMD that the registers allow of the others.
+struct Cost {
+  float start, mult, fetch, alone, tile;
+};
+template <class Tile, int KIND, int OCC>
+constexpr GemmAlgo entry(const char* name, Cost c) {
+  constexpr bool kByRegisters = KIND != 2 && KIND != 8;
+  return {name, Tile::BM, Tile::BN, Tile::BK, Tile::NT, Tile::KVEC, Tile::kLdsBytes,
+          kByRegisters ? dma_wgs_per_cu(Tile::NT, OCC, Tile::kLdsBytes) : OCC, KIND, LayoutMask<Tile>::value, &launch_tile<Tile>,
+          KIND == 4 ? &workspace_of<Tile> : nullptr, {c.start, c.mult, c.fetch, c.alone, c.tile}};
+}
 
 const GemmAlgo kAlgos[] = {
-#define AITAMD_GEMM_TILE(BM, BN, BK, WM, WN, KV)                                              \
-  {"gemm_rcr_" AITAMD_DT_NAME "_" #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_v" #KV,                \
-   BM, BN, BK, GemmTile<BM, BN, BK, WM, WN, KV>::NT, KV, GemmTile<BM, BN, BK, WM, WN, KV>::kLdsBytes, \
-   staged_wgs_per_cu(BM, BN, GemmTile<BM, BN, BK, WM, WN, KV>::NT,                                  \
-                     GemmTile<BM, BN, BK, WM, WN, KV>::kLdsBytes),                                  \
-   0, LayoutMask<GemmTile<BM, BN, BK, WM, WN, KV>>::value, &launch_tile<GemmTile<BM, BN, BK, WM, WN, KV>>, nullptr},
-#define AITAMD_GEMM_TILE_DMA(BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX)                                 \
-  {"gemm_rcr_" AITAMD_DT_NAME "_" #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_dma" #NS "_o" #OCC "_p" #PIPE "_m" #MT \
-   "_c" #AUX,                                                                                              \
-   BM, BN, BK, GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX>::NT, 8,                             \
-   GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX>::kLdsBytes,                                     \
-   dma_wgs_per_cu(GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX>::NT, OCC,                        \
-                  GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX>::kLdsBytes),                      \
-   1, LayoutMask<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX>>::value,                            \
-   &launch_tile<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX>>, nullptr},
-#define AITAMD_GEMM_TILE_PERSIST(BM, BN, BK, WM, WN, NS, MT, LBM)                                         \
-  {"gemm_rcr_" AITAMD_DT_NAME "_" #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_persist" #NS "_m" #MT,                \
-   BM, BN, BK, GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM>::NT, 8,                                     \
-   GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM>::kLdsBytes,                                             \
-   1, 2, 1, &launch_tile<GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM>>, nullptr},
-#define AITAMD_GEMM_TILE_DMA_SPLITK(BM, BN, BK, WM, WN, NS, OCC, PIPE, MT)                                   \
-  {"gemm_rcr_" AITAMD_DT_NAME "_" #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_dma" #NS "_o" #OCC "_p" #PIPE "_m" #MT \
-   "_splitk",                                                                                             \
-   BM, BN, BK, GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 1>::NT, 8,                             \
-   GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 1>::kLdsBytes,                                     \
-   dma_wgs_per_cu(GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 1>::NT, OCC,                        \
-                  GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 1>::kLdsBytes),                      \
-   4, 1, &launch_tile<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 1>>,                             \
-   &workspace_of<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 1>>},
-#define AITAMD_GEMM_TILE_DMA_K2(BM, BN, BK, WM, WN, NS, OCC, PIPE, MT)                                      \
-  {"gemm_rcr_" AITAMD_DT_NAME "_" #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_dma" #NS "_o" #OCC "_p" #PIPE "_m" #MT \
-   "_k2",                                                                                                 \
-   BM, BN, BK, GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 2>::NT, 2,                             \
-   GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 2>::kLdsBytes,                                     \
-   dma_wgs_per_cu(GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 2>::NT, OCC,                        \
-                  GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 2>::kLdsBytes),                      \
-   1, 1, &launch_tile<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 2>>, nullptr},
-#define AITAMD_GEMM_TILE_DMA_SPLITK_K2(BM, BN, BK, WM, WN, NS, OCC, PIPE, MT)                                \
-  {"gemm_rcr_" AITAMD_DT_NAME "_" #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_dma" #NS "_o" #OCC "_p" #PIPE "_m" #MT \
-   "_k2_splitk",                                                                                          \
-   BM, BN, BK, GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 3>::NT, 2,                             \
-   GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 3>::kLdsBytes,                                     \
-   dma_wgs_per_cu(GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 3>::NT, OCC,                        \
-                  GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 3>::kLdsBytes),                      \
-   4, 1, &launch_tile<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 3>>,                             \
-   &workspace_of<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 3>>},
+#define AITAMD_NAME "gemm_rcr_" AITAMD_DT_NAME "_"
+#define AITAMD_GEMM_TILE_DMA(BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX, ...)                                        \
+  entry<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, AUX>, 1, OCC>(                                            \
+      AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_dma" #NS "_o" #OCC "_p" #PIPE "_m" #MT "_c" #AUX, {__VA_ARGS__}),
+#define AITAMD_GEMM_TILE_PERSIST(BM, BN, BK, WM, WN, NS, MT, LBM, ...)                                               \
+  entry<GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM>, 2, 1>(                                                     \
+      AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_persist" #NS "_m" #MT, {__VA_ARGS__}),
+#define AITAMD_GEMM_TILE_DMA_SPLITK(BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, ...)                                      \
+  entry<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 1>, 4, OCC>(                                           \
+      AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_dma" #NS "_o" #OCC "_p" #PIPE "_m" #MT "_splitk", {__VA_ARGS__}),
+#define AITAMD_GEMM_TILE_DMA_K2(BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, ...)                                          \
+  entry<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 2>, 1, OCC>(                                           \
+      AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_dma" #NS "_o" #OCC "_p" #PIPE "_m" #MT "_k2", {__VA_ARGS__}),
+#define AITAMD_GEMM_TILE_DMA_SPLITK_K2(BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, ...)                                   \
+  entry<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 3>, 4, OCC>(                                           \
+      AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_dma" #NS "_o" #OCC "_p" #PIPE "_m" #MT "_k2_splitk", {__VA_ARGS__}),
+#define AITAMD_GEMM_TILE_STAGED(BM, BN, BK, WM, WN, NS, OCC, MT, ...)                                                \
+  entry<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, 0, MT, 0, 4>, 0, OCC>(                                              \
+      AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_reg" #NS "_o" #OCC "_v1", {__VA_ARGS__}),
+#define AITAMD_GEMM_ROWS(MT, NW, U, ...)                                                                             \
+  entry<GemmTileRows<MT, NW, U, 0>, 8, 4>(AITAMD_NAME "rows" #MT "_n" #NW "_u" #U "_k2", {__VA_ARGS__}),             \
+  entry<GemmTileRows<MT, NW, U, 1>, 8, 4>(AITAMD_NAME "rows" #MT "_n" #NW "_u" #U "_v1", {__VA_ARGS__}),
 #include "gemm_tiles.inc"
-#undef AITAMD_GEMM_TILE
 #undef AITAMD_GEMM_TILE_DMA
-#undef AITAMD_GEMM_TILE_DMA_K2
-#undef AITAMD_GEMM_TILE_DMA_SPLITK_K2
 #undef AITAMD_GEMM_TILE_PERSIST
 #undef AITAMD_GEMM_TILE_DMA_SPLITK
+#undef AITAMD_GEMM_TILE_DMA_K2
+#undef AITAMD_GEMM_TILE_DMA_SPLITK_K2
+#undef AITAMD_GEMM_TILE_STAGED
+#undef AITAMD_GEMM_ROWS
+#undef AITAMD_NAME
 };
 
 }  // namespace

@@ -1,7 +1,6 @@
 // RCR GEMM main loop with direct global->LDS loads (buffer_load_dwordx4 ... lds)
 // and an NS-deep LDS ring, plus an LDS-transposed epilogue with 128-bit stores.
 //
-// Differences from gemm_kernel.hpp (same math, same operand layout):
 //  * A/B slabs never pass through VGPRs: each wave's load instruction fills one
 //    contiguous 1 KiB of LDS (64 lanes x 16 bytes); the XOR swizzle is applied
 //    on the *global* side by choosing which 16-byte chunk of the row each lane
@@ -31,11 +30,20 @@ namespace aitamd {
 // as they are; the K loop runs over the whole 16-byte pieces of a row, and the 2, 4 or 6 elements behind them are
 // fetched once per tile with dword loads straight into MFMA operands (lanes of the first k-chunk, zeros elsewhere)
 // and multiplied after the loop.  Nothing is read past the end of a row.
+//
+// MODE 4, element alignment: K, the pitches and the operand pointers may be anything (odd K: every other row starts
+// on an odd element).  The slabs go through registers: the same 16-byte pieces, read at 2-byte aligned addresses,
+// are written to the place in LDS where the direct load would have put them; NS - 1 slabs are on their way in
+// registers and two LDS stages alternate.  The last slab is read in whole dwords (five per piece, shifted together
+// afterwards): an element that shares its dword with the first bytes past the end of the buffer would be lost
+// otherwise, and what lies past the end of K is cleared.  (Five dwords in every slab: 2048 x 6912 x 8313 takes 352 us
+// instead of 298.)  All operand layouts.
 template <int BM_, int BN_, int BK_, int WGM_, int WGN_, int NS_, int OCC_, int PIPE_ = 0, int MT_ = 32, int AUX_ = 0,
           int MODE_ = 0>
 struct GemmTileDma {
   static constexpr int SPLITK = MODE_ & 1;          // MODE bit 0
   static constexpr int KTAIL = (MODE_ >> 1) & 1;    // MODE bit 1
+  static constexpr int STAGED = (MODE_ >> 2) & 1;   // MODE bit 2
   static constexpr int64_t kSlotBytes = (int64_t)BM_ * BN_ * 4;
   static constexpr int64_t kCounterAlign = 4096;
   // scratch bytes for `tiles` (batch x tile) pairs shared by `splits` workgroups each: one counter per pair,
@@ -55,7 +63,7 @@ struct GemmTileDma {
   static constexpr int ACC_N = MT * MT / 64;         // fp32 accumulators per lane per MFMA tile
   static constexpr int BM = BM_, BN = BN_, BK = BK_;
   static constexpr int WGM = WGM_, WGN = WGN_, NS = NS_, OCC = OCC_;
-  static constexpr int KVEC = KTAIL ? 2 : 8;
+  static constexpr int KVEC = STAGED ? 1 : (KTAIL ? 2 : 8);
   static constexpr int NW = WGM * WGN;
   static constexpr int NT = NW * kWaveSize;
   static constexpr int WTM = BM / WGM, WTN = BN / WGN;
@@ -72,7 +80,7 @@ struct GemmTileDma {
   // epilogue staging: one MT-row strip per wave, fp32, padded by 4 floats per row
   static constexpr int EPI_PITCH = WTN + 4;
   static constexpr int EPI_BYTES = NW * MT * EPI_PITCH * 4;
-  static constexpr int MAIN_BYTES = NS * STAGE_ELEMS * 2;
+  static constexpr int MAIN_BYTES = (STAGED ? 2 : NS) * STAGE_ELEMS * 2;
   static constexpr int kLdsBytes = MAIN_BYTES > EPI_BYTES ? MAIN_BYTES : EPI_BYTES;
   // operands that are not K-contiguous need whole k-rows per 1 KiB wave-load and at least 8 chunks per row
   static constexpr bool kTransposable = MT == 32 && (BM == 64 || BM == 128 || BM == 256) &&
@@ -85,6 +93,7 @@ struct GemmTileDma {
   static_assert((NS - 2) * LOADS_PER_STEP <= 63, "vmcnt field is 6 bits");
   static_assert(PIPE == 0 || (NS >= 3 && (KK == 1 || KK % 2 == 0)), "cross-slab prefetch needs 3 stages");
   static_assert(WTN % 8 == 0, "epilogue needs 8-column groups");
+  static_assert(!STAGED || (PIPE == 0 && !SPLITK && !KTAIL && NS >= 2), "the register-staged form has a loop of its own");
 };
 
 template <class Tile>
@@ -276,8 +285,13 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
     const T* Bb = reinterpret_cast<const T*>(p.b) + (int64_t)batch * p.sb + (B_T ? (int64_t)n0 : (int64_t)n0 * p.ldb);
     const int64_t bytes_a = A_T ? (((int64_t)p.K - 1) * p.lda + rows_a) * 2 : (((int64_t)rows_a - 1) * p.lda + p.K) * 2;
     const int64_t bytes_b = B_T ? (((int64_t)p.K - 1) * p.ldb + rows_b) * 2 : (((int64_t)rows_b - 1) * p.ldb + p.K) * 2;
-    const __amdgpu_buffer_rsrc_t ra = make_rsrc(Ab, clamp_records(bytes_a));
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(Bb, clamp_records(bytes_b));
+    // (staged: descriptors start at a dword and end with one, so that no element of an operand at an odd place is cut off)
+    const uint32_t odd_a = Tile::STAGED ? (uint32_t)(reinterpret_cast<uintptr_t>(Ab) & 3) : 0u;
+    const uint32_t odd_b = Tile::STAGED ? (uint32_t)(reinterpret_cast<uintptr_t>(Bb) & 3) : 0u;
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(reinterpret_cast<const char*>(Ab) - odd_a,
+                                                clamp_records(Tile::STAGED ? (bytes_a + odd_a + 3) & ~3ll : bytes_a));
+    const __amdgpu_buffer_rsrc_t rb = make_rsrc(reinterpret_cast<const char*>(Bb) - odd_b,
+                                                clamp_records(Tile::STAGED ? (bytes_b + odd_b + 3) & ~3ll : bytes_b));
 
     // Issue the wave-loads of K-slab `kt` into ring slot `stage`.  Slabs past
     // the end of K are still issued (every chunk out of range -> zero fill) so
@@ -309,6 +323,36 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
 #pragma unroll
         for (int e = 0; e < ACC_N; ++e) acc[mi][ni][e] = 0.0f;
 
+    // Epilogue coordinates.  What the epilogue reads of the bias and of the residuals of a small tile is requested
+    // here, ahead of the slabs: read after the K loop it costs a trip to memory per tile, as long as three slabs.
+    constexpr int LANES_PER_ROW = Tile::WTN / 8;             // lanes covering one strip row
+    constexpr int ROWS_PER_PASS = 64 / LANES_PER_ROW;        // rows read back per pass
+    constexpr int ACTIVE = ROWS_PER_PASS * LANES_PER_ROW;    // lanes used in a pass
+    constexpr int PASSES = (MT + ROWS_PER_PASS - 1) / ROWS_PER_PASS;
+    const int rd_row = lane / LANES_PER_ROW;
+    const int rd_col = (lane % LANES_PER_ROW) * 8;
+    const int n_epi = n0 + wn * Tile::WTN + rd_col;          // the lane's 8 columns, the same in every pass
+    const T* D0b = Epi::kNumD >= 1 ? reinterpret_cast<const T*>(p.d0) + (int64_t)batch * p.sd : nullptr;
+    const T* D1b = Epi::kNumD >= 2 ? reinterpret_cast<const T*>(p.d1) + (int64_t)batch * p.sd : nullptr;
+    const T* bias = reinterpret_cast<const T*>(p.bias);
+    auto epi_row = [&](int mi, int ps) { return m0 + wm * Tile::WTM + mi * MT + ps * ROWS_PER_PASS + rd_row; };
+    constexpr bool kEarlyBias = Epi::kHasBias && BM * BN <= 128 * 128;
+    constexpr int kEarlyD = MI * PASSES <= 2 ? MI * PASSES : 0;
+    vec8 bias_v = {}, d0_e[kEarlyD > 0 ? kEarlyD : 1] = {}, d1_e[kEarlyD > 0 ? kEarlyD : 1] = {};
+    if constexpr (kEarlyBias) {
+      if (n_epi + 8 <= p.N) bias_v = load_vec<vec8>(bias + n_epi);
+    }
+    if constexpr (kEarlyD > 0 && Epi::kNumD >= 1) {
+#pragma unroll
+      for (int i = 0; i < kEarlyD; ++i) {
+        const int m = epi_row(i / PASSES, i % PASSES);
+        if (m < p.M && n_epi + 8 <= p.N) {
+          d0_e[i] = load_vec<vec8>(D0b + (int64_t)m * p.ldd + n_epi);
+          if constexpr (Epi::kNumD >= 2) d1_e[i] = load_vec<vec8>(D1b + (int64_t)m * p.ldd + n_epi);
+        }
+      }
+    }
+
     // dword K tail: the up to three dwords behind the last whole 16-byte piece of each of the lane's operand rows,
     // requested before the slab loads (so every wait of the loop covers them) and used after the loop
     uint32_t tail_a[Tile::KTAIL ? MI : 1][3], tail_b[Tile::KTAIL ? NI : 1][3];
@@ -333,7 +377,9 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
     // the L_IT wave-loads of a slab are issued in KK equal portions, one per MFMA step
     constexpr int L_PER = (L_IT + KK - 1) / KK;
     constexpr int L_P0 = L_PER < L_IT ? L_PER : L_IT;  // size of portion 0
-    if constexpr (Tile::PIPE == 0) {
+    if constexpr (Tile::STAGED != 0) {
+      // (the staged loop fills its own pipeline)
+    } else if constexpr (Tile::PIPE == 0) {
 #pragma unroll
       for (int s = 0; s < NS - 1; ++s) issue_loads(s, s, 0, L_IT);
     } else {
@@ -374,7 +420,79 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
     // fragments are double-buffered in registers: step kk+1 is read from LDS
     // while step kk is multiplied
     vec8 af[2][MI], bf[2][NI];
-    if constexpr (Tile::PIPE == 0) {
+    if constexpr (Tile::STAGED != 0) {
+      constexpr int D = NS - 1;  // slabs on their way in registers
+      u32x4 reg[D][L_IT];
+      uint32_t fifth[L_IT] = {};  // of the last slab's pieces
+      auto is_a_load = [&](int i) { return Tile::A_LOADS % Tile::NW == 0 ? i * Tile::NW < Tile::A_LOADS : wave + i * Tile::NW < Tile::A_LOADS; };
+      // byte offset of the lane's piece i of slab kt
+      auto piece_at = [&](int kt, int i) {
+        const uint32_t step = (A_T || B_T) ? (uint32_t)(kt * BK) * l_kbytes[i] : (uint32_t)(kt * BK * 2);
+        return l_off[i] + step + (is_a_load(i) ? odd_a : odd_b);
+      };
+      auto fetch = [&](int kt, auto d_c) {
+        constexpr int d = decltype(d_c)::value;
+        const bool last = kt == k_tiles - 1;  // (wave-uniform)
+#pragma unroll
+        for (int i = 0; i < L_IT; ++i) {
+          const bool is_a = is_a_load(i);
+          uint32_t off = (kt * BK + l_chunk_k[i] < p.K) ? piece_at(kt, i) : kOobOffset;
+          if (last) {
+            off &= ~3u;
+            fifth[i] = is_a ? buffer_load_4B(ra, off + 16) : buffer_load_4B(rb, off + 16);
+          }
+          reg[d][i] = is_a ? buffer_load_16B(ra, off) : buffer_load_16B(rb, off);
+        }
+      };
+      auto put = [&](int kt, auto d_c) {
+        constexpr int d = decltype(d_c)::value;
+        T* sbase = smem + (kt & 1) * Tile::STAGE_ELEMS;
+        const bool last = kt == k_tiles - 1;
+#pragma unroll
+        for (int i = 0; i < L_IT; ++i) {
+          u32x4 v = reg[d][i];
+          if (last) {
+            // (elements of the piece that exist; the columns of a transposed operand's piece may be anything)
+            const int left = (is_a_load(i) ? A_T : B_T) ? 8 : p.K - (kt * BK + l_chunk_k[i]);
+            const uint32_t shift = (piece_at(kt, i) & 2u) * 8u;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+              const uint32_t x = __builtin_amdgcn_alignbit(w < 3 ? reg[d][i][w + 1] : fifth[i], reg[d][i][w], shift);
+              v[w] = x & (left >= 2 * w + 2 ? 0xffffffffu : (left == 2 * w + 1 ? 0xffffu : 0u));
+            }
+          }
+          *reinterpret_cast<u32x4*>(sbase + (wave + i * Tile::NW) * 512 + lane * 8) = v;
+        }
+      };
+      auto barrier = [&]() {  // this wave's LDS writes are done; the loads on their way stay there
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+      };
+      constexpr std::integral_constant<int, 0> d_0{};
+      static_for<0, D>([&](auto d) { fetch(d, d); });
+      put(0, d_0);
+      fetch(D, d_0);
+      barrier();
+      for (int kt0 = 0; kt0 < k_tiles; kt0 += D) {
+        static_for<0, D>([&](auto u) {
+          const int kt = kt0 + u;
+          if (D > 1 && kt >= k_tiles) return;
+          const T* cur = smem + (kt & 1) * Tile::STAGE_ELEMS;
+          load_frags(cur, 0, af[0], bf[0]);
+#pragma unroll
+          for (int kk = 0; kk < KK; ++kk) {
+            if (kk + 1 < KK) load_frags(cur, kk + 1, af[(kk & 1) ^ 1], bf[(kk & 1) ^ 1]);
+            mfmas(af[kk & 1], bf[kk & 1]);
+          }
+          // slab kt + 1 takes the stage of slab kt - 1, which every wave has left; its registers take slab kt + 1 + D
+          constexpr std::integral_constant<int, (decltype(u)::value + 1) % D> nx{};
+          put(kt + 1, nx);
+          fetch(kt + 1 + D, nx);
+          barrier();
+        });
+      }
+    } else if constexpr (Tile::PIPE == 0) {
       for (int kt = 0; kt < k_tiles; ++kt) {
         // slab kt has landed once at most the (NS-2) younger slabs are in flight
         wait_vmcnt<(NS - 2) * Tile::LOADS_PER_STEP>();
@@ -524,29 +642,16 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
     // ---------------- epilogue: acc -> LDS (fp32, per-wave strip) -> 16-byte stores --------
     T* Cb = reinterpret_cast<T*>(p.c) + out_batch_offset(p, batch);
     const __amdgpu_buffer_rsrc_t rc = make_rsrc(Cb, kStoreRecords);
-    const T* D0b = Epi::kNumD >= 1 ? reinterpret_cast<const T*>(p.d0) + (int64_t)batch * p.sd : nullptr;
-    const T* D1b = Epi::kNumD >= 2 ? reinterpret_cast<const T*>(p.d1) + (int64_t)batch * p.sd : nullptr;
-    const T* bias = reinterpret_cast<const T*>(p.bias);
-
-    // vector form for the lanes whose 8 columns lie inside the row: multi-dword global and buffer accesses need
-    // dword alignment only, so even pitches and 4-byte aligned pointers are enough
-    bool vec_ok = ((p.ldc & 1) == 0) && ((p.sc & 1) == 0) && (!PERM || ((p.perm_n2 & 7) == 0 && (p.N & 7) == 0)) &&
-        ((reinterpret_cast<uintptr_t>(p.c) & 3) == 0);
-    if (Epi::kHasBias) vec_ok = vec_ok && ((reinterpret_cast<uintptr_t>(p.bias) & 3) == 0);
-    if (Epi::kNumD >= 1)
-      vec_ok = vec_ok && ((p.ldd & 1) == 0) && ((p.sd & 1) == 0) && ((reinterpret_cast<uintptr_t>(p.d0) & 3) == 0);
-    if (Epi::kNumD >= 2) vec_ok = vec_ok && ((reinterpret_cast<uintptr_t>(p.d1) & 3) == 0);
+    // vector form for the lanes whose 8 columns lie inside the row, at any alignment (element by element, an odd N
+    // took 29 us where its even neighbour took 18: 2000 x 3001 x 500); the streaming stores need even pitches and a
+    // dword-aligned pointer
+    const bool vec_ok = !PERM || ((p.perm_n2 & 7) == 0 && (p.N & 7) == 0);
+    const bool stream_ok = p.nt_store != 0 && ((p.ldc & 1) == 0) && ((p.sc & 1) == 0) && ((reinterpret_cast<uintptr_t>(p.c) & 3) == 0);
 
     float one = 1.0f;
     asm volatile("" : "+s"(one));  // (opaque to the optimizer: see to_float_plus)
     constexpr int PITCH = Tile::EPI_PITCH;
     float* strip = reinterpret_cast<float*>(smem_raw) + wave * MT * PITCH;
-    constexpr int LANES_PER_ROW = Tile::WTN / 8;             // lanes covering one strip row
-    constexpr int ROWS_PER_PASS = 64 / LANES_PER_ROW;        // rows read back per pass
-    constexpr int ACTIVE = ROWS_PER_PASS * LANES_PER_ROW;    // lanes used in a pass
-    constexpr int PASSES = (MT + ROWS_PER_PASS - 1) / ROWS_PER_PASS;
-    const int rd_row = lane / LANES_PER_ROW;
-    const int rd_col = (lane % LANES_PER_ROW) * 8;
     constexpr int NG = ACC_N / 4;  // groups of 4 consecutive columns per lane per MFMA tile
 
 #pragma unroll
@@ -569,8 +674,8 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
       for (int ps = 0; ps < PASSES; ++ps) {
         const int row = ps * ROWS_PER_PASS + rd_row;
         const bool lane_on = (ACTIVE == 64 || lane < ACTIVE) && (MT % ROWS_PER_PASS == 0 || row < MT);
-        const int m = m0 + wm * Tile::WTM + mi * MT + row;
-        const int n = n0 + wn * Tile::WTN + rd_col;
+        const int m = epi_row(mi, ps);
+        const int n = n_epi;
         if (lane_on && m < p.M && n < p.N) {
           const f32x4 v0 = *reinterpret_cast<const f32x4*>(strip + row * PITCH + rd_col);
           const f32x4 v1 = *reinterpret_cast<const f32x4*>(strip + row * PITCH + rd_col + 4);
@@ -578,10 +683,10 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
           const int64_t c_idx = out_index<PERM>(p, m, n);
           const int64_t d_idx = (int64_t)m * p.ldd + n;
           if (vec_ok && n + 8 <= p.N) {
-            vec8 bv = {}, d0v = {}, d1v = {};
-            if constexpr (Epi::kHasBias) bv = *reinterpret_cast<const vec8*>(bias + n);
-            if constexpr (Epi::kNumD >= 1) d0v = *reinterpret_cast<const vec8*>(D0b + d_idx);
-            if constexpr (Epi::kNumD >= 2) d1v = *reinterpret_cast<const vec8*>(D1b + d_idx);
+            vec8 bv = bias_v, d0v = d0_e[kEarlyD > 0 ? mi * PASSES + ps : 0], d1v = d1_e[kEarlyD > 0 ? mi * PASSES + ps : 0];
+            if constexpr (Epi::kHasBias && !kEarlyBias) bv = load_vec<vec8>(bias + n);
+            if constexpr (Epi::kNumD >= 1 && kEarlyD == 0) d0v = load_vec<vec8>(D0b + d_idx);
+            if constexpr (Epi::kNumD >= 2 && kEarlyD == 0) d1v = load_vec<vec8>(D1b + d_idx);
             vec8 o;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
@@ -589,7 +694,7 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
               const float xb = Epi::kHasBias ? Tr::to_float_plus(bv[j], one, v[j]) : v[j];
               o[j] = Tr::from_float(apply_folded<Epi, T>(xb, d0v[j], d1v[j], one));
             }
-            store_out(Cb, c_idx, o, p.nt_store != 0, rc);
+            store_out(Cb, c_idx, o, stream_ok, rc);
           } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {

@@ -46,6 +46,7 @@ struct GemmTilePersist {
   static constexpr int PAIR = PAIR_;
   static constexpr int MT = MT_, KSTEP = MT == 32 ? 16 : 32, QN = 64 / MT, ACC_N = MT * MT / 64;
   static constexpr int BM = BM_, BN = BN_, BK = BK_;
+  static constexpr int KVEC = 8;
   static constexpr int WGM = WGM_, WGN = WGN_, NS = NS_;
   static constexpr int NW = WGM * WGN;
   static constexpr int NT = NW * kWaveSize;
@@ -331,14 +332,12 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_persist_kernel(const Gem
 
   // ---- epilogue -------------------------------------------------------------------------------
   const T* bias = reinterpret_cast<const T*>(p.bias);
-  // vector form for the lanes whose 8 columns lie inside the row: multi-dword global and buffer accesses need
-  // dword alignment only, so even pitches and 4-byte aligned pointers are enough
-  bool vec_ok = ((p.ldc & 1) == 0) && ((p.sc & 1) == 0) && (!PERM || ((p.perm_n2 & 7) == 0 && (p.N & 7) == 0)) &&
-      ((reinterpret_cast<uintptr_t>(p.c) & 3) == 0);
-  if (Epi::kHasBias) vec_ok = vec_ok && ((reinterpret_cast<uintptr_t>(p.bias) & 3) == 0);
-  if (Epi::kNumD >= 1)
-    vec_ok = vec_ok && ((p.ldd & 1) == 0) && ((p.sd & 1) == 0) && ((reinterpret_cast<uintptr_t>(p.d0) & 3) == 0);
-  if (Epi::kNumD >= 2) vec_ok = vec_ok && ((reinterpret_cast<uintptr_t>(p.d1) & 3) == 0);
+  // vector form for the lanes whose 8 columns lie inside the row (at any alignment: see load_vec); buffer accesses,
+  // i.e. the fast addressing and the streaming stores, need even pitches and dword-aligned pointers
+  const bool vec_ok = !PERM || ((p.perm_n2 & 7) == 0 && (p.N & 7) == 0);
+  bool dword_ok = ((p.ldc & 1) == 0) && ((p.sc & 1) == 0) && ((reinterpret_cast<uintptr_t>(p.c) & 3) == 0);
+  if (Epi::kNumD >= 1) dword_ok = dword_ok && ((p.ldd & 1) == 0) && ((p.sd & 1) == 0) && ((reinterpret_cast<uintptr_t>(p.d0) & 3) == 0);
+  if (Epi::kNumD >= 2) dword_ok = dword_ok && ((reinterpret_cast<uintptr_t>(p.d1) & 3) == 0);
   // strip addressing: row r, 16-byte chunk c lives at r * PITCH + ((c ^ (r % SC)) << 4)
   const int r_row = lane / SC;
   const int r_c = lane % SC;
@@ -369,7 +368,7 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_persist_kernel(const Gem
   // 2 GiB): the output and the residuals are addressed through buffer descriptors that start at the wave's
   // corner of the tile, with 32-bit byte offsets that advance by a scalar per 8-row pass - no 64-bit index
   // arithmetic per pass, rows past M cut off by the descriptor's size, columns past N by an out-of-range offset.
-  const bool fast_addr = !PERM && vec_ok && (p.N & 7) == 0 && (int64_t)BM * p.ldc * 2 < 0x7fffffffll &&
+  const bool fast_addr = !PERM && dword_ok && (p.N & 7) == 0 && (int64_t)BM * p.ldc * 2 < 0x7fffffffll &&
       (Epi::kNumD == 0 || (int64_t)BM * p.ldd * 2 < 0x7fffffffll);
   const uint32_t lane_off_c = (uint32_t)((r_row * (int)p.ldc + r_c * 8) * 2);
   const uint32_t lane_off_d = (uint32_t)((r_row * (int)p.ldd + r_c * 8) * 2);
@@ -402,7 +401,7 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_persist_kernel(const Gem
     float bf8[8] = {};
     if constexpr (Epi::kHasBias) {
       if (col_ok) {
-        const vec8 bv = *reinterpret_cast<const vec8*>(bias + n);
+        const vec8 bv = load_vec<vec8>(bias + n);
 #pragma unroll
         for (int j = 0; j < 8; ++j) bf8[j] = Tr::to_float(bv[j]);
       }
@@ -464,7 +463,7 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_persist_kernel(const Gem
     float bf8[8] = {};  // the lane's 8 bias values, converted once per tile
     if constexpr (Epi::kHasBias) {
       if (vec_ok && n + 8 <= p.N) {
-        const vec8 bv = *reinterpret_cast<const vec8*>(bias + n);
+        const vec8 bv = load_vec<vec8>(bias + n);
 #pragma unroll
         for (int j = 0; j < 8; ++j) bf8[j] = Tr::to_float(bv[j]);
       }
@@ -487,13 +486,13 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_persist_kernel(const Gem
           const int64_t d_idx = (int64_t)m * p.ldd + n;
           if (vec_ok && n + 8 <= p.N) {
             vec8 d0v = {}, d1v = {};
-            if constexpr (Epi::kNumD >= 1) d0v = *reinterpret_cast<const vec8*>(D0b + d_idx);
-            if constexpr (Epi::kNumD >= 2) d1v = *reinterpret_cast<const vec8*>(D1b + d_idx);
+            if constexpr (Epi::kNumD >= 1) d0v = load_vec<vec8>(D0b + d_idx);
+            if constexpr (Epi::kNumD >= 2) d1v = load_vec<vec8>(D1b + d_idx);
             vec8 o;
 #pragma unroll
             for (int j = 0; j < 8; ++j)
               o[j] = Tr::from_float(Epi::apply(Tr::to_float(raw[j]), bf8[j], Tr::to_float(d0v[j]), Tr::to_float(d1v[j])));
-            store_out(Cb, c_idx, o, p.nt_store != 0, rc);
+            store_out(Cb, c_idx, o, p.nt_store != 0 && dword_ok, rc);
           } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {

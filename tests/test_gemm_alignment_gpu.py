@@ -1,0 +1,64 @@
+"""Instances for operands at any element and for few rows, at the edges of their tiles, slabs and pieces."""
+import pytest
+import torch
+
+from aitemplate_amd import _kernels, eager
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _rand(shape, seed, scale=1.0, dtype=torch.float16):
+    return (torch.randn(*shape, generator=torch.Generator().manual_seed(seed)) * scale).to(dtype)
+
+
+def _instances(epi, dtype):
+    return [(i, n) for i, n in enumerate(_kernels.gemm_algo_names(epi, dtype)) if n.endswith("_v1") or "rows" in n]
+
+
+# K around the 8-element pieces, the 64- and 128-deep slabs and the 1024 that a few-rows workgroup takes together
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (1, 33, 7), (16, 16, 127), (17, 15, 129), (5, 100, 1025), (40, 31, 1151),
+                                   (65, 129, 63), (255, 65, 65), (130, 257, 191), (64, 64, 64), (3, 50, 2050)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_operands_at_any_element(M, N, K, dtype):
+    lib = _kernels.load()
+    dt = 0 if dtype == torch.float16 else 1
+    # views one element into their buffers; what lies before, behind and between the rows must not count
+    x, w = _rand((M, K), 1, dtype=dtype), _rand((N, K), 2, K ** -0.5, dtype)
+    b, d = _rand((N,), 3, dtype=dtype), _rand((M, N), 4, dtype=dtype)
+    want = oracle.torch_gemm("gemm_rcr_bias_add", x, w, b, d).to(dtype).float()
+    for pitch in (K, K + 3):
+        xb = torch.full((M * pitch + 1,), float("nan"), dtype=dtype, device="cuda")
+        wb = torch.full((N * pitch + 1,), float("nan"), dtype=dtype, device="cuda")
+        xv, wv = (t[1:].view(-1, pitch)[:, :K] for t in (xb, wb))
+        xv.copy_(x)
+        wv.copy_(w)
+        ran = 0
+        for algo, name in _instances(4, dt):
+            if not lib.aitamd_gemm_algo_supported(4, dt, algo, M, N, K, pitch, pitch, 2):
+                continue
+            print(f"case instance={name} M={M} N={N} K={K} pitch={pitch}", flush=True)
+            got = eager.gemm("gemm_rcr_bias_add", xv, wv, b.cuda(), d.cuda(), algo=algo)
+            tol = 1e-2 if dt == 0 else 3e-2
+            torch.testing.assert_close(got.cpu().float(), want, atol=tol, rtol=tol)
+            ran += 1
+        assert ran >= 4
+
+
+@pytest.mark.parametrize("layout", ["rcr", "rrr", "ccr", "crr"])
+@pytest.mark.parametrize("B,M,N,K", [(3, 127, 129, 65), (2, 257, 33, 1), (5, 9, 255, 130), (1, 64, 64, 64)])
+def test_layouts_at_any_element(layout, B, M, N, K):
+    lib = _kernels.load()
+    lay = _kernels.LAYOUT_ID[layout]
+    a = _rand((B, K, M) if layout[0] == "c" else (B, M, K), 1)
+    b = _rand((B, N, K) if layout[1] == "c" else (B, K, N), 2, K ** -0.5)
+    want = oracle.torch_bmm(layout, a, b).half().float()
+    ad, bd = a.cuda(), b.cuda()
+    ran = 0
+    for algo, name in _instances(0, 0):
+        if not lib.aitamd_gemm_algo_supported_layout(0, 0, lay, algo, M, N, K, a.shape[2], b.shape[2], 2):
+            continue
+        print(f"case bmm_{layout} instance={name} B={B} M={M} N={N} K={K}", flush=True)
+        torch.testing.assert_close(eager.bmm(layout, ad, bd, algo=algo).cpu().float(), want, atol=1e-2, rtol=1e-2)
+        ran += 1
+    assert ran >= 3
