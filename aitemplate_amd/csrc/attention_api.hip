@@ -3,9 +3,11 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 #include "../../include/aitemplate_amd_kernels.h"
 #include "attention_kernel.hpp"
+#include "attention_pipe.hpp"
 #include "errors.hpp"
 
 namespace aitamd {
@@ -13,7 +15,7 @@ namespace {
 
 constexpr int kMaxDevices = 64;
 
-// Variant forced by aitamd_attention_set_variant: -1 automatic, 0..3 a MODE below.  The environment variable
+// Variant forced by aitamd_attention_set_variant: -1 automatic, 0..3 a Form below.  The environment variable
 // AITAMD_ATTN_MODE gives the initial value and is read once, not on every launch.
 constexpr int kVariantUnset = -2;
 std::atomic<int> g_forced_variant{kVariantUnset};
@@ -28,62 +30,48 @@ int forced_variant() {
   return m;
 }
 
-// MODE 0: four waves (128 query rows), two LDS stages, two workgroups per CU.
-// MODE 1: eight waves (256 query rows) share each K / V tile and four LDS stages keep three tiles in flight.
-// MODE 2: as 1 with two groups of eight waves that take alternate tiles (sixteen waves per CU).
-template <int KS, int OT, int MODE>
-struct TileOf {
-  using type = AttnTile<KS, OT>;
-};
-constexpr int wide_bn(int ks, int ot) { return (16 * ks + 32 * ot) <= 128 ? 128 : 64; }
-constexpr bool wide_fits(int ks, int ot) {  // four stages of the wide tile within the LDS
-  return 4 * wide_bn(ks, ot) * (16 * ks + 8 + 32 * ot) * 2 <= 160 * 1024;
-}
-template <int KS, int OT, bool FITS = wide_fits(KS, OT)>
-struct WideTile {  // head dims too large for the wide forms keep the four-wave tile
-  using one = AttnTile<KS, OT>;
-  using two = AttnTile<KS, OT>;
-};
-template <int KS, int OT>
-struct WideTile<KS, OT, true> {
-  using one = AttnTile<KS, OT, wide_bn(KS, OT), 8, 4>;
-  // (two groups only where the merge fits the ring's memory: the small head dims this mode is chosen for)
-  static constexpr bool kMergeFits = (16 * KS + 32 * OT) <= 128 && (16 * OT + 2) * 8 * 64 * 4 <= one::kLdsBytes;
-  using two = AttnTile<KS, OT, wide_bn(KS, OT), 8, 4, kMergeFits ? 2 : 1>;
-};
-template <int KS, int OT>
-struct TileOf<KS, OT, 1> {
-  using type = typename WideTile<KS, OT>::one;
-};
-template <int KS, int OT>
-struct TileOf<KS, OT, 2> {
-  using type = typename WideTile<KS, OT>::two;
+// Work decompositions of the pipelined kernel.
+//   kRows128: four waves of 32 query rows and tiles of 32 keys.  Head dims up to 64 fit four workgroups on a CU.
+//   kRows256: four waves of 64 rows, which read every K and V fragment once for two matrix instructions; head dims of
+//             one 64-wide instance only (the registers of larger ones leave a SIMD one wave, of smaller ones the
+//             exponentials bound it and not the reads).
+//   kGroups:  as kRows128 in eight waves, two groups on alternate halves of larger tiles.
+//   kSmall:   two groups of two waves, 64 rows: four workgroups for every one of kGroups.
+//   kRows64:  two waves, 64 rows: sequences that leave the other half of 128 rows empty.
+enum Form { kRows128 = 0, kRows256 = 1, kGroups = 2, kSmall = 3, kRows64 = 4 };
+template <int KS, int OT, int FORM>
+struct PipeOf {
+  static constexpr bool kNarrow = KS <= 4 && OT <= 2;
+  using type = std::conditional_t<
+      FORM == kRows256 && kNarrow, AttnPipe<KS, OT, 1, 4, kNarrow ? 2 : 1, 1, 1, 2>,
+      std::conditional_t<FORM == kGroups, AttnPipe<KS, OT, kNarrow ? 2 : 1, 4, 1, 2, 1, 2>,
+                         std::conditional_t<FORM == kSmall, AttnPipe<KS, OT, 1, 2, 1, 2, 1, 2>,
+                                            std::conditional_t<FORM == kRows64, AttnPipe<KS, OT, 1, 2, 1, 1, 1, 2>,
+                                                               AttnPipe<KS, OT, 1, 4, 1, 1, 1, kNarrow ? 4 : 2>>>>>;
 };
 
-// MODE 3: as 0 with two groups of four waves on alternate tiles and four LDS stages: for grids that leave CUs idle.
-template <int KS, int OT>
-struct TileOf<KS, OT, 3> {
-  using Base = AttnTile<KS, OT>;
-  static constexpr bool kFits = (16 * OT + 2) * 4 * 64 * 4 <= 2 * Base::kLdsBytes && 2 * Base::kLdsBytes <= 160 * 1024;
-  using type = AttnTile<KS, OT, Base::BN, 4, kFits ? 4 : 2, kFits ? 2 : 1>;
+// the kernel's opt-in to more than 64 KiB of LDS, once per device; the outcome is kept: a failed opt-in must fail every
+// later call too, not only the first
+struct LdsOptIn {
+  std::once_flag once[kMaxDevices];
+  hipError_t err[kMaxDevices];
+  hipError_t operator()(const void* kernel, int bytes) {
+    int dev = 0;
+    const hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    dev %= kMaxDevices;
+    std::call_once(once[dev], [&] { err[dev] = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes); });
+    return err[dev];
+  }
 };
 
-template <class T, int KS, int OT, bool VEC, bool DMA, int MODE>
-hipError_t launch_attention(const AttnParams& p, hipStream_t stream) {
-  using Tile = typename TileOf<KS, OT, MODE>::type;
-  auto kernel = attention_kernel<T, Tile, VEC, DMA>;
-  static std::once_flag once[kMaxDevices];
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
+template <class T, int KS, int OT, int FORM>
+hipError_t launch_pipe(const AttnParams& p, hipStream_t stream) {
+  using Tile = typename PipeOf<KS, OT, FORM>::type;
+  auto kernel = attention_pipe_kernel<T, Tile>;
+  static LdsOptIn opt_in;
+  const hipError_t e = opt_in(reinterpret_cast<const void*>(kernel), Tile::kLdsBytes);
   if (e != hipSuccess) return e;
-  // the outcome is kept per device: a failed opt-in must fail every later call too, not only the first
-  static hipError_t attr_errs[kMaxDevices];
-  hipError_t& attr_err = attr_errs[dev % kMaxDevices];
-  std::call_once(once[dev % kMaxDevices], [&] {
-    attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, Tile::kLdsBytes);
-  });
-  if (attr_err != hipSuccess) return attr_err;
   int64_t m_tiles = (p.M + Tile::BM - 1) / Tile::BM;
   if (p.paired) m_tiles = (m_tiles + 1) / 2;
   dim3 grid((unsigned)m_tiles, (unsigned)(p.B < 65535 ? p.B : 65535), 1);
@@ -91,22 +79,75 @@ hipError_t launch_attention(const AttnParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// operands that do not come in whole, aligned 16-byte pieces (VEC: that do, in matrices beyond 32-bit offsets)
+template <class T, int KS, int OT, bool VEC>
+hipError_t launch_staged(const AttnParams& p, hipStream_t stream) {
+  using Tile = AttnTile<KS, OT>;
+  auto kernel = attention_kernel<T, Tile, VEC>;
+  static LdsOptIn opt_in;
+  const hipError_t e = opt_in(reinterpret_cast<const void*>(kernel), Tile::kLdsBytes);
+  if (e != hipSuccess) return e;
+  const int64_t m_tiles = (p.M + Tile::BM - 1) / Tile::BM;
+  dim3 grid((unsigned)m_tiles, (unsigned)(p.B < 65535 ? p.B : 65535), 1);
+  hipLaunchKernelGGL(kernel, grid, dim3(Tile::NT), Tile::kLdsBytes, stream, p);
+  return hipGetLastError();
+}
+
 typedef hipError_t (*AttnLaunch)(const AttnParams&, hipStream_t);
 
-template <class T, bool VEC, bool DMA, int MODE>
-AttnLaunch pick(int ks, int ot) {
+// smallest padded head dims first; (K <= 16 KS, O <= 32 OT); 160: the deepest attention of Stable Diffusion v1 (1280
+// channels, 8 heads)
+#define AITAMD_ATTN_DIMS(X) X(2, 1) X(3, 2) X(4, 2) X(4, 4) X(6, 3) X(8, 4) X(10, 5)
+template <class T, int FORM>
+AttnLaunch pick_pipe(int ks, int ot) {
 #define AITAMD_ATTN_CASE(KS, OT) \
-  if (ks <= KS && ot <= OT) return &launch_attention<T, KS, OT, VEC, DMA, MODE>;
-  // smallest padded head dims first; (K <= 16 KS, O <= 32 OT)
-  AITAMD_ATTN_CASE(2, 1)
-  AITAMD_ATTN_CASE(3, 2)
-  AITAMD_ATTN_CASE(4, 2)
-  AITAMD_ATTN_CASE(4, 4)
-  AITAMD_ATTN_CASE(6, 3)
-  AITAMD_ATTN_CASE(8, 4)
-  AITAMD_ATTN_CASE(10, 5)  // head dim 160: the deepest attention of Stable Diffusion v1 (1280 channels, 8 heads)
+  if (ks <= KS && ot <= OT) return &launch_pipe<T, KS, OT, FORM>;
+  AITAMD_ATTN_DIMS(AITAMD_ATTN_CASE)
 #undef AITAMD_ATTN_CASE
   return nullptr;
+}
+template <class T>
+AttnLaunch pick_pipe(int form, int ks, int ot) {
+  switch (form) {
+    case kRows256: return pick_pipe<T, kRows256>(ks, ot);
+    case kGroups: return pick_pipe<T, kGroups>(ks, ot);
+    case kSmall: return pick_pipe<T, kSmall>(ks, ot);
+    case kRows64: return pick_pipe<T, kRows64>(ks, ot);
+    default: return pick_pipe<T, kRows128>(ks, ot);
+  }
+}
+template <class T, bool VEC>
+AttnLaunch pick_staged(int ks, int ot) {
+#define AITAMD_ATTN_CASE(KS, OT) \
+  if (ks <= KS && ot <= OT) return &launch_staged<T, KS, OT, VEC>;
+  AITAMD_ATTN_DIMS(AITAMD_ATTN_CASE)
+#undef AITAMD_ATTN_CASE
+  return nullptr;
+}
+
+// The form for a problem, and whether causal query tiles go in pairs (us below: head dim 64 unless named, one box).
+Form choose_form(int64_t B, int64_t M, int64_t N, int ks, int ot, bool causal, int32_t* paired) {
+  const int64_t t64 = (M + 63) / 64, t128 = (M + 127) / 128, t256 = (M + 255) / 256;
+  // Causal: a workgroup's work grows with its rows' position.  Pairs of query tiles, the last with the first and so on,
+  // are all the same length: taken by one workgroup each where they fill the chip (two four-wave workgroups per CU or
+  // one of two groups), and where there are enough tiles that an odd one in the middle is no matter.  Otherwise the
+  // longest go first.  4 x 16 x 2048^2 59 / 50 (in order of length / pairs), 2 x 8 x 4096^2 at head dim 40 63 / 43.
+  if (causal && B <= 65535 && (t128 % 2 == 0 || t128 >= 9)) {
+    const int64_t pairs = (t128 + 1) / 2 * B;
+    *paired = pairs >= 512 || (t128 >= 8 && pairs >= 192 && pairs <= 256);
+    if (*paired) return pairs >= 512 ? kRows128 : kGroups;
+  }
+  // Grids that leave CUs idle: 64-row workgroups whose groups share the keys; 128 rows while those do fill the chip.
+  // 1 x 12 x 384^2 8.9 (128 rows, one group) / 8.5 (128, two) / 7.1 (64, two); 1 x 12 x 2048^2 31 / 24 / 24;
+  // 1 x 8 x 2048^2 at head dim 128 41 / 38 / 33, at 512 workgroups of 64 rows (1 x 16 x 2000^2) 46 / 43 / 64.  Few
+  // keys give the groups nothing to share: 6 x 12 x 316 x 77 at head dim 128 8.4 / 10.2 / 15.6.
+  if (t64 * B <= 256 || (t64 * B <= 400 && N >= 256)) return kSmall;
+  if (M <= 64) return kRows64;  // 62 x 16 x 34^2: 6.6, 8.2 with 128 rows
+  if (t128 * B <= 256 && N >= 512) return kGroups;
+  // 64 rows per wave where K and V are read often enough to be the bound: 1 x 16 x 8192^2 288, 312 with 32 rows; even
+  // at 62 x 4 x 1472^2 and at head dim 40
+  if (!causal && ks == 4 && ot == 2 && M >= 2048 && t256 * B >= 512) return kRows256;
+  return kRows128;
 }
 
 // x rounded to the nearest fp16 (dtype 0) or bf16 value, ties to even, as a float.  Done on the bits: host-side
@@ -188,64 +229,20 @@ int attention_entry(const char* who, int dtype, const void* q, const void* k, co
       ((reinterpret_cast<uintptr_t>(k) & 15) == 0) && ((reinterpret_cast<uintptr_t>(v) & 15) == 0);
   // direct-to-LDS tiles address K and V of one batch entry with 32-bit byte offsets
   const int64_t kv_dim = K > O ? K : O;
-  // (tiles are issued up to three past the last one, hence the slack)
-  const bool dma = vec && (N + 4 * 128) * kv_dim * 2 < 0x7fffffffll;
-  // 256-row workgroups for small head dims (where re-streaming K / V per 128 query rows costs most; measured
-  // slower at head dims 64 and 128) once there are enough of them to fill the CUs
-  const bool wide = dma && (16 * ks + 32 * ot) <= 112 && ((M + 255) / 256) * B >= 256;
-  // two wave groups pay when a CU holds one workgroup anyway: measured 4.5 % faster with 256 workgroups
-  // (16 heads x 4096 rows, head dim 40), 2 % slower with 512
-  // (wave groups take alternate key tiles: with fewer than four tiles there is nothing to share out - the 77 text
-  // tokens of a cross-attention are a single tile)
-  const int64_t bn = (16 * ks + 32 * ot) <= 112 ? 128 : 64;
-  const bool groups_pay = N >= 4 * bn;
-  int mode = wide ? ((((M + 255) / 256) * B <= 256 && groups_pay) ? 2 : 1) : 0;
-  // grids of 128-row workgroups that leave CUs idle take the two-group form of those too: 8-19 % faster from 48 to
-  // 256 workgroups (head dims 40 and 64), 7 % slower at 384
-  if (mode == 0 && dma && groups_pay && ((M + 127) / 128) * B <= 256) mode = 3;
-  // head dim 64: the 256-row form with two wave groups when its grid is at most one workgroup per CU (and the
-  // 128-row grid is too large for the rule above): 5-10 % faster on 4 x 16384^2, 8 x 8192^2, 16 x 4096^2, 32 x 2048^2;
-  // no gain from 512 workgroups on
-  if (mode == 0 && dma && groups_pay && (16 * ks + 32 * ot) <= 128 && ((M + 255) / 256) * B <= 256) mode = 2;
-  // Causal: a workgroup's work grows with its rows' position.  Pairs of query tiles, the last with the first and so on,
-  // are all the same length: taken by one workgroup each where they fill the chip twice over in 128-row form (two
-  // workgroups per CU) or once in the two-group form, and where there are enough tiles that an odd one in the middle
-  // is no matter.  Otherwise the longest go first, in 128-row workgroups (256 rows waste more above the diagonal).
-  // us, head dim 128, in order / longest first / pairs: 2 x 16 x 4096 237 / 210 / 177, 1 x 16 x 4096 - / 143 / 95,
-  // 16 x 16 x 1024 156 / 153 / 130; pairs of a three-tile sequence (64 x 12 x 384) 113 against 97, of 288 pairs (3 x 8 x
-  // 3000) 120 against 96.
-  if (causal && dma) {
-    const int64_t t = (M + 127) / 128, pairs = (t + 1) / 2 * B;
-    mode = groups_pay && t * B <= 256 ? 3 : 0;
-    if (B <= 65535 && (t % 2 == 0 || t >= 9)) {
-      if (pairs >= 512) {
-        p.paired = 1;
-        mode = 0;
-      } else if (groups_pay && t >= 8 && pairs >= 192 && pairs <= 256) {
-        p.paired = 1;
-        mode = 3;
-      }
-    }
-  }
-  // aitamd_attention_set_variant(0|1|2|3) forces a variant where the shape allows it (a test and measurement knob)
-  {
-    const int m = forced_variant();
-    if (m >= 0 && m <= 2 && dma && (16 * ks + 32 * ot) <= 128) mode = m;
-    if (m == 3 && dma) mode = 3;
-  }
+  // (tiles are issued past the last one, and out-of-range offsets are the largest of these and 2^31 added up)
+  const bool dma = vec && (N + 4 * 128) * kv_dim * 2 < 0x70000000;
   AttnLaunch fn = nullptr;
-  if (dtype == 0)
-    fn = mode == 3 ? pick<f16, true, true, 3>(ks, ot)
-       : mode == 2 ? pick<f16, true, true, 2>(ks, ot)
-                   : (mode == 1 ? pick<f16, true, true, 1>(ks, ot)
-                                : (dma ? pick<f16, true, true, 0>(ks, ot)
-                                       : (vec ? pick<f16, true, false, 0>(ks, ot) : pick<f16, false, false, 0>(ks, ot))));
-  else
-    fn = mode == 3 ? pick<bf16, true, true, 3>(ks, ot)
-       : mode == 2 ? pick<bf16, true, true, 2>(ks, ot)
-                   : (mode == 1 ? pick<bf16, true, true, 1>(ks, ot)
-                                : (dma ? pick<bf16, true, true, 0>(ks, ot)
-                                       : (vec ? pick<bf16, true, false, 0>(ks, ot) : pick<bf16, false, false, 0>(ks, ot))));
+  if (dma) {
+    int form = choose_form(B, M, N, ks, ot, causal != 0, &p.paired);
+    // aitamd_attention_set_variant(0|1|2|3) forces a form (a test and measurement knob)
+    if (forced_variant() >= 0) form = forced_variant();
+    if (form == kRows256) p.paired = 0;
+    fn = dtype == 0 ? pick_pipe<f16>(form, ks, ot) : pick_pipe<bf16>(form, ks, ot);
+  } else if (dtype == 0) {
+    fn = vec ? pick_staged<f16, true>(ks, ot) : pick_staged<f16, false>(ks, ot);
+  } else {
+    fn = vec ? pick_staged<bf16, true>(ks, ot) : pick_staged<bf16, false>(ks, ot);
+  }
   if (!fn) return fail("%s: no instance for K=%lld O=%lld", who, (long long)K, (long long)O);
   const hipError_t e = fn(p, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail("%s: launch failed: %s", who, hipGetErrorString(e));

@@ -2,9 +2,9 @@
 // folded into the store (bmm_softmax_bmm_permute), gfx950.
 //
 // The score matrix never leaves the chip.  One wave owns 32 query rows and walks
-// the keys/values in blocks of 32 (64 for the smallest head dims); a workgroup of 4 or
-// 8 waves shares each 64- or 128-row K / V tile through LDS, and the 16-wave form runs
-// two such groups on alternate tiles of the same rows and merges them at the end.
+// the keys/values in blocks of 32 (64 for the smallest head dims); a workgroup of 4 waves
+// shares each 64- or 128-row K / V tile through LDS.  This kernel takes operands at any
+// alignment through registers; attention_pipe.hpp has the one for whole 16-byte pieces.
 //
 //  * S^T = K Q^T is computed with v_mfma_f32_32x32x16 (K tile rows as the A
 //    operand, the wave's Q rows - kept in registers for the whole kernel - as
@@ -28,12 +28,6 @@
 
 #include "common.hpp"
 
-#ifndef AITAMD_ATTN_FAST
-#define AITAMD_ATTN_FAST 1
-#endif
-#ifndef AITAMD_ATTN_BATCH_READS
-#define AITAMD_ATTN_BATCH_READS 0
-#endif
 #ifndef AITAMD_ATTN_KB
 #define AITAMD_ATTN_KB(KS, OT) (((KS) + 2 * (OT)) <= 7 ? 2 : 1)
 #endif
@@ -60,20 +54,17 @@ struct AttnParams {
   int32_t paired;
 };
 
-// NW_ waves (32 query rows each) share the K / V tiles; NS_ LDS stages.  The register-staged
-// loaders use two stages; the direct-to-LDS path keeps NS_ - 1 tiles in flight.
-// NG_ groups of NW_ waves each take every NG_-th tile of the same query rows and merge their running
-// sums at the end: twice the waves per SIMD for the same K / V traffic.
-template <int KS_, int OT_, int BN_ = ((16 * KS_ + 32 * OT_) <= 112 ? 128 : 64), int NW_ = 4, int NS_ = 2, int NG_ = 1>
+// NW waves (32 query rows each) share the K / V tiles in two LDS stages
+template <int KS_, int OT_>
 struct AttnTile {
   static constexpr int KS = KS_;          // K padded to 16 * KS
   static constexpr int OT = OT_;          // O padded to 32 * OT
   static constexpr int KP = 16 * KS;
   static constexpr int OP = 32 * OT;
-  static constexpr int NW = NW_, NS = NS_, NG = NG_;
+  static constexpr int NW = 4, NS = 2;
   static constexpr int BM = 32 * NW;      // query rows per workgroup
-  static constexpr int BN = BN_;          // keys per LDS tile: 128 while two workgroups still fit one CU's LDS
-  static constexpr int NT = 64 * NW * NG;
+  static constexpr int BN = (16 * KS_ + 32 * OT_) <= 112 ? 128 : 64;  // keys per LDS tile: 128 while two workgroups still fit one CU's LDS
+  static constexpr int NT = 64 * NW;
   static constexpr int K_PITCH = KP + 8;  // halves; keeps 16 consecutive rows on distinct banks
   // V rows carry no pad.  The transposing read fetches, per 32 lanes, 64 bytes of each of 4 consecutive rows; the
   // four pieces have to fall into four different quarters of the 64 banks.  Rows of 64 or 192 bytes do that as
@@ -90,8 +81,6 @@ struct AttnTile {
   static constexpr int V_IT = (V_CHUNKS + NT - 1) / NT;
   static constexpr int kLdsBytes = NS * BN * (K_PITCH + V_PITCH) * 2;
   static_assert(kLdsBytes <= 160 * 1024, "LDS budget");
-  static_assert(NG == 1 || (NS % NG == 0 && NS >= 2 * NG), "the groups' tiles and the next ones in flight need a stage each");
-  static_assert(NG == 1 || (16 * OT + 2) * NW * 64 * 4 <= kLdsBytes, "the merge goes through the ring's memory");
 };
 
 // LDS transpose read: 4 x 16-bit per lane, gathered across the 16 lanes of a block (__restrict__: see tr_read16)
@@ -154,38 +143,17 @@ AITAMD_DEVICE float sum_across_halves(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// VEC: K and O are multiples of 8 and all base pointers 16-byte aligned -> 128-bit
-// loads; otherwise elements are gathered one by one (slow, any shape).
-// DMA (needs VEC, and each K / V matrix of a batch entry below 2 GiB): the K / V tiles go
-// global -> LDS directly (buffer_load ... lds) instead of through registers: lane i of a wave-load
-// fills the i-th 16-byte chunk of a 1 KiB LDS block, the rows' pad chunk and the rows past N are
-// out-of-range lanes (zero fill), and one s_waitcnt vmcnt(0) + s_barrier per tile replaces the
-// register staging, the LDS stores and the full __syncthreads().
 template <int N>
 AITAMD_DEVICE void attn_wait_vmcnt() {
   // s_waitcnt simm16: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14]; only vmcnt is waited for
   constexpr int imm = (N & 0xf) | ((N >> 4) << 14) | (0x7 << 4) | (0xf << 8);
   __builtin_amdgcn_s_waitcnt(imm);
 }
-template <int N>
-AITAMD_DEVICE void attn_wait_vmcnt_upto(int n) {
-  // wave-uniform n: waits until at most min(n, N) vector-memory operations are outstanding
-  if constexpr (N == 0) {
-    attn_wait_vmcnt<0>();
-  } else {
-    if (n >= N)
-      attn_wait_vmcnt<N>();
-    else
-      attn_wait_vmcnt_upto<N - 1>(n);
-  }
-}
-
-template <class T, class Tile, bool VEC, bool DMA = false>
-__global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_kernel(const AttnParams p) {
-  static_assert(!DMA || VEC, "the direct-to-LDS path needs 16-byte chunks");
-  static_assert(DMA || Tile::NS == 2, "the register-staged loaders double-buffer");
-  static_assert(DMA || Tile::NG == 1, "wave groups need the direct-to-LDS loader");
-  constexpr int NS = Tile::NS, NW = Tile::NW, NG = Tile::NG, NWT = NW * NG;
+// VEC: K and O are multiples of 8 and all base pointers 16-byte aligned -> 128-bit
+// loads; otherwise elements are gathered one by one (slow, any shape).
+template <class T, class Tile, bool VEC>
+__global__ void __launch_bounds__(Tile::NT, 2) attention_kernel(const AttnParams p) {
+  constexpr int NS = Tile::NS;
   using Tr = ElemTraits<T>;
   using vec8 = typename Tr::vec8;
   using vec4 = typename Tr::vec4;
@@ -198,36 +166,11 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave_all = tid >> 6;
-  const int grp = __builtin_amdgcn_readfirstlane(wave_all / NW);  // which tiles this wave takes
-  const int wave = wave_all % NW;                                 // which 32 query rows
+  const int wave = tid >> 6;  // which 32 query rows
   const int r32 = lane & 31;
   const int h = lane >> 5;
-  // Workgroup -> (query tile, batch entry).  The hardware deals consecutive workgroup ids round-robin over the
-  // 8 XCDs, each with its own L2; dealt plainly, the workgroups of one batch entry land on all of them and every
-  // L2 fetches that entry's K and V.  Instead XCD x works through the batch entries x, x + 8, x + 16, ... one after
-  // the other, so the workgroups that stream the same K / V share one L2.  (Eighths of consecutive entries share as
-  // well, but give whole XCDs the long or the short sequences where lengths follow the batch order: 64 x 12 x 384
-  // with lengths spread from all to a quarter of the keys ran in 53 us so, against 46.)  The up to seven entries
-  // that are left over go round the XCDs tile by tile.
-  // Causal: the longest rows first, so that the short ones fill the end of the launch.
-  int bx = blockIdx.x, by = blockIdx.y;
-  if ((int)gridDim.y == p.B) {
-    const int id = blockIdx.x + gridDim.x * blockIdx.y;
-    const int tiles = gridDim.x, even = p.B & ~(kNumXcd - 1);
-    if (id < even * tiles) {
-      const int slot = id / kNumXcd, entry = slot / tiles;
-      by = entry * kNumXcd + id % kNumXcd;
-      bx = slot - entry * tiles;
-    }
-    if (p.causal) bx = tiles - 1 - bx;
-  }
-  const int m_tiles = (p.M + Tile::BM - 1) / Tile::BM;
-  const int first_tile = p.paired ? m_tiles - 1 - ((int)gridDim.x - 1 - bx) : bx;
-  const int passes = p.paired && 2 * first_tile != m_tiles - 1 ? 2 : 1;
-
-  for (int b = by, pass = 0; b < p.B; pass = pass + 1 < passes ? pass + 1 : 0, b += pass == 0 ? gridDim.y : 0) {
-    const int m0 = (pass == 0 ? first_tile : m_tiles - 1 - first_tile) * Tile::BM;
+  const int m0 = blockIdx.x * Tile::BM;
+  for (int b = blockIdx.y; b < p.B; b += gridDim.y) {
     const int q_row = m0 + wave * 32 + r32;  // this lane's query row
     const T* Qb = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.M * p.K;
     const T* Kb = reinterpret_cast<const T*>(p.k) + (int64_t)b * p.N * p.K;
@@ -319,46 +262,7 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
       }
     };
 
-    // ---- direct-to-LDS tile loader: the KL + VL wave-loads of a tile are dealt round-robin to the waves
-    constexpr int KC1 = KP / 8 + 1, VC1 = OP / 8;            // chunks per LDS row (K: pad chunk included)
-    constexpr int KL = BN * KC1 / 64, VL = BN * VC1 / 64;     // wave-loads per K / V tile
-    constexpr int L_W = (KL + VL + NWT - 1) / NWT;
-    static_assert((BN * KC1) % 64 == 0 && (BN * VC1) % 64 == 0, "tiles must be whole wave-loads");
-    static_assert(Tile::K_PITCH == KC1 * 8 && Tile::V_PITCH == VC1 * 8, "LDS rows are whole chunks");
-    typedef __attribute__((address_space(3))) void lds_void;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    const int wave_ld = __builtin_amdgcn_readfirstlane(wave_all);  // the loads are dealt over all waves
-    uint32_t d_off[L_W];  // byte offset of the lane's chunk inside K (or V) for n0 = 0; kOobOffset = always zero
-    if constexpr (DMA) {
-#pragma unroll
-      for (int i = 0; i < L_W; ++i) {
-        const int j = wave_ld + NWT * i;
-        const bool is_k = j < KL;
-        const int idx = (is_k ? j : j - KL) * 64 + lane;
-        const int c1 = is_k ? KC1 : VC1;
-        const int dim = is_k ? p.K : p.O;
-        const int row = idx / c1;
-        // the lane fills chunk slot idx - row * c1 of the row; for V that slot holds chunk slot ^ v_swz(row)
-        const int c = is_k ? idx - row * c1 : (idx - row * c1) ^ Tile::v_swz(row);
-        d_off[i] = (c * 8 < dim) ? (uint32_t)((row * dim + c * 8) * 2) : kOobOffset;
-      }
-    }
-    // (the K / V choice of a wave-load is wave-uniform: scalar selects, no branches)
-    auto issue_tile = [&](int n0, int stage) {
-      T* dK = sK + stage * BN * KPI;
-      T* dV = sV + stage * BN * VPI;
-#pragma unroll
-      for (int i = 0; i < L_W; ++i) {
-        const int j = wave_ld + NWT * i;
-        if ((i + 1) * NWT > KL + VL && j >= KL + VL) continue;  // only the last round can run past the tile
-        const bool is_k = j < KL;
-        const uint32_t off =
-            d_off[i] != kOobOffset ? d_off[i] + (uint32_t)(n0 * (is_k ? p.K : p.O) * 2) : kOobOffset;
-        T* dst = is_k ? dK + j * 512 : dV + (j - KL) * 512;
-        const __amdgpu_buffer_rsrc_t r = make_rsrc(is_k ? Kb : Vb, (uint32_t)((int64_t)N * (is_k ? p.K : p.O) * 2));
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)dst, 16, off, 0, 0, 0);
-      }
-    };
 
     // keys this workgroup has to visit (causal: nothing right of the last query row)
     int n_end = N;
@@ -378,31 +282,13 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
     const float c = __builtin_fabsf(p.scale_log2e);
     float m_run = -INFINITY;
     float l_run = 0.0f;       // running sum over this lane's half of the keys
-#if AITAMD_ATTN_FAST
     bool ref_ok = false;      // (wave-uniform) every row of the wave has a finite reference point
-#endif
 
-    // wave-loads this wave issues per tile
-    const int my_loads = (KL + VL - wave_ld + NWT - 1) / NWT;
-    if constexpr (DMA && NG > 1) {
-      // every group's first tile; later tiles are issued one iteration ahead (see the loop)
-#pragma unroll
-      for (int g = 0; g < NG; ++g)
-        if (g < n_tiles) issue_tile(g * BN, g);
-    } else if constexpr (DMA) {
-      // NS - 1 tiles in flight; tiles past the last one are all out of range (zero fill, no traffic),
-      // issued all the same so that the number of loads per tile stays constant for the waits
-      if (n_tiles > 0) {
-#pragma unroll
-        for (int s0 = 0; s0 < NS - 1; ++s0) issue_tile(s0 * BN, s0);
-      }
-    } else {
-      if (n_tiles > 0) {
-        load_tiles(0);
-        store_tiles(0);
-      }
-      __syncthreads();
+    if (n_tiles > 0) {
+      load_tiles(0);
+      store_tiles(0);
     }
+    __syncthreads();
 
     // source-lane address pattern of the LDS transpose read (see file header):
     // 16-lane block = one 4-key x 16-column patch; lane i of the block points at
@@ -419,32 +305,9 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
     constexpr int KB = AITAMD_ATTN_KB(KS, OT);
     static_assert(BN % (32 * KB) == 0, "a tile is whole blocks");
     int cur = 0;
-    const int n_iters = (n_tiles + NG - 1) / NG;
-    for (int it = 0; it < n_iters; ++it) {
-      const int t = it * NG + grp;  // this wave's tile
+    for (int t = 0; t < n_tiles; ++t) {
       const bool has_next = (t + 1) < n_tiles;
-      if constexpr (DMA && NG > 1) {
-        // the tiles of this iteration were issued one iteration ago; past the barrier the stages of the
-        // previous iteration are free and take the next iteration's tiles
-        attn_wait_vmcnt<0>();
-        __builtin_amdgcn_s_barrier();
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-          const int tn = (it + 1) * NG + g;
-          if (tn < n_tiles) issue_tile(tn * BN, tn % NS);
-        }
-        cur = t % NS;
-        if (t >= n_tiles) continue;  // the last iteration can be short of tiles
-      } else if constexpr (DMA) {
-        // this wave's part of tile t has landed once only the NS - 2 younger tiles are in flight; past
-        // the barrier everybody's has, and nobody reads the stage of tile t - 1 any more, so tile
-        // t + NS - 1 starts landing there
-        attn_wait_vmcnt_upto<(NS - 2) * L_W>((NS - 2) * my_loads);
-        __builtin_amdgcn_s_barrier();
-        issue_tile((t + NS - 1) * BN, cur == 0 ? NS - 1 : cur - 1);
-      } else {
-        if (has_next) load_tiles((t + 1) * BN);
-      }
+      if (has_next) load_tiles((t + 1) * BN);
       const T* cK = sK + cur * BN * KPI;
       const T* cV = sV + cur * BN * VPI;
       // The lane's LDS addresses of the tile, one per operand (and per 32-column block of V, whose swizzle sits
@@ -468,25 +331,6 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
         // (issuing the next block's product ahead of this block's softmax was measured: no gain at
         // head dim 40 and a quarter slower at head dim 64, where the extra live accumulator costs more)
         f32x16 s[KB];
-#if AITAMD_ATTN_BATCH_READS
-        // all K fragments of the block first, then its MFMAs: the reads overlap each other and the first MFMAs
-        // instead of each being waited for right behind its issue
-        {
-          vec8 kf[KB][KS];
-#pragma unroll
-          for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-              kf[kb][ks] = *reinterpret_cast<const vec8*>(cK + ((blk * KB + kb) * 32 + r32) * KPI + ks * 16 + h * 8);
-#pragma unroll
-          for (int kb = 0; kb < KB; ++kb) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) s[kb][e] = 0.0f;
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) s[kb] = Tr::mfma32(kf[kb][ks], qf[ks], s[kb]);
-          }
-        }
-#else
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) {
 #pragma unroll
@@ -498,7 +342,6 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
             s[kb] = Tr::mfma32(kf, qf[ks], s[kb]);
           }
         }
-#endif
         // lane holds keys nb + 32 kb + 8 g + 4 h + r (element 4 g + r of sub-block kb) of query row q_row.
         // The running maximum is kept on the raw scores and the scale is folded into the exponent:
         // p = exp2(s * c - m * c) is one FMA and one v_exp per score (c > 0: a negative scale was moved into
@@ -555,7 +398,6 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
           m_run = m_new;
         };
         const float m_before = m_run, l_before = l_run;
-#if AITAMD_ATTN_FAST
         // Fast form of an unmasked block: no row maximum at all.  The probabilities are taken against the reference
         // point the row already has, p = exp2((s - m) c); that is exact whatever m is, as long as no p leaves the
         // element type's range, and a p beyond it shows as an infinite (or NaN) row sum, for which the block is
@@ -588,12 +430,6 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
             softmax_block(std::false_type{}, std::false_type{});
           ref_ok = __builtin_amdgcn_ballot_w64(__builtin_isinf(m_run)) == 0;
         }
-#else
-        if (need_mask)
-          softmax_block(std::true_type{}, std::false_type{});
-        else
-          softmax_block(std::false_type{}, std::false_type{});
-#endif
         // A NaN score (a NaN in Q or in a K row) counts as -inf, i.e. its key is left out, as in the reference, whose
         // kernel applies ScaleAndResetNaNToMinusInfinity to the scores
         // (python/aitemplate/backend/rocm/gemm/bmm_softmax_bmm_permute.py:106, bmm_softmax_bmm.py:99).  The running
@@ -604,9 +440,7 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
           m_run = m_before;
           l_run = l_before;
           softmax_block(std::true_type{}, std::true_type{});
-#if AITAMD_ATTN_FAST
           ref_ok = __builtin_amdgcn_ballot_w64(__builtin_isinf(m_run)) == 0;
-#endif
         }
         if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
 #pragma unroll
@@ -615,29 +449,6 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
             for (int e = 0; e < 16; ++e) oacc[ot][e] *= alpha;
         }
         // ---- O^T += V^T P^T over the block's 16-key steps
-#if AITAMD_ATTN_BATCH_READS
-        {
-          // all V^T fragments of the block first (the score registers are free by now), then the MFMAs
-          vec8 vfs[2 * KB][OT];
-#pragma unroll
-          for (int st = 0; st < 2 * KB; ++st)
-#pragma unroll
-            for (int ot = 0; ot < OT; ++ot) {
-              const T* vb = cV + (blk * KB * 32 + st * 16 + h * 4 + tr_row) * VPI + ((ot * 32) ^ tr_swz) + tr_col;
-              const vec4 lo = AttnVec<T>::tr_read(vb);
-              const vec4 hi = AttnVec<T>::tr_read(vb + 8 * VPI);
-#pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                vfs[st][ot][j] = lo[j];
-                vfs[st][ot][4 + j] = hi[j];
-              }
-            }
-#pragma unroll
-          for (int st = 0; st < 2 * KB; ++st)
-#pragma unroll
-            for (int ot = 0; ot < OT; ++ot) oacc[ot] = Tr::mfma32(vfs[st][ot], pf[st], oacc[ot]);
-        }
-#else
 #pragma unroll
         for (int st = 0; st < 2 * KB; ++st) {
 #pragma unroll
@@ -654,55 +465,17 @@ __global__ void __launch_bounds__(Tile::NT, Tile::NW == 4 ? 2 : 1) attention_ker
             oacc[ot] = Tr::mfma32(vf, pf[st], oacc[ot]);
           }
         }
-#endif
       }
 
-      if constexpr (!DMA) {
-        if (has_next) store_tiles(cur ^ 1);
-        __syncthreads();
-      }
-      if constexpr (NG == 1) cur = cur + 1 == NS ? 0 : cur + 1;
-    }
-
-    // ---- wave groups: the other groups hand their running state to group 0 through the ring's memory
-    if constexpr (NG > 1) {
-      attn_wait_vmcnt<0>();
-      __syncthreads();  // nobody reads tiles any more and nothing is landing
-      float* xch = reinterpret_cast<float*>(smem_raw);
-      constexpr int NV = 16 * OT + 2;
-      static_assert(NG == 2, "the merge below pairs two groups");
-      if (grp == 1) {
-#pragma unroll
-        for (int ot = 0; ot < OT; ++ot)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) xch[((ot * 16 + e) * NW + wave) * 64 + lane] = oacc[ot][e];
-        xch[((NV - 2) * NW + wave) * 64 + lane] = m_run;
-        xch[((NV - 1) * NW + wave) * 64 + lane] = l_run;
-      }
+      if (has_next) store_tiles(cur ^ 1);
       __syncthreads();
-      if (grp == 0) {
-        const float m1 = xch[((NV - 2) * NW + wave) * 64 + lane];
-        const float l1 = xch[((NV - 1) * NW + wave) * 64 + lane];
-        // both states are sums of exp2((s - m) c) terms for their own reference m: bring them to the larger one
-        const float m = fmaxf(m_run, m1);
-        const float a0 = __builtin_isinf(m_run) ? 0.0f : __builtin_amdgcn_exp2f((m_run - m) * c);
-        const float a1 = __builtin_isinf(m1) ? 0.0f : __builtin_amdgcn_exp2f((m1 - m) * c);
-        l_run = l_run * a0 + l1 * a1;
-#pragma unroll
-        for (int ot = 0; ot < OT; ++ot)
-#pragma unroll
-          for (int e = 0; e < 16; ++e)
-            oacc[ot][e] = oacc[ot][e] * a0 + xch[((ot * 16 + e) * NW + wave) * 64 + lane] * a1;
-      }
+      cur ^= 1;
     }
 
-    // the tiles issued past the last one: nothing may be landing when the workgroup ends or the stages are refilled
-    // (waited for ahead of the stores, which nobody waits for)
-    if constexpr (DMA) attn_wait_vmcnt<0>();
     // ---- normalise and store permuted: out[b / G][m][b % G][o]
     const float l_tot = sum_across_halves(l_run);
     const float inv = (l_tot > 0.0f && q_row < m_rows) ? 1.0f / l_tot : 0.0f;
-    if (q_row < p.M && grp == 0) {
+    if (q_row < p.M) {
       T* orow = reinterpret_cast<T*>(p.out) + (((int64_t)(b / p.G) * p.M + q_row) * p.G + (b % p.G)) * p.O;
       const bool vec_ok = ((p.O & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.out) & 7) == 0);
 #pragma unroll

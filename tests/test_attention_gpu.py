@@ -310,3 +310,18 @@ def test_causal_pairs_of_query_tiles(batch, heads, S, d):
     short = S // 3
     part = eager.mem_eff_attention(q[:, :, :short].contiguous(), k[:, :, :short].contiguous(), v[:, :, :short].contiguous(), causal=True)
     torch.testing.assert_close(got[:, :short].float(), part.float(), atol=2e-3, rtol=2e-2)
+
+
+# the pipelined kernel's forms at the edges of their tiles (32 and 64 keys, 64, 128 and 256 rows), head dims from one
+# matrix instruction to the widest, and the rules' own choices from a single row up
+@pytest.mark.parametrize("mode", [None, 0, 1, 2, 3])
+@pytest.mark.parametrize("batch,heads,S,Skv,d,dv", [(1, 3, 1, 1, 64, 64), (2, 2, 33, 31, 8, 16), (1, 2, 64, 65, 64, 64), (1, 2, 129, 97, 128, 128),
+                                                    (2, 1, 257, 256, 40, 40), (1, 1, 100, 161, 160, 152), (70, 8, 31, 33, 64, 64), (1, 2, 63, 700, 96, 88)])
+def test_forms_at_the_edges_of_their_tiles(attn_variant, mode, batch, heads, S, Skv, d, dv):
+    if mode is not None:
+        attn_variant(mode)
+    for dtype in (torch.float16, torch.bfloat16):
+        for causal in (False, True):
+            print(f"case mode={mode} {dtype} causal={causal}", flush=True)
+            _check_mem_eff(batch, heads, S, Skv, d, dv, [Skv - (i % 3) for i in range(batch)] if Skv > 2 else None, dtype=dtype,
+                           causal=causal, seed=S)
