@@ -12,16 +12,15 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/Context.h>
-#include <ATen/hip/EmptyTensor.h>
-#include <c10/hip/HIPStream.h>
-#include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstring>
 #include <string>
 #include <vector>
 
 #include "../../include/aitemplate_amd_kernels.h"
 #include "../../include/model_interface.h"
+#include "native_device.h"
 
 namespace {
 
@@ -55,10 +54,14 @@ const OpInfo kOps[] = {
 PyObject* not_ordinary() { Py_RETURN_NOTIMPLEMENTED; }
 
 // A plain tensor on the GPU, or null (also for None and for subclasses, which may intercept what is done to them).
+// The wrappers of torch.func and of functionalization are of the exact type torch.Tensor and report the device of what
+// they wrap, but have no memory of their own.
 const at::Tensor* gpu_tensor(PyObject* o) {
   if (!THPVariable_CheckExact(o)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);
-  return t.is_cuda() && t.layout() == at::kStrided ? &t : nullptr;
+  constexpr c10::DispatchKeySet wrappers(
+      {c10::DispatchKey::Functionalize, c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper});
+  return on_device(t) && t.layout() == at::kStrided && t.has_storage() && !t.key_set().has_any(wrappers) ? &t : nullptr;
 }
 
 int dtype_id(const at::Tensor& t) {
@@ -70,12 +73,6 @@ int dtype_id(const at::Tensor& t) {
 bool plain_allocation() {
   return !(at::globalContext().deterministicAlgorithms() && at::globalContext().deterministicFillUninitializedMemory());
 }
-
-at::Tensor empty_like_device(at::IntArrayRef sizes, const at::Tensor& like) {
-  return at::Tensor(at::detail::empty_cuda(sizes, like.scalar_type(), like.device(), std::nullopt));
-}
-
-void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
 // Row pitch of a [rows, cols] view with contiguous rows; false where the rows are not contiguous.
 bool row_pitch(const at::Tensor& t, int64_t* pitch) {
@@ -110,14 +107,19 @@ PyObject* guarded(F&& body) {
   }
 }
 
-// The launch itself runs without the interpreter lock, as it does through ctypes.
+// The launch itself runs without the interpreter lock, as it does through ctypes.  What it takes is plain pointers and
+// numbers, read beforehand: a tensor's accessors may throw, and the error is raised with the lock held.
+struct Unlocked {
+  PyThreadState* const save = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(save); }
+};
 template <class F>
 int unlocked(F&& launch) {
-  PyThreadState* save = PyEval_SaveThread();
-  const int rc = launch();
-  PyEval_RestoreThread(save);
-  return rc;
+  const Unlocked here;
+  return launch();
 }
+
+const void* pointer(const at::Tensor* t) { return t == nullptr ? nullptr : t->data_ptr(); }
 
 // gemm(op, a, b, bias, d0, d1, out, algo, workspace)
 PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -181,11 +183,11 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
     const int algo = (int)PyLong_AsLong(args[7]);
     if (algo == -1 && PyErr_Occurred()) return nullptr;
-    auto ptr = [](const at::Tensor* t) -> const void* { return t == nullptr ? nullptr : t->data_ptr(); };
+    const void *pa = pointer(a), *pb = pointer(b), *bias = pointer(opt[0]), *d0 = pointer(opt[1]), *d1 = pointer(opt[2]);
     void* stream = current_stream();
     const int rc = unlocked([&] {
-      return aitamd_gemm_rcr_ws(info->epilogue, dt, algo, a->data_ptr(), b->data_ptr(), ptr(opt[0]), ptr(opt[1]), ptr(opt[2]), c,
-                                M, N, K, lda, ldb, ldc, ldd, ws, ws_bytes, stream);
+      return aitamd_gemm_rcr_ws(info->epilogue, dt, algo, pa, pb, bias, d0, d1, c, M, N, K, lda, ldb, ldc, ldd, ws, ws_bytes,
+                                stream);
     });
     return finish(rc, info->name, made.defined() ? &made : nullptr, args[6]);
   });
@@ -223,10 +225,11 @@ PyObject* bmm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       c = out->data_ptr();
     }
     const int64_t sa = ba == 1 && B > 1 ? 0 : M * K, sb = bb == 1 && B > 1 ? 0 : N * K;
+    const int64_t lda = a->size(-1), ldb = b->size(-1);
+    const void *pa = pointer(a), *pb = pointer(b);
     void* stream = current_stream();
     const int rc = unlocked([&] {
-      return aitamd_bmm(layout, dt, algo, a->data_ptr(), b->data_ptr(), c, B, M, N, K, a->size(-1), b->size(-1), N, sa, sb, M * N,
-                        d1, stream);
+      return aitamd_bmm(layout, dt, algo, pa, pb, c, B, M, N, K, lda, ldb, N, sa, sb, M * N, d1, stream);
     });
     return finish(rc, PyUnicode_AsUTF8(args[6]), made.defined() ? &made : nullptr, args[3]);
   });
@@ -272,10 +275,10 @@ PyObject* bmm_softmax_bmm_permute(PyObject*, PyObject* const* args, Py_ssize_t n
     if (out == nullptr) return not_ordinary();
     const float scale = (float)PyFloat_AS_DOUBLE(args[4]);
     const int causal = args[5] == Py_True;
+    const void *q = pointer(t[0]), *k = pointer(t[1]), *v = pointer(t[2]);
     void* stream = current_stream();
     const int rc = unlocked([&] {
-      return aitamd_bmm_softmax_bmm_permute(dt, t[0]->data_ptr(), t[1]->data_ptr(), t[2]->data_ptr(), out, B, M, N, K, O, G, scale,
-                                            causal, stream);
+      return aitamd_bmm_softmax_bmm_permute(dt, q, k, v, out, B, M, N, K, O, G, scale, causal, stream);
     });
     return finish(rc, "bmm_softmax_bmm_permute", made.defined() ? &made : nullptr, args[6]);
   });
@@ -305,10 +308,10 @@ PyObject* mem_eff_attention(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     if (out == nullptr) return not_ordinary();
     const float scale = (float)std::pow((double)K, -0.5);
     const int causal = args[3] == Py_True;
+    const void *q = pointer(t[0]), *k = pointer(t[1]), *v = pointer(t[2]);
     void* stream = current_stream();
     const int rc = unlocked([&] {
-      return aitamd_mem_eff_attention(dt, t[0]->data_ptr(), t[1]->data_ptr(), t[2]->data_ptr(), out, B, H, M, N, K, O, scale, causal,
-                                      lengths[0], lengths[1], stream);
+      return aitamd_mem_eff_attention(dt, q, k, v, out, B, H, M, N, K, O, scale, causal, lengths[0], lengths[1], stream);
     });
     return finish(rc, "mem_eff_attention", made.defined() ? &made : nullptr, args[6]);
   });
