@@ -10,12 +10,14 @@
 // For anything else they return NotImplemented without having done anything, and the caller's Python path, which
 // handles the remaining cases and words the errors, takes the call.
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <ATen/Context.h>
 
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/aitemplate_amd_kernels.h"
@@ -334,40 +336,47 @@ bool model_dtype(at::ScalarType s, AITemplateDtype* out) {
   }
 }
 
-// The tensors of a list, or of a dict ordered by `index` (name -> position); false where they are not ordinary.
-bool model_tensors(PyObject* params, PyObject* index, std::vector<const at::Tensor*>* out) {
-  auto usable = [](PyObject* o) -> const at::Tensor* {
+typedef std::vector<std::pair<THPObjectPtr, size_t>> Names;
+
+// The tensors of a list, or of a dict ordered by `index` (name -> position), and the names in the order of the caller's
+// dict (of `index` for a list); false where they are not ordinary.  Both are held, not borrowed: the caller's containers
+// may change while the run has given up the interpreter lock.
+bool model_tensors(PyObject* params, PyObject* index, std::vector<at::Tensor>* out, Names* names) {
+  auto hold = [&](size_t i, PyObject* o) {
     const at::Tensor* t = gpu_tensor(o);
-    return t != nullptr && t->is_contiguous() ? t : nullptr;
+    if (t == nullptr || !t->is_contiguous()) return false;
+    (*out)[i] = *t;
+    return true;
   };
   const Py_ssize_t n = PyDict_Size(index);
-  out->assign((size_t)n, nullptr);
-  if (PyDict_CheckExact(params)) {
+  out->resize((size_t)n);
+  const bool by_name = PyDict_CheckExact(params);
+  if (by_name) {
     if (PyDict_Size(params) != n) return false;
-    PyObject *name, *value;
-    Py_ssize_t pos = 0;
-    while (PyDict_Next(params, &pos, &name, &value)) {
-      PyObject* at_index = PyDict_GetItemWithError(index, name);
-      if (at_index == nullptr) return false;
-      (*out)[(size_t)PyLong_AsLong(at_index)] = usable(value);
-    }
-  } else if (PyList_CheckExact(params) || PyTuple_CheckExact(params)) {
-    if (PySequence_Fast_GET_SIZE(params) != n) return false;
-    for (Py_ssize_t i = 0; i < n; ++i) (*out)[(size_t)i] = usable(PySequence_Fast_GET_ITEM(params, i));
   } else {
-    return false;
+    if ((!PyList_CheckExact(params) && !PyTuple_CheckExact(params)) || PySequence_Fast_GET_SIZE(params) != n) return false;
+    for (Py_ssize_t i = 0; i < n; ++i)
+      if (!hold((size_t)i, PySequence_Fast_GET_ITEM(params, i))) return false;
   }
-  for (const at::Tensor* t : *out)
-    if (t == nullptr) return false;
+  PyObject *name, *value;
+  Py_ssize_t pos = 0;
+  while (PyDict_Next(by_name ? params : index, &pos, &name, &value)) {
+    if (!PyUnicode_CheckExact(name)) return false;
+    PyObject* at_index = PyDict_GetItemWithError(index, name);
+    if (at_index == nullptr) return false;
+    const size_t i = (size_t)PyLong_AsLong(at_index);
+    if (i >= (size_t)n || (by_name && !hold(i, value))) return false;
+    if (names != nullptr) names->emplace_back(THPObjectPtr::dup(name), i);
+  }
   return true;
 }
 
-bool model_data(const std::vector<const at::Tensor*>& tensors, std::vector<AITData>* out) {
-  for (const at::Tensor* t : tensors) {
+bool model_data(const std::vector<at::Tensor>& tensors, std::vector<AITData>* out) {
+  for (const at::Tensor& t : tensors) {
     AITData d;
-    d.ptr = t->data_ptr();
-    d.shape = AITemplateParamShape(t->sizes().data(), t->sizes().size());
-    if (!model_dtype(t->scalar_type(), &d.dtype)) return false;
+    d.ptr = t.data_ptr();
+    d.shape = AITemplateParamShape(t.sizes().data(), t.sizes().size());
+    if (!model_dtype(t.scalar_type(), &d.dtype)) return false;
     out->push_back(d);
   }
   return true;
@@ -379,8 +388,9 @@ PyObject* model_run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (nargs != 10 || !PyDict_CheckExact(args[2]) || !PyDict_CheckExact(args[3]) || !PyList_CheckExact(args[4]) ||
         !PyBool_Check(args[8]) || !PyBool_Check(args[9]))
       return not_ordinary();
-    std::vector<const at::Tensor*> in, out;
-    if (!model_tensors(args[5], args[2], &in) || !model_tensors(args[6], args[3], &out)) return not_ordinary();
+    std::vector<at::Tensor> in, out;
+    Names names;
+    if (!model_tensors(args[5], args[2], &in, nullptr) || !model_tensors(args[6], args[3], &out, &names)) return not_ordinary();
     std::vector<AITData> in_data, out_data;
     if (!model_data(in, &in_data) || !model_data(out, &out_data)) return not_ordinary();
     const size_t n_out = out.size();
@@ -390,7 +400,7 @@ PyObject* model_run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if ((size_t)PyList_GET_SIZE(args[4]) != n_out) return not_ordinary();
     for (size_t i = 0; i < n_out; ++i) {
       const int64_t rank = PyLong_AsLongLong(PyList_GET_ITEM(args[4], (Py_ssize_t)i));
-      if (rank != out[i]->dim() || dims.size() + (size_t)rank > dims.capacity()) return not_ordinary();
+      if (rank != out[i].dim() || dims.size() + (size_t)rank > dims.capacity()) return not_ordinary();
       shapes[i] = dims.data() + dims.size();
       dims.resize(dims.size() + (size_t)rank);
     }
@@ -405,25 +415,16 @@ PyObject* model_run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     });
     if (rc != 0) return PyErr_Format(PyExc_RuntimeError, "Error in function: AITemplateModelContainerRun");
     // every output under its name (a caller's dict keeps its order), as a view of the shape of this run
-    PyObject* result = PyDict_New();
-    if (result == nullptr) return nullptr;
-    PyObject *name, *at_index;
-    Py_ssize_t pos = 0;
-    PyObject* order = PyDict_CheckExact(args[6]) ? args[6] : args[3];
-    while (PyDict_Next(order, &pos, &name, &at_index)) {
-      const size_t i = (size_t)PyLong_AsLong(PyDict_GetItemWithError(args[3], name));
-      const at::Tensor& t = *out[i];
+    THPObjectPtr result(PyDict_New());
+    if (!result) return nullptr;
+    for (const auto& [name, i] : names) {
+      const at::Tensor& t = out[i];
       const at::IntArrayRef shape(shapes[i], (size_t)t.dim());
       const int64_t numel = c10::multiply_integers(shape);
-      PyObject* view = THPVariable_Wrap(numel == t.numel() ? t.view(shape) : t.flatten().narrow(0, 0, numel).view(shape));
-      if (view == nullptr || PyDict_SetItem(result, name, view) != 0) {
-        Py_XDECREF(view);
-        Py_DECREF(result);
-        return nullptr;
-      }
-      Py_DECREF(view);
+      THPObjectPtr view(THPVariable_Wrap(numel == t.numel() ? t.view(shape) : t.flatten().narrow(0, 0, numel).view(shape)));
+      if (!view || PyDict_SetItem(result.get(), const_cast<PyObject*>(name.get()), view.get()) != 0) return nullptr;
     }
-    return result;
+    return result.release();
   });
 }
 

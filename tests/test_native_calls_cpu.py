@@ -84,3 +84,45 @@ def test_wrappers_without_memory_of_their_own_are_declined(module, transform):
             torch.func.functionalize(declined)(q)
         assert launches() == 0
     """)
+
+
+@pytest.mark.parametrize("kind", ["dict", "list"])
+@pytest.mark.parametrize("change", ["replace", "remove", "clear"])
+def test_a_run_keeps_what_it_was_given(module, kind, change):
+    """The caller's containers may change while a run is on (the run gives up the interpreter lock): the
+    run's tensors live on, and the results are the ones it wrote."""
+    _run(module, f"""
+        import gc
+        RUN = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_size_t,
+                               ctypes.c_void_p, ctypes.c_bool, ctypes.c_bool, ctypes.POINTER(ctypes.POINTER(ctypes.c_int64)))
+        class AITData(ctypes.Structure):
+            _fields_ = [("ptr", ctypes.c_void_p), ("shape", ctypes.c_void_p), ("rank", ctypes.c_size_t), ("dtype", ctypes.c_int)]
+        names = {{"y": 1, "z": 0}}
+        fresh = lambda: {{"y": torch.zeros(4, 8), "z": torch.zeros(4)}}
+        outputs = fresh() if "{kind}" == "dict" else [fresh()["z"], fresh()["y"]]
+        inputs = {{"x": torch.ones(3)}} if "{kind}" == "dict" else [torch.ones(3)]
+        def run(handle, ins, n_in, outs, n_out, stream, sync, graph, shapes):
+            if "{change}" == "replace":
+                for key in (list(outputs) if "{kind}" == "dict" else range(2)):
+                    outputs[key] = torch.full((64,), 7.0)
+                for key in (list(inputs) if "{kind}" == "dict" else range(1)):
+                    inputs[key] = None
+            elif "{change}" == "remove":
+                outputs.pop("z" if "{kind}" == "dict" else 0)
+            else:
+                outputs.clear()
+                inputs.clear()
+            gc.collect()
+            hold.extend(torch.full((64,), 9.0) for _ in range(64))   # takes up memory that was given back
+            data = ctypes.cast(outs, ctypes.POINTER(AITData))
+            for i, numel in ((0, 2), (1, 16)):
+                ctypes.memmove(data[i].ptr, (ctypes.c_float * numel)(*[float(i + 1)] * numel), 4 * numel)
+            shapes[0][0], shapes[1][0], shapes[1][1] = 2, 2, 8
+            return 0
+        hold, callback = [], RUN(run)
+        result = native.model_run(ctypes.cast(callback, ctypes.c_void_p).value, 1, {{"x": 0}}, names, [1, 2], inputs, outputs,
+                                  None, True, False)
+        assert list(result) == ["y", "z"], result
+        assert torch.equal(result["y"], torch.full((2, 8), 2.0)) and torch.equal(result["z"], torch.ones(2))
+        assert all((t == 9).all() for t in hold)
+    """)
