@@ -6,13 +6,15 @@
 // with this module).  These
 // functions read the same attributes from the C++ tensors, allocate the result and call the same C ABI.
 //
-// They take ordinary arguments only: plain GPU tensors of one type whose shapes fit and whose rows are contiguous.
-// For anything else they return NotImplemented without having done anything, and the caller's Python path, which
-// handles the remaining cases and words the errors, takes the call.
+// They take ordinary arguments only: plain GPU tensors of one type whose shapes fit and whose rows are contiguous, and
+// outside of torch's modes.  For anything else they return NotImplemented without having done anything, and the caller's
+// Python path, which handles the remaining cases and words the errors, takes the call.
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 
 #include <ATen/Context.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 
 #include <cmath>
 #include <cstring>
@@ -71,7 +73,16 @@ int dtype_id(const at::Tensor& t) {
   return s == at::kHalf ? 0 : (s == at::kBFloat16 ? 1 : -1);
 }
 
-// results of torch.empty that torch would have to fill, or a mode that would see the allocation: not ordinary
+// False under a mode that sees, changes, records or refuses what the Python path does through torch (its allocation,
+// reshapes and views): dispatch modes, fake tensors among them, function modes (torch.set_default_device is one),
+// torch.func transforms, functionalization, tracing.  All but the function modes put a key of theirs into the thread's
+// dispatch keys; autocast, no_grad and inference mode put none.
+bool ordinary_context() {
+  return (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() &&
+      at::impl::PythonTorchFunctionTLS::stack_len() == 0;
+}
+
+// results of torch.empty that torch would have to fill are not ordinary
 bool plain_allocation() {
   return !(at::globalContext().deterministicAlgorithms() && at::globalContext().deterministicFillUninitializedMemory());
 }
@@ -102,7 +113,7 @@ PyObject* finish(int rc, const char* what, const at::Tensor* made, PyObject* out
 template <class F>
 PyObject* guarded(F&& body) {
   try {
-    return body();
+    return ordinary_context() ? body() : not_ordinary();
   } catch (const std::exception& e) {
     PyErr_SetString(PyExc_RuntimeError, e.what());
     return nullptr;

@@ -126,3 +126,48 @@ def test_a_run_keeps_what_it_was_given(module, kind, change):
         assert torch.equal(result["y"], torch.full((2, 8), 2.0)) and torch.equal(result["z"], torch.ones(2))
         assert all((t == 9).all() for t in hold)
     """)
+
+
+@pytest.mark.parametrize("mode", ["dispatch", "fake", "function", "vmap", "trace"])
+def test_calls_under_a_mode_are_declined(module, mode):
+    """The Python path's torch calls (its allocation, reshapes and views) are what a mode sees, refuses or records."""
+    _run(module, f"""
+        from torch._subclasses.fake_tensor import FakeTensorMode
+        from torch.overrides import TorchFunctionMode
+        from torch.utils._python_dispatch import TorchDispatchMode
+        class Dispatch(TorchDispatchMode):
+            def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+                return func(*args, **(kwargs or {{}}))
+        class Function(TorchFunctionMode):
+            def __torch_function__(self, func, types, args=(), kwargs=None):
+                return func(*args, **(kwargs or {{}}))
+        nowhere = 8   # an address that must not be called
+        y = torch.zeros(6, 72).half()
+        q4 = q[None]   # (arguments made outside of the mode)
+        def calls():
+            yield native.gemm("gemm_rcr", x, w, None, None, None, None, -1, None)
+            yield native.gemm("gemm_rcr", x, w, None, None, None, y, -1, None)
+            yield native.bmm(0, q, q, None, 0, -1, "bmm_rcr")
+            yield native.bmm_softmax_bmm_permute(q, q, q, 1, 0.125, False, None)
+            yield native.mem_eff_attention(q4, q4, q4, False, None, None, None)
+            yield native.model_run(nowhere, 1, {{"x": 0}}, {{"y": 0}}, [2], [x], [y], None, True, False)
+        declined = lambda: all(result is NotImplemented for result in calls())
+        if "{mode}" == "vmap":
+            seen = []
+            torch.vmap(lambda t: (seen.append(declined()), t)[1])(torch.zeros(2, 3))
+            assert seen == [True]
+        elif "{mode}" == "trace":
+            seen = []
+            torch.jit.trace(lambda t: (seen.append(declined()), t + 1)[1], (torch.zeros(3),), check_trace=False)
+            assert all(seen) and seen
+        else:
+            with dict(dispatch=Dispatch, fake=FakeTensorMode, function=Function)["{mode}"]():
+                assert declined()
+        assert launches() == 0
+        # and no longer once it is over, nor in what autograd and autocast modes leave to the kernels as before
+        with torch.inference_mode(), torch.autocast("cpu"):
+            assert native.gemm("gemm_rcr", x, w, None, None, None, None, -1, None).is_inference()
+        with torch.no_grad():
+            assert native.bmm(0, q, q, None, 0, -1, "bmm_rcr") is not NotImplemented
+        assert launches() == 2
+    """)
