@@ -9,6 +9,7 @@
 // They take ordinary arguments only: plain GPU tensors of one type whose shapes fit and whose rows are contiguous, and
 // outside of torch's modes.  For anything else they return NotImplemented without having done anything, and the caller's
 // Python path, which handles the remaining cases and words the errors, takes the call.
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 
@@ -110,14 +111,12 @@ PyObject* finish(int rc, const char* what, const at::Tensor* made, PyObject* out
   return out;
 }
 
+// torch's own translation of C++ exceptions: the types and texts that its bindings raise
 template <class F>
 PyObject* guarded(F&& body) {
-  try {
-    return ordinary_context() ? body() : not_ordinary();
-  } catch (const std::exception& e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
-  }
+  HANDLE_TH_ERRORS
+  return ordinary_context() ? body() : not_ordinary();
+  END_HANDLE_TH_ERRORS
 }
 
 // The launch itself runs without the interpreter lock, as it does through ctypes.  What it takes is plain pointers and

@@ -9,6 +9,7 @@ namespace {
 bool on_device(const at::Tensor& t) { return t.is_cpu(); }
 
 at::Tensor empty_like_device(at::IntArrayRef sizes, const at::Tensor& like) {
+  TORCH_CHECK_WITH(OutOfMemoryError, like.scalar_type() == at::kHalf, "host memory is out of bfloat16");
   return at::Tensor(at::detail::empty_cpu(sizes, like.scalar_type()));
 }
 

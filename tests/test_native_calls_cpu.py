@@ -171,3 +171,15 @@ def test_calls_under_a_mode_are_declined(module, mode):
             assert native.bmm(0, q, q, None, 0, -1, "bmm_rcr") is not NotImplemented
         assert launches() == 2
     """)
+
+
+def test_errors_keep_their_types(module):
+    """What torch raises through its own bindings: an allocation that fails is an OutOfMemoryError, without a C++ trace."""
+    _run(module, """
+        try:
+            native.gemm("gemm_rcr", x.bfloat16(), w.bfloat16(), None, None, None, None, -1, None)
+        except torch.OutOfMemoryError as e:
+            assert str(e) == "host memory is out of bfloat16", str(e)
+        else:
+            assert False
+    """)
