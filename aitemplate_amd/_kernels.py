@@ -13,6 +13,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 from typing import List, Optional
 
 _LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib")
@@ -173,26 +174,32 @@ def load() -> ctypes.CDLL:
         return lib
 
 
-class _MissingNative:
-    """Stands in for the extension module where it has not been built: every use raises."""
-
-    def __init__(self, why: str):
-        self._why = why
+class _NoNative:
+    """Stands in for the extension module where there is none: declines every call, as the module declines those that it
+    leaves to the Python path."""
 
     def __getattr__(self, name):
-        raise KernelLibraryMissing(f"the extension module aitemplate_amd._native cannot be loaded ({self._why}): build it "
-                                   "with `make -C aitemplate_amd/csrc -j8` (or __graft_entry__.build())")
+        return lambda *args: NotImplemented
 
 
 def load_native():
-    """The extension module of the eager calls and model runs (csrc/native_calls.cpp)."""
-    import torch  # noqa: F401  (its libraries have to be in the process first)
+    """The extension module of the eager calls and model runs (csrc/native_calls.cpp).  It holds no kernels and only
+    saves host time, so where it was not built, or was built for another torch, a warning says so and the Python code
+    behind every one of its calls takes them."""
+    import torch  # (its libraries have to be in the process first)
 
     try:
         from . import _native
+
+        built_for = getattr(_native, "torch_version", "unknown")
+        if built_for == torch.__version__.split("+")[0]:
+            return _native
+        why = f"it was built for torch {built_for}, this is {torch.__version__}"
     except ImportError as e:
-        return _MissingNative(str(e))
-    return _native
+        why = str(e)
+    warnings.warn(f"the extension module aitemplate_amd._native is not used ({why}): eager calls and model runs take 10 to 50 us "
+                  "longer; build it with `make -C aitemplate_amd/csrc -j8` (or __graft_entry__.build())", RuntimeWarning)
+    return _NoNative()
 
 
 def last_error() -> str:

@@ -12,6 +12,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
+#include <torch/headeronly/version.h>
 
 #include <ATen/Context.h>
 #include <ATen/PythonTorchFunctionTLS.h>
@@ -454,4 +455,9 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "Eager calls and model 
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native() { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__native() {
+  THPObjectPtr module(PyModule_Create(&kModule));
+  // (the loader compares it with the torch that is there)
+  if (!module || PyModule_AddStringConstant(module.get(), "torch_version", TORCH_VERSION) != 0) return nullptr;
+  return module.release();
+}

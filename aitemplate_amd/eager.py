@@ -9,7 +9,8 @@ a missing library or a CPU tensor raises.
 
 The calls with ordinary arguments (plain GPU tensors that fit, contiguous rows) go through the extension module
 ``_native`` (``csrc/native_calls.cpp``): the same checks and the same C ABI call, 2 to 3 us of host time instead of
-12 to 16.  It returns NotImplemented for anything else, which the Python code here then handles or refuses.
+12 to 16.  It returns NotImplemented for anything else, which the Python code here then handles or refuses; without
+the module that code takes every call.
 """
 from __future__ import annotations
 

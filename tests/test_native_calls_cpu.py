@@ -183,3 +183,54 @@ def test_errors_keep_their_types(module):
         else:
             assert False
     """)
+
+
+@pytest.mark.parametrize("why", ["not built", "built for another torch"])
+def test_without_the_extension_module_the_python_path_takes_every_call(why):
+    """The module saves host time and computes nothing: without it, calls and model runs do as before it was there."""
+    body = f"""
+        import ctypes, sys, types, warnings
+        import torch
+        sys.modules["aitemplate_amd._native"] = None
+        if "{why}" != "not built":
+            sys.modules["aitemplate_amd._native"] = types.ModuleType("aitemplate_amd._native")
+            sys.modules["aitemplate_amd._native"].torch_version = "1.0.0"
+            import aitemplate_amd
+            aitemplate_amd._native = sys.modules["aitemplate_amd._native"]
+        with warnings.catch_warnings(record=True) as seen:
+            warnings.simplefilter("always")
+            from aitemplate_amd import eager
+        assert any("_native" in str(w.message) for w in seen), seen
+        from aitemplate_amd.compiler import Model
+        x, q = torch.randn(2, 64).half(), torch.randn(1, 2, 5, 64).half()
+        calls = dict(gemm=lambda: eager.gemm("gemm_rcr", x, x), bmm_rcr=lambda: eager.bmm_rcr(q[0], q[0]),
+                     bmm=lambda: eager.bmm("rrr", q[0], q[0]), mem_eff=lambda: eager.mem_eff_attention(q, q, q),
+                     attention=lambda: eager.bmm_softmax_bmm_permute(q[0], q[0], q[0], (2,)))
+        for name, call in calls.items():
+            try:
+                call()
+            except ValueError as e:
+                assert "no CPU path" in str(e), (name, e)
+            else:
+                assert False, name
+        model = object.__new__(Model)
+        model.DLL = types.SimpleNamespace(is_open=True, close=lambda: None, DLL=types.SimpleNamespace(
+            AITemplateModelContainerRun=ctypes.CFUNCTYPE(ctypes.c_int)(lambda: 1)))
+        model.handle = model.allocator_handle = ctypes.c_void_p()
+        model._native_run, model._input_name_to_index, model._output_name_to_index, model._output_ndims = None, {{"x": 0}}, {{"y": 0}}, [2]
+        try:
+            model.run_with_tensors([x], [x])
+        except ValueError as e:
+            assert "contiguous and on GPU" in str(e), e
+        else:
+            assert False
+    """
+    done = subprocess.run([sys.executable, "-c", textwrap.dedent(body)], cwd=ROOT, text=True, stdout=subprocess.PIPE,
+                          stderr=subprocess.STDOUT, timeout=120)
+    assert done.returncode == 0, done.stdout
+
+
+def test_the_built_module_fits_this_torch():
+    from aitemplate_amd import _kernels
+
+    assert _kernels.load_native().torch_version == torch.__version__.split("+")[0]
