@@ -234,3 +234,17 @@ def test_the_built_module_fits_this_torch():
     from aitemplate_amd import _kernels
 
     assert _kernels.load_native().torch_version == torch.__version__.split("+")[0]
+
+
+def test_the_kernel_library_builds_without_torch(tmp_path):
+    """`make` builds everything but the extension module where python has no torch (or there is no python)."""
+    no_torch = tmp_path / "python3"
+    no_torch.write_text(f"#!/bin/sh\nexec {sys.executable} -S \"$@\"\n")   # (-S: no site-packages)
+    no_torch.chmod(0o755)
+    for python, built in ((sys.executable, True), (str(no_torch), False), (str(tmp_path / "none"), False)):
+        out = subprocess.run(["make", "-B", "-n", "-C", CSRC, f"PYTHON={python}"], text=True, stdout=subprocess.PIPE,
+                             stderr=subprocess.STDOUT)
+        assert out.returncode == 0, out.stdout[-2000:]
+        assert ("native_calls.cpp" in out.stdout) is built
+        assert "profiler_main.cpp" in out.stdout and "gemm_inst_0_0.o" in out.stdout
+        assert ("_native.so is not built" in out.stdout) is not built
