@@ -258,10 +258,12 @@ int profile_gemm_like(const std::string& op, int dtype, int64_t B, int64_t M, in
     } else if (!aitamd_gemm_algo_supported(epi, dtype, algo, M, N, K, K, K, 16)) {
       continue;
     }
-    // what other instances do better on every problem of the kind is not timed: loads in dwords where whole 16-byte
-    // pieces fit, the few-rows kernel for many rows
-    if (K % 8 == 0 && strstr(name, "_k2") && !strstr(name, "_rows")) continue;
-    if (M > 64 && strstr(name, "_rows")) continue;
+    // what other instances do better on every problem of the kind is not timed unless it is asked for: loads in dwords
+    // where whole 16-byte pieces fit, the few-rows kernel for many rows
+    if (!(only && *only)) {
+      if (K % 8 == 0 && strstr(name, "_k2") && !strstr(name, "_rows")) continue;
+      if (M > 64 && strstr(name, "_rows")) continue;
+    }
     const bool plain = !batched && !perm.layout && perm.operands == AITAMD_LAYOUT_RCR;
     const int64_t ws = plain ? aitamd_gemm_workspace_bytes(epi, dtype, algo, 1, M, N, K) : 0;
     if (!plain && strstr(name, "_splitk")) continue;  // (the other entry points take no scratch memory)

@@ -1,4 +1,7 @@
 """Instances for operands at any element and for few rows, at the edges of their tiles, slabs and pieces."""
+import os
+import subprocess
+
 import pytest
 import torch
 
@@ -62,3 +65,14 @@ def test_layouts_at_any_element(layout, B, M, N, K):
         torch.testing.assert_close(eager.bmm(layout, ad, bd, algo=algo).cpu().float(), want, atol=1e-2, rtol=1e-2)
         ran += 1
     assert ran >= 3
+
+
+# AITAMD_PROF_ALGO asks for one instance: it is timed also where the profiler by itself would leave it out
+@pytest.mark.parametrize("part,M,N,K", [("_k2", 64, 128, 256), ("rows", 128, 128, 256)])
+def test_profiler_times_the_instance_asked_for(part, M, N, K):
+    lib = _kernels.load()
+    name = next(n for i, n in enumerate(_kernels.gemm_algo_names(0, 0)) if part in n and "splitk" not in n
+                and lib.aitamd_gemm_algo_supported(0, 0, i, M, N, K, K, K, 16))
+    out = subprocess.run([os.path.join(os.path.dirname(_kernels.KERNEL_LIB_PATH), "aitamd_profiler"), "gemm", "gemm_rcr", "0", str(M),
+                          str(N), str(K)], env={**os.environ, "AITAMD_PROF_ALGO": name}, stdout=subprocess.PIPE, text=True, timeout=60)
+    assert out.returncode == 0 and out.stdout.startswith(f"OP:{name},TIME:") and out.stdout.count("OP:") == 1, out.stdout
