@@ -143,6 +143,13 @@ AITAMD_DEVICE float sum_across_halves(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// The row sum (of one lane's half of the keys) up to which probabilities may be taken against an old reference point;
+// beyond it, and at NaN, a tile is done again in the full form.  The accumulators hold the sum times the values, so
+// they stay finite for values up to 2^87; a bound near the largest float, which only the probabilities of bf16 get to
+// without being infinite, let the product with values above 1 overflow.  The full form itself lets a row's sum grow to
+// 2^8 a key (kLazyLog2), 2^39 for the most keys there can be, which therefore does not trip it.
+constexpr float kMaxRowSum = 0x1p40f;
+
 template <int N>
 AITAMD_DEVICE void attn_wait_vmcnt() {
   // s_waitcnt simm16: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt_hi[15:14]; only vmcnt is waited for
@@ -399,11 +406,11 @@ __global__ void __launch_bounds__(Tile::NT, 2) attention_kernel(const AttnParams
         };
         const float m_before = m_run, l_before = l_run;
         // Fast form of an unmasked block: no row maximum at all.  The probabilities are taken against the reference
-        // point the row already has, p = exp2((s - m) c); that is exact whatever m is, as long as no p leaves the
-        // element type's range, and a p beyond it shows as an infinite (or NaN) row sum, for which the block is
+        // point the row already has, p = exp2((s - m) c); that is exact whatever m is, as long as neither p nor its
+        // product with the values leaves its type's range, and a row sum that is NaN or beyond kMaxRowSum has the block
         // redone below in the full form (maximum, moved reference point, rescaled accumulators).  After a row's
         // first block - always the full form: there is no reference point yet - that takes a score 16 binary orders
-        // above everything the row has seen (fp16; never in practice for bf16), so nearly every block saves the
+        // above everything the row has seen (fp16; some 36 for bf16), so nearly every block saves the
         // maximum's 16 three-way compares, the exchange across the wave's halves and the bookkeeping of the
         // reference point: 96 instead of 128 vector instructions per 64 keys.
         bool full = need_mask || !ref_ok;
@@ -418,7 +425,7 @@ __global__ void __launch_bounds__(Tile::NT, 2) attention_kernel(const AttnParams
             }
             l_run = add_elements(pf[st], l_run);
           }
-          if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(l_run <= 3.0e38f)) != 0, 0)) {
+          if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(l_run <= kMaxRowSum)) != 0, 0)) {
             l_run = l_before;
             full = true;
           }

@@ -7,8 +7,8 @@
 //     S(t) = K(t) Q^T;   O += V(t-1) P(t-1)  and, between its matrix instructions,  P(t) = exp2(c S(t) - c m)
 // in one straight line, so the matrix unit works on tile t-1 while the exponentials of tile t are taken, and nothing
 // of the tile is waited for but its scores.  The V ring keeps one tile more than the K ring for it.
-//  * P against the reference point m the row already has (exact whatever m is, as long as no P leaves the element
-//    type's range; one that does shows as an infinite or NaN row sum, and the tile is done again in the full form).
+//  * P against the reference point m the row already has (exact whatever m is, as long as neither P nor its product with
+//    the values leaves its type's range; a row sum that is NaN or beyond kMaxRowSum has the tile done again in the full form).
 //  * full form: a row's first tile, tiles that reach past the keys or over the causal diagonal, NaN scores, and rows
 //    whose maximum has grown out of range: masks, maximum, moved reference point, rescaled accumulators.
 //  * NG groups of NW waves take alternate parts of a tile of NG x BN keys and merge at the end: for grids that leave
@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) attention_pipe_kernel(con
           }
           bool bad = false;
 #pragma unroll
-          for (int qb = 0; qb < QB; ++qb) bad = bad || !(l_run[qb] <= 3.0e38f);
+          for (int qb = 0; qb < QB; ++qb) bad = bad || !(l_run[qb] <= kMaxRowSum);
           if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0, 0)) {
 #pragma unroll
             for (int qb = 0; qb < QB; ++qb) l_run[qb] = l_before[qb];

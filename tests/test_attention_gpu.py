@@ -325,3 +325,21 @@ def test_forms_at_the_edges_of_their_tiles(attn_variant, mode, batch, heads, S, 
             print(f"case mode={mode} {dtype} causal={causal}", flush=True)
             _check_mem_eff(batch, heads, S, Skv, d, dv, [Skv - (i % 3) for i in range(batch)] if Skv > 2 else None, dtype=dtype,
                            causal=causal, seed=S)
+
+
+@pytest.mark.parametrize("mode", [-1, 0, 1, 2, 3])
+@pytest.mark.parametrize("K,O", [(64, 64), (40, 40), (128, 128), (20, 12)])   # (20, 12): the form for unaligned operands
+def test_bf16_scores_far_above_a_rows_first_keys(attn_variant, mode, K, O):
+    """A row's first 128 keys score 0, the others about 118 binary orders above: against the first keys' reference point
+    the row sum 384 * 2^118 still is a float, its product with values of 64 is not.  All late keys weigh the same, so the
+    result is the mean of their values (relative error 2^-8 of each rounded probability and of the result)."""
+    B, M, N, G = 4, 150, 512, 2
+    attn_variant(mode)
+    print(f"case bf16 late large scores mode={mode} K={K} O={O}", flush=True)
+    q = torch.ones(B, M, K, dtype=torch.bfloat16)
+    k = torch.zeros(B, N, K, dtype=torch.bfloat16)
+    k[:, 128:] = 82.0 / K   # a score of 82 is 82 log2(e) = 118.3 binary orders
+    v = (64 + _rand((B, N, O), torch.float32, 7)).bfloat16()
+    got = eager.bmm_softmax_bmm_permute(q.cuda(), k.cuda(), v.cuda(), (G,), scale=1.0).cpu().float()
+    want = v[:, 128:].float().mean(1).reshape(B // G, 1, G, O).expand(B // G, M, G, O)
+    torch.testing.assert_close(got, want, atol=0.0, rtol=2 ** -7)
