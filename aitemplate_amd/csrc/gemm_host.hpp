@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "device.hpp"
 #include "gemm_kernel.hpp"
 
 namespace aitamd {
@@ -44,28 +45,6 @@ inline int split_k_rule(int64_t tiles, int64_t k_tiles, int cus) {
   if (s > k_tiles / 2) s = k_tiles / 2;
   if (s > 16) s = 16;
   return (int)(s < 1 ? 1 : s);
-}
-
-// Compute units of a device, looked up once per device (256 where the device cannot be asked).  The launcher's grid
-// and split-K factor and the instance choice all use this one figure.
-inline int device_cus(int dev) {
-  constexpr int kSlots = 64;
-  static int cus[kSlots] = {};
-  if (dev < 0) dev = 0;
-  int v = cus[dev % kSlots];
-  if (v == 0) {
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || v <= 0) v = 256;
-    cus[dev % kSlots] = v;
-  }
-  return v;
-}
-inline int current_device_cus() {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) {
-    (void)hipGetLastError();  // no device: the instance choice still answers, priced for a 256-CU part
-    return 256;
-  }
-  return device_cus(dev);
 }
 
 // Defined once per (epilogue, dtype) translation unit; nullptr table when that

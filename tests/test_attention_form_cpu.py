@@ -1,0 +1,47 @@
+"""The choice of an attention form (csrc/attention_form.hpp), host code compiled and called here."""
+import ctypes
+import os
+import random
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "aitemplate_amd", "csrc")
+ROWS128, ROWS256, GROUPS, SMALL, ROWS64 = range(5)
+
+
+@pytest.fixture(scope="module")
+def choose(tmp_path_factory):
+    build = tmp_path_factory.mktemp("form")
+    (build / "form.cpp").write_text("""
+        #include "attention_form.hpp"
+        extern "C" int choose(int64_t B, int64_t M, int64_t N, int ks, int ot, int causal, int cus, int32_t* paired) {
+          return aitamd::choose_form(B, M, N, ks, ot, causal != 0, cus, paired);
+        }""")
+    subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", "-I" + CSRC, str(build / "form.cpp"), "-o", str(build / "form.so")], check=True)
+    fn = ctypes.CDLL(str(build / "form.so")).choose
+    fn.argtypes = [ctypes.c_int64] * 3 + [ctypes.c_int] * 4 + [ctypes.POINTER(ctypes.c_int32)]
+
+    def call(B, M, N, d, causal, cus):
+        paired = ctypes.c_int32(0)
+        return fn(B, M, N, (d + 15) // 16, (d + 31) // 32, causal, cus, ctypes.byref(paired)), paired.value
+    return call
+
+
+# (batch x heads, queries, keys, head dim, causal) on 256 CUs, around the measured lines
+@pytest.mark.parametrize("case,form,paired", [
+    ((12, 384, 384, 64, 0), SMALL, 0), ((66, 384, 384, 64, 0), SMALL, 0), ((67, 384, 384, 64, 0), ROWS128, 0),
+    ((72, 316, 77, 128, 0), ROWS128, 0), ((992, 34, 34, 64, 0), ROWS64, 0), ((12, 2048, 2048, 64, 0), SMALL, 0),
+    ((16, 2000, 2000, 128, 0), GROUPS, 0), ((16, 8192, 8192, 64, 0), ROWS256, 0), ((16, 4096, 4096, 40, 0), ROWS128, 0),
+    ((64, 2048, 2048, 64, 1), ROWS128, 1), ((16, 4096, 4096, 40, 1), GROUPS, 1), ((32, 4096, 4096, 128, 1), ROWS128, 1),
+    ((24, 900, 900, 64, 1), SMALL, 0)])
+def test_lines_on_256_cus(choose, case, form, paired):
+    assert choose(*case, 256) == (form, paired)
+
+
+def test_lines_move_with_the_number_of_cus(choose):
+    """An eighth of the CUs takes an eighth of the batch the same way."""
+    rng = random.Random(0)
+    for _ in range(3000):
+        B, M, N, d, causal = rng.randint(1, 200), rng.randint(1, 5000), rng.randint(1, 5000), rng.choice([40, 64, 128]), rng.randint(0, 1)
+        assert choose(B, M, N, d, causal, 32) == choose(8 * B, M, N, d, causal, 256), (B, M, N, d, causal)
