@@ -17,7 +17,7 @@ namespace {
 
 constexpr int kMaxDevices = 64;
 
-// Variant forced by aitamd_attention_set_variant: -1 automatic, 0..3 a Form below.  The environment variable
+// Variant forced by aitamd_attention_set_variant: -1 automatic, 0..4 a Form (attention_form.hpp).  The environment variable
 // AITAMD_ATTN_MODE gives the initial value and is read once, not on every launch.
 constexpr int kVariantUnset = -2;
 std::atomic<int> g_forced_variant{kVariantUnset};
@@ -26,7 +26,7 @@ int forced_variant() {
   if (m == kVariantUnset) {
     const char* env = getenv("AITAMD_ATTN_MODE");
     const int from_env = env ? atoi(env) : -1;
-    g_forced_variant.compare_exchange_strong(m, from_env >= 0 && from_env <= 3 ? from_env : -1);
+    g_forced_variant.compare_exchange_strong(m, from_env >= 0 && from_env <= kRows64 ? from_env : -1);
     m = g_forced_variant.load(std::memory_order_relaxed);
   }
   return m;
@@ -202,7 +202,7 @@ int attention_entry(const char* who, int dtype, const void* q, const void* k, co
   AttnLaunch fn = nullptr;
   if (dma) {
     int form = choose_form(B, M, N, ks, ot, causal != 0, current_device_cus(), &p.paired);
-    // aitamd_attention_set_variant(0|1|2|3) forces a form (a test and measurement knob)
+    // aitamd_attention_set_variant(0|1|2|3|4) forces a form (a test and measurement knob)
     if (forced_variant() >= 0) form = forced_variant();
     if (form == kRows256) p.paired = 0;
     fn = dtype == 0 ? pick_pipe<f16>(form, ks, ot) : pick_pipe<bf16>(form, ks, ot);
@@ -220,7 +220,8 @@ int attention_entry(const char* who, int dtype, const void* q, const void* k, co
 }  // namespace
 
 extern "C" int aitamd_attention_set_variant(int variant) {
-  if (variant < -1 || variant > 3) return fail("aitamd_attention_set_variant: variant %d is not one of -1, 0, 1, 2, 3", variant);
+  if (variant < -1 || variant > kRows64)
+    return fail("aitamd_attention_set_variant: variant %d is not one of -1, 0, 1, 2, 3, 4", variant);
   g_forced_variant.store(variant, std::memory_order_relaxed);
   return 0;
 }

@@ -257,9 +257,9 @@ AITAMD_API int aitamd_mem_eff_attention(int dtype,
                                         int64_t head_dim, int64_t head_dim_v, float scale, int causal,
                                         const int32_t* lengths_kv, const int32_t* lengths_q, void* stream);
 
-/* Test and measurement knob of the two attention entry points above: force one of the kernel's four work
+/* Test and measurement knob of the two attention entry points above: force one of the kernel's five work
  * decompositions wherever the shape allows it (0: four waves of 32 query rows; 1: of 64 rows, at head dims up to 64;
- * 2: as 0 with two wave groups that share the keys; 3: two groups of two waves), or -1 (the default) to let
+ * 2: as 0 with two wave groups that share the keys; 3: two groups of two waves; 4: two waves of 32 rows), or -1 (the default) to let
  * the launcher choose from the shape.  Process-wide; the results are the same in every variant up to rounding.
  * The environment variable AITAMD_ATTN_MODE sets the initial value and is read once.  No counterpart in the
  * reference (CK instances are chosen by its profiler only). */

@@ -55,7 +55,7 @@ def test_ragged_and_odd_shapes(B, M, N, K, O, G, causal):
     _check(B, M, N, K, O, G, causal, seed=3)
 
 
-@pytest.mark.parametrize("mode", [0, 1, 2, 3])
+@pytest.mark.parametrize("mode", [0, 1, 2, 3, 4])
 @pytest.mark.parametrize("B,M,N,K,O,G,causal,scale", [
     (8, 300, 1000, 40, 40, 4, False, None),    # 8 key tiles: both wave groups busy
     (8, 300, 900, 40, 40, 4, True, None),      # causal: workgroups stop at different tiles
@@ -65,8 +65,8 @@ def test_ragged_and_odd_shapes(B, M, N, K, O, G, causal):
     (2, 260, 0, 40, 40, 2, False, None),       # no keys at all
 ])
 def test_every_variant_of_the_small_head_dims(attn_variant, mode, B, M, N, K, O, G, causal, scale):
-    # aitamd_attention_set_variant picks the variant where the shape allows it: 0 four waves, 1 eight waves, 2 (3) two groups of
-    # eight (four) waves that take alternate key tiles and merge their running sums at the end
+    # aitamd_attention_set_variant picks the variant where the shape allows it: 0 four waves, 1 four waves of 64 rows, 2 (3) two
+    # groups of four (two) waves that take alternate parts of a key tile and merge their running sums at the end, 4 two waves
     attn_variant(mode)
     print(f"case attention mode={mode} B={B} M={M} N={N} K={K} causal={causal} scale={scale}", flush=True)
     _check(B, M, N, K, O, G, causal=causal, scale=scale, seed=mode + N)
@@ -145,7 +145,7 @@ def _check_mem_eff(batch, heads, S, Skv, d, dv, lens, causal=False, dtype=torch.
     torch.testing.assert_close(got.cpu().float(), want, atol=TOL, rtol=TOL)
 
 
-@pytest.mark.parametrize("mode", [None, 0, 1, 2, 3])
+@pytest.mark.parametrize("mode", [None, 0, 1, 2, 3, 4])
 @pytest.mark.parametrize("batch,heads,S,Skv,d,dv,lens,causal", [
     (4, 2, 300, 1000, 40, 40, [1000, 517, 128, 1], False),   # whole tiles, a ragged last tile, one key
     (4, 2, 300, 900, 40, 40, [900, 300, 77, 0], True),       # causal bound and key length, whichever is shorter
@@ -171,7 +171,7 @@ def test_mem_eff_attention_shapes_and_dtypes(dtype, batch, heads, S, Skv, d, dv,
     _check_mem_eff(batch, heads, S, Skv, d, dv, lens, dtype=dtype, seed=d)
 
 
-@pytest.mark.parametrize("mode", [None, 0, 1, 2, 3])
+@pytest.mark.parametrize("mode", [None, 0, 1, 2, 3, 4])
 @pytest.mark.parametrize("causal", [False, True])
 def test_mem_eff_attention_query_lengths(attn_variant, mode, causal):
     """Rows past a query length are zeros (whole blocks of them visit no keys), the rows before are unchanged."""
@@ -284,7 +284,7 @@ def test_nan_key_and_lengths_at_head_dim_40(attn_variant):
     k[1, 650, 1] = float("nan")
     want = oracle.torch_bmm_softmax_bmm_permute(q, k, v, K ** -0.5, G, False).half().float()
     assert not torch.isnan(want).any()
-    for mode in (-1, 0, 1, 2, 3):
+    for mode in (-1, 0, 1, 2, 3, 4):
         attn_variant(mode)
         print(f"case attention NaN reset head dim 40 variant {mode}", flush=True)
         got = eager.bmm_softmax_bmm_permute(q.cuda(), k.cuda(), v.cuda(), (G,), scale=K ** -0.5).cpu().float()
@@ -314,7 +314,7 @@ def test_causal_pairs_of_query_tiles(batch, heads, S, d):
 
 # the pipelined kernel's forms at the edges of their tiles (32 and 64 keys, 64, 128 and 256 rows), head dims from one
 # matrix instruction to the widest, and the rules' own choices from a single row up
-@pytest.mark.parametrize("mode", [None, 0, 1, 2, 3])
+@pytest.mark.parametrize("mode", [None, 0, 1, 2, 3, 4])
 @pytest.mark.parametrize("batch,heads,S,Skv,d,dv", [(1, 3, 1, 1, 64, 64), (2, 2, 33, 31, 8, 16), (1, 2, 64, 65, 64, 64), (1, 2, 129, 97, 128, 128),
                                                     (2, 1, 257, 256, 40, 40), (1, 1, 100, 161, 160, 152), (70, 8, 31, 33, 64, 64), (1, 2, 63, 700, 96, 88)])
 def test_forms_at_the_edges_of_their_tiles(attn_variant, mode, batch, heads, S, Skv, d, dv):
@@ -327,7 +327,7 @@ def test_forms_at_the_edges_of_their_tiles(attn_variant, mode, batch, heads, S, 
                            causal=causal, seed=S)
 
 
-@pytest.mark.parametrize("mode", [-1, 0, 1, 2, 3])
+@pytest.mark.parametrize("mode", [-1, 0, 1, 2, 3, 4])
 @pytest.mark.parametrize("K,O", [(64, 64), (40, 40), (128, 128), (20, 12)])   # (20, 12): the form for unaligned operands
 def test_bf16_scores_far_above_a_rows_first_keys(attn_variant, mode, K, O):
     """A row's first 128 keys score 0, the others about 118 binary orders above: against the first keys' reference point
