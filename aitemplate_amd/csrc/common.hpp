@@ -15,12 +15,10 @@ using bf16 = __bf16;
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
@@ -124,14 +122,8 @@ AITAMD_DEVICE __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t num_by
 AITAMD_DEVICE u32x4 buffer_load_16B(__amdgpu_buffer_rsrc_t r, uint32_t voffset) {
   return __builtin_amdgcn_raw_buffer_load_b128(r, voffset, 0, 0);
 }
-AITAMD_DEVICE u32x2 buffer_load_8B(__amdgpu_buffer_rsrc_t r, uint32_t voffset) {
-  return __builtin_amdgcn_raw_buffer_load_b64(r, voffset, 0, 0);
-}
 AITAMD_DEVICE uint32_t buffer_load_4B(__amdgpu_buffer_rsrc_t r, uint32_t voffset) {
   return __builtin_amdgcn_raw_buffer_load_b32(r, voffset, 0, 0);
-}
-AITAMD_DEVICE uint16_t buffer_load_2B(__amdgpu_buffer_rsrc_t r, uint32_t voffset) {
-  return __builtin_amdgcn_raw_buffer_load_b16(r, voffset, 0, 0);
 }
 
 // A vector at an address of element alignment: one load or store (the gfx950 target reads and writes global memory
