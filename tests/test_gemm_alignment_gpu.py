@@ -67,6 +67,45 @@ def test_layouts_at_any_element(layout, B, M, N, K):
     assert ran >= 3
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("layout", ["rcr", "rrr", "ccr", "crr"])
+@pytest.mark.parametrize("B,M,N,K", [(3, 127, 129, 65), (2, 33, 255, 7), (2, 64, 64, 128)])
+def test_layouts_between_guards(layout, B, M, N, K, dtype):
+    """Operands one element into their buffers, rows 3 and batches 5 elements apart, NaN in every gap: only the operands
+    count.  The result's buffer keeps what lies around and between its rows."""
+    lib = _kernels.load()
+    lay, dt = _kernels.LAYOUT_ID[layout], 0 if dtype == torch.float16 else 1
+    a = _rand((B, K, M) if layout[0] == "c" else (B, M, K), 1, dtype=dtype)
+    b = _rand((B, N, K) if layout[1] == "c" else (B, K, N), 2, K ** -0.5, dtype)
+    want = oracle.torch_bmm(layout, a, b).to(dtype).float()
+    tol = 1e-2 if dt == 0 else 3e-2
+
+    def placed(shape, fill):
+        pitch = shape[2] + 3
+        stride = shape[1] * pitch + 5
+        buffer = torch.full((1 + shape[0] * stride,), fill, dtype=dtype, device="cuda")
+        return buffer, buffer[1:].as_strided(shape, (stride, pitch, 1), 1), pitch, stride
+
+    _, av, lda, sa = placed(a.shape, float("nan"))
+    _, bv, ldb, sb = placed(b.shape, float("nan"))
+    av.copy_(a)
+    bv.copy_(b)
+    ran = 0
+    for algo, name in _instances(0, dt):
+        if not lib.aitamd_gemm_algo_supported_layout(0, dt, lay, algo, M, N, K, lda, ldb, 2):
+            continue
+        print(f"case bmm_{layout} instance={name} B={B} M={M} N={N} K={K} {dtype}", flush=True)
+        buffer, cv, ldc, sc = placed((B, M, N), 7.0)
+        rc = lib.aitamd_bmm(lay, dt, algo, av.data_ptr(), bv.data_ptr(), cv.data_ptr(), B, M, N, K, lda, ldb, ldc, sa, sb, sc, 0,
+                            torch.cuda.current_stream().cuda_stream)
+        _kernels.check(rc, name)
+        torch.testing.assert_close(cv.cpu().float(), want, atol=tol, rtol=tol)
+        cv.fill_(7.0)
+        assert (buffer == 7.0).all(), name
+        ran += 1
+    assert ran >= 3
+
+
 # AITAMD_PROF_ALGO asks for one instance: it is timed also where the profiler by itself would leave it out
 @pytest.mark.parametrize("part,M,N,K", [("_k2", 64, 128, 256), ("rows", 128, 128, 256)])
 def test_profiler_times_the_instance_asked_for(part, M, N, K):
