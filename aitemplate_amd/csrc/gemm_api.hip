@@ -39,7 +39,7 @@ bool algo_supported(const GemmAlgo& a, int64_t M, int64_t N, int64_t K, int64_t 
   if (align_bytes < kv * 2) return false;
   // an operand that is K-contiguous is fetched in pieces of kv elements along K; a transposed one in
   // 16-byte pieces along its rows of M (or N) elements, which only constrains its row pitch
-  // (the register-staged instance reads a transposed operand element by element: any pitch)
+  // (the register-staged instances read it in 16-byte pieces too, but at any address: any pitch)
   // With a padded pitch and M (or N) not a multiple of 8 the last 16-byte piece of k-row K-1 would reach past the
   // end of the operand (and of its buffer descriptor), so the row length has to be whole pieces as well.
   const int tv = a.direct_lds ? 8 : 1;
@@ -181,7 +181,7 @@ int run_gemm(int epilogue, int dtype, int algo, const GemmParams& p, hipStream_t
   }
   if (algo < 0) {
     algo = remembered_heuristic(t, p.batch, p.M, p.N, p.K, p.lda, p.ldb, align, p.layout, p.ws != nullptr && p.perm_on == 0);
-    // (the heuristic prices stream-K on the grid it would get; a buffer too small for that falls back)
+    // (the heuristic prices split-K with the split it would get; a buffer too small for that falls back)
     if (algo >= 0 && t.algos[algo].workspace_bytes && t.algos[algo].workspace_bytes(p) > p.ws_bytes)
       algo = remembered_heuristic(t, p.batch, p.M, p.N, p.K, p.lda, p.ldb, align, p.layout, false);
     if (algo < 0) return fail("aitamd_gemm: no instance supports M=%d N=%d K=%d", p.M, p.N, p.K);

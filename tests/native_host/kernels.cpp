@@ -1,15 +1,18 @@
-// The entry points of the kernel library that native_calls.cpp calls, without kernels: they count their calls.
+// The entry points of the kernel library that native_calls.cpp calls, without kernels: they count their calls and keep
+// the last epilogue.
 #include "../../include/aitemplate_amd_kernels.h"
 
 extern "C" {
 
 __attribute__((visibility("default"))) int stub_launches = 0;
+__attribute__((visibility("default"))) int stub_epilogue = -1;
 
 const char* aitamd_last_error(void) { return "stub"; }
 
-int aitamd_gemm_rcr_ws(int, int, int, const void*, const void*, const void*, const void*, const void*, void*, int64_t, int64_t,
+int aitamd_gemm_rcr_ws(int epilogue, int, int, const void*, const void*, const void*, const void*, const void*, void*, int64_t, int64_t,
                        int64_t, int64_t, int64_t, int64_t, int64_t, void*, int64_t, void*) {
   ++stub_launches;
+  stub_epilogue = epilogue;
   return 0;
 }
 

@@ -67,6 +67,22 @@ def test_ordinary_calls_launch(module):
     """)
 
 
+def test_op_table_is_the_python_paths(module):
+    _run(module, """
+        from aitemplate_amd import _kernels
+        bias, d = torch.zeros(72).half(), torch.zeros(6, 72).half()
+        for op, epilogue in _kernels.EPILOGUE_OF_OP.items():
+            if op == "bmm_rcr":
+                continue
+            residuals = _kernels.NUM_RESIDUALS_OF_EPILOGUE[epilogue]
+            args = [bias if epilogue else None, d if residuals >= 1 else None, d if residuals >= 2 else None]
+            assert native.gemm(op, x, w, *args, None, -1, None) is not NotImplemented, op
+            assert ctypes.c_int.in_dll(stub, "stub_epilogue").value == epilogue, op
+            if residuals:
+                assert native.gemm(op, x, w, bias, None, None, None, -1, None) is NotImplemented, op
+    """)
+
+
 @pytest.mark.parametrize("transform", ["vmap", "grad", "functionalize"])
 def test_wrappers_without_memory_of_their_own_are_declined(module, transform):
     """torch.func's tensors are of the exact type torch.Tensor and have no storage: the Python path words the error."""
