@@ -15,6 +15,7 @@
 #include <torch/headeronly/version.h>
 
 #include <ATen/Context.h>
+#include <ATen/core/DimVector.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 
@@ -382,13 +383,21 @@ bool model_tensors(PyObject* params, PyObject* index, std::vector<at::Tensor>* o
   return true;
 }
 
-bool model_data(const std::vector<at::Tensor>& tensors, std::vector<AITData>* out) {
-  for (const at::Tensor& t : tensors) {
-    AITData d;
+// What a run gets of its tensors.  The sizes are copied: a tensor's own move when it is given another shape.
+struct ModelData {
+  std::vector<AITData> data;
+  std::vector<c10::DimVector> sizes;
+};
+bool model_data(const std::vector<at::Tensor>& tensors, ModelData* out) {
+  out->data.resize(tensors.size());
+  out->sizes.reserve(tensors.size());
+  for (size_t i = 0; i < tensors.size(); ++i) {
+    const at::Tensor& t = tensors[i];
+    const c10::DimVector& sizes = out->sizes.emplace_back(t.sizes().begin(), t.sizes().end());
+    AITData& d = out->data[i];
     d.ptr = t.data_ptr();
-    d.shape = AITemplateParamShape(t.sizes().data(), t.sizes().size());
+    d.shape = AITemplateParamShape(sizes.data(), sizes.size());
     if (!model_dtype(t.scalar_type(), &d.dtype)) return false;
-    out->push_back(d);
   }
   return true;
 }
@@ -402,7 +411,7 @@ PyObject* model_run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     std::vector<at::Tensor> in, out;
     Names names;
     if (!model_tensors(args[5], args[2], &in, nullptr) || !model_tensors(args[6], args[3], &out, &names)) return not_ordinary();
-    std::vector<AITData> in_data, out_data;
+    ModelData in_data, out_data;
     if (!model_data(in, &in_data) || !model_data(out, &out_data)) return not_ordinary();
     const size_t n_out = out.size();
     std::vector<int64_t> dims;
@@ -411,7 +420,7 @@ PyObject* model_run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if ((size_t)PyList_GET_SIZE(args[4]) != n_out) return not_ordinary();
     for (size_t i = 0; i < n_out; ++i) {
       const int64_t rank = PyLong_AsLongLong(PyList_GET_ITEM(args[4], (Py_ssize_t)i));
-      if (rank != out[i].dim() || dims.size() + (size_t)rank > dims.capacity()) return not_ordinary();
+      if (rank != (int64_t)out_data.sizes[i].size() || dims.size() + (size_t)rank > dims.capacity()) return not_ordinary();
       shapes[i] = dims.data() + dims.size();
       dims.resize(dims.size() + (size_t)rank);
     }
@@ -421,7 +430,7 @@ PyObject* model_run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (PyErr_Occurred()) return nullptr;
     const bool sync = args[8] == Py_True, graph = args[9] == Py_True;
     const int rc = unlocked([&] {
-      return (int)run(handle, in_data.data(), in_data.size(), out_data.data(), n_out,
+      return (int)run(handle, in_data.data.data(), in.size(), out_data.data.data(), n_out,
                       reinterpret_cast<AITemplateStreamHandle>(stream), sync, graph, shapes.data());
     });
     if (rc != 0) return PyErr_Format(PyExc_RuntimeError, "Error in function: AITemplateModelContainerRun");
@@ -430,7 +439,7 @@ PyObject* model_run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!result) return nullptr;
     for (const auto& [name, i] : names) {
       const at::Tensor& t = out[i];
-      const at::IntArrayRef shape(shapes[i], (size_t)t.dim());
+      const at::IntArrayRef shape(shapes[i], out_data.sizes[i].size());
       const int64_t numel = c10::multiply_integers(shape);
       THPObjectPtr view(THPVariable_Wrap(numel == t.numel() ? t.view(shape) : t.flatten().narrow(0, 0, numel).view(shape)));
       if (!view || PyDict_SetItem(result.get(), const_cast<PyObject*>(name.get()), view.get()) != 0) return nullptr;

@@ -144,6 +144,33 @@ def test_a_run_keeps_what_it_was_given(module, kind, change):
     """)
 
 
+def test_a_run_keeps_the_shapes_it_was_given(module):
+    """A tensor that is given another shape while a run is on: the run's pointers to shapes stay what they were."""
+    _run(module, """
+        RUN = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_size_t,
+                               ctypes.c_void_p, ctypes.c_bool, ctypes.c_bool, ctypes.POINTER(ctypes.POINTER(ctypes.c_int64)))
+        class AITData(ctypes.Structure):
+            _fields_ = [("ptr", ctypes.c_void_p), ("shape", ctypes.POINTER(ctypes.c_int64)), ("rank", ctypes.c_size_t),
+                        ("dtype", ctypes.c_int)]
+        a, b, y = torch.ones(3, 4), torch.ones(5), torch.zeros(4, 8)
+        seen = []
+        def run(handle, ins, n_in, outs, n_out, stream, sync, graph, shapes):
+            a.resize_(1, 2, 3, 2, 1, 1, 1)
+            b.resize_(5, 1)
+            y.resize_(2, 2, 2, 2, 2, 1, 1)
+            data = ctypes.cast(ins, ctypes.POINTER(AITData))
+            for d in (data[0], data[1], ctypes.cast(outs, ctypes.POINTER(AITData))[0]):
+                seen.append([d.shape[i] for i in range(d.rank)])
+            shapes[0][0], shapes[0][1] = 3, 8
+            return 0
+        callback = RUN(run)
+        result = native.model_run(ctypes.cast(callback, ctypes.c_void_p).value, 1, {"a": 0, "b": 1}, {"y": 0}, [2], [a, b], [y],
+                                  None, True, False)
+        assert seen == [[3, 4], [5], [4, 8]], seen
+        assert result["y"].shape == (3, 8)
+    """)
+
+
 @pytest.mark.parametrize("mode", ["dispatch", "fake", "function", "vmap", "trace"])
 def test_calls_under_a_mode_are_declined(module, mode):
     """The Python path's torch calls (its allocation, reshapes and views) are what a mode sees, refuses or records."""
