@@ -47,10 +47,12 @@ bool algo_supported(const GemmAlgo& a, int64_t M, int64_t N, int64_t K, int64_t 
   if (b_t ? (ldb % tv != 0 || N % tv != 0 || ldb < N) : (K % kv != 0 || ldb % kv != 0)) return false;
   // Per-tile byte offsets are 32-bit, with the top bit reserved for "out of range".
   if ((a_t ? K * lda : (int64_t)a.bm * lda) * 2 >= 0x7fffffffll) return false;
-  if ((b_t ? K * ldb : (int64_t)a.bn * ldb) * 2 >= 0x7fffffffll) return false;
+  if ((b_t ? K * ldb : (int64_t)(a.direct_lds == 16 ? 256 : a.bn) * ldb) * 2 >= 0x7fffffffll) return false;
   if (M > 0x7fffffffll || K > 0x3fffffffll) return false;
   // the persistent kernels write a tile when its last K-slab has been multiplied: they need one
   if (a.direct_lds == 2 && K < 1) return false;
+  // the four-wave kernels are built of three slab pairs at least, and store whole 16-byte pieces
+  if (a.direct_lds == 16 && ((kv == 8 ? K : (K & ~7ll)) <= 128 || N % 8 != 0)) return false;
   return true;
 }
 
@@ -87,7 +89,7 @@ int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64
     const GemmAlgo& a = t.algos[i];
     if (!algo_supported(a, M, N, K, lda, ldb, align_bytes, layout)) continue;
     // (the dword-aligned twins of the direct-to-LDS tiles are for what the 16-byte ones cannot take)
-    if (a.kvec == 2 && (a.direct_lds & 5) != 0 && align_bytes >= 16 && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0) continue;
+    if (a.kvec == 2 && (a.direct_lds & 21) != 0 && align_bytes >= 16 && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0) continue;
     int64_t slabs = ((a.kvec == 2 && a.direct_lds != 8 ? K & ~7ll : K) + a.bk - 1) / a.bk;
     int64_t tiles = ((M + a.bm - 1) / a.bm) * ((N + a.bn - 1) / a.bn) * batches;
     double cost = a.cost.start;

@@ -10,6 +10,7 @@
 #include "gemm_kernel_dma.hpp"
 #include "gemm_kernel_persist.hpp"
 #include "gemm_kernel_rows.hpp"
+#include "gemm_kernel_wide.hpp"
 
 #ifndef AITAMD_EPI
 #error "compile with -DAITAMD_EPI=<id>"
@@ -62,6 +63,10 @@ template <int MT, int NW, int U, int ELEM, bool PERM, int LAYOUT>
 struct KernelOf<GemmTileRows<MT, NW, U, ELEM>, PERM, LAYOUT> {
   static constexpr auto value = gemm_rcr_rows_kernel<Elem, GemmTileRows<MT, NW, U, ELEM>, Epi, PERM>;
 };
+template <int MI, int NI, int KTAIL, bool PERM, int LAYOUT>
+struct KernelOf<GemmTileWide<MI, NI, KTAIL>, PERM, LAYOUT> {
+  static constexpr auto value = gemm_rcr_wide_kernel<Elem, GemmTileWide<MI, NI, KTAIL>, Epi>;
+};
 // the slab-pair form of a persistent tile (the tile itself where it has none)
 template <class Tile>
 struct PairOf {
@@ -104,6 +109,15 @@ struct IsPersistent {
 };
 template <int BM, int BN, int BK, int WM, int WN, int NS, int MT, int LBM, int PAIR>
 struct IsPersistent<GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM, PAIR>> {
+  static constexpr bool value = true;
+};
+
+template <class Tile>
+struct IsWide {
+  static constexpr bool value = false;
+};
+template <int MI, int NI, int KTAIL>
+struct IsWide<GemmTileWide<MI, NI, KTAIL>> {
   static constexpr bool value = true;
 };
 
@@ -180,14 +194,16 @@ hipError_t launch_kernel(const GemmParams& p_in, hipStream_t stream) {
   const int64_t total = tiles * p.batch;
   if (total > 0x7fffffffll) return hipErrorInvalidValue;
   dim3 grid((unsigned)total, 1, 1);
-  if constexpr (IsPersistent<Tile>::value) {
+  if constexpr (IsPersistent<Tile>::value || IsWide<Tile>::value) {
     const int cus = device_cus(dev);
     grid = dim3((unsigned)(total < cus ? total : cus), 1, 1);
     p.xcd_cols = xcd_column_blocks(p, Tile::BN, (int)grid.x);
     // few tile columns: the grouped walk goes row by row, so that the run of tiles of an XCD ends inside at most
     // one row of tiles whose A panel a second XCD then fetches too (eight rows with the default group height;
     // measured on M=24576 N=768 K=3072 and M=12608 N=1024 K=4096: 1 % less time)
-    p.group_m = p.tiles_n <= 4 ? 1 : 8;
+    // (the four-wave tiles: groups of four rows, so that more XCDs work on the same columns at a time; 8192^3 on the
+    // metric's kind of operands 712 us against 731 with eight)
+    p.group_m = p.tiles_n <= 4 ? 1 : (IsWide<Tile>::value ? 4 : 8);
   }
   if constexpr (IsSplitK<Tile>::value) {
     // tiles are shared along K only with enough scratch memory to hold the partial tiles; without it the
@@ -201,8 +217,27 @@ hipError_t launch_kernel(const GemmParams& p_in, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// What a four-wave kernel stores with its one epilogue: plain rows of whole 8-column pieces through buffer accesses.
+template <class Tile>
+bool wide_takes(const GemmParams& p) {
+  auto dwords = [](const void* v) { return (reinterpret_cast<uintptr_t>(v) & 3) == 0; };
+  bool ok = p.perm_on == 0 && (p.N & 7) == 0 && (p.ldc & 1) == 0 && (p.sc & 1) == 0 && (p.sc_outer & 1) == 0 && dwords(p.c) &&
+      (int64_t)Tile::BM * p.ldc * 2 < 0x7fffffffll;
+  if (Epi::kNumD >= 1) ok = ok && (p.ldd & 1) == 0 && (p.sd & 1) == 0 && dwords(p.d0) && (int64_t)Tile::BM * p.ldd * 2 < 0x7fffffffll;
+  if (Epi::kNumD >= 2) ok = ok && dwords(p.d1);
+  return ok;
+}
+
 template <class Tile>
 hipError_t launch_tile(const GemmParams& p, hipStream_t stream) {
+  if constexpr (IsWide<Tile>::value) {
+    if (p.layout != 0) return hipErrorInvalidValue;
+    if (wide_takes<Tile>(p)) return launch_kernel<Tile, false>(p, stream);
+    // (other stores: the instance that takes the same operands and any output)
+    using Other = std::conditional_t<Tile::KTAIL != 0, GemmTileDma<128, 128, 64, 2, 4, 4, 1, 1, 32, 0, 2>,
+                                     GemmTilePersist<256, 256, 32, 2, 4, 4, 16, 256>>;
+    return launch_tile<Other>(p, stream);
+  } else {
   if (p.layout != 0) {
     constexpr int mask = LayoutMask<Tile>::value;
     if ((p.perm_on != 0) != kLayoutsArePermuted) return hipErrorInvalidValue;
@@ -246,6 +281,7 @@ hipError_t launch_tile(const GemmParams& p, hipStream_t stream) {
     return hipErrorInvalidValue;
   }
   return launch_kernel<Tile, false>(p, stream);
+  }
 }
 
 // Workgroups one CU can hold: limited by LDS (160 KiB) and by the register file
@@ -265,7 +301,7 @@ struct Cost {
 };
 template <class Tile, int KIND, int OCC>
 constexpr GemmAlgo entry(const char* name, Cost c) {
-  constexpr bool kByRegisters = KIND != 2 && KIND != 8;
+  constexpr bool kByRegisters = KIND != 2 && KIND != 8 && KIND != 16;
   return {name, Tile::BM, Tile::BN, Tile::BK, Tile::NT, Tile::KVEC, Tile::kLdsBytes,
           kByRegisters ? dma_wgs_per_cu(Tile::NT, OCC, Tile::kLdsBytes) : OCC, KIND, LayoutMask<Tile>::value, &launch_tile<Tile>,
           KIND == 4 ? &workspace_of<Tile> : nullptr, {c.start, c.mult, c.fetch, c.alone, c.tile}};
@@ -279,6 +315,10 @@ const GemmAlgo kAlgos[] = {
 #define AITAMD_GEMM_TILE_PERSIST(BM, BN, BK, WM, WN, NS, MT, LBM, ...)                                               \
   entry<GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM>, 2, 1>(                                                     \
       AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_persist" #NS "_m" #MT, {__VA_ARGS__}),
+#define AITAMD_GEMM_TILE_WIDE(MI, NI, BM, BN, ...)                                                                   \
+  entry<GemmTileWide<MI, NI, 0>, 16, 1>(AITAMD_NAME #BM "x" #BN "x32_w2x2_wide", {__VA_ARGS__}),
+#define AITAMD_GEMM_TILE_WIDE_K2(MI, NI, BM, BN, ...)                                                                \
+  entry<GemmTileWide<MI, NI, 1>, 16, 1>(AITAMD_NAME #BM "x" #BN "x32_w2x2_wide_k2", {__VA_ARGS__}),
 #define AITAMD_GEMM_TILE_DMA_SPLITK(BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, ...)                                      \
   entry<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 1>, 4, OCC>(                                           \
       AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_dma" #NS "_o" #OCC "_p" #PIPE "_m" #MT "_splitk", {__VA_ARGS__}),
@@ -297,6 +337,8 @@ const GemmAlgo kAlgos[] = {
 #include "gemm_tiles.inc"
 #undef AITAMD_GEMM_TILE_DMA
 #undef AITAMD_GEMM_TILE_PERSIST
+#undef AITAMD_GEMM_TILE_WIDE
+#undef AITAMD_GEMM_TILE_WIDE_K2
 #undef AITAMD_GEMM_TILE_DMA_SPLITK
 #undef AITAMD_GEMM_TILE_DMA_K2
 #undef AITAMD_GEMM_TILE_DMA_SPLITK_K2
