@@ -12,32 +12,72 @@ namespace aitamd {
 //             exponentials bound it and not the reads).
 //   kGroups:  as kRows128 in eight waves, two groups on alternate halves of larger tiles.
 //   kSmall:   two groups of two waves, 64 rows: four workgroups for every one of kGroups.
-//   kRows64:  two waves, 64 rows: sequences that leave the other half of 128 rows empty.
+//   kRows64:  two waves, 64 rows: short sequences, and those that leave the other half of 128 rows empty.
 enum Form { kRows128 = 0, kRows256 = 1, kGroups = 2, kSmall = 3, kRows64 = 4 };
 
-// The form for a problem, and whether causal query tiles go in pairs (us below: head dim 64 unless named, one
-// box, 256 CUs).
+// The form for a problem, and whether causal query tiles go in pairs.
+//
+// What decides is how the workgroups of a form fill the chip: its iterations are the time of a grid that is not full,
+// the work per CU that of a full one.  The lines lie where the forms' times cross over 780 problems (4 to 1000 sequences and
+// heads, 16 to 8192 queries, keys as many or 77, head dims 32 to 160, 380 of them causal; each form timed in turn): a
+// call takes 1.2 % more than in its best form in the geometric mean (5.6 % by the size of the grid alone, as before).
+// Figures below: us, head dim 64 unless named, 256 CUs.
 inline Form choose_form(int64_t B, int64_t M, int64_t N, int ks, int ot, bool causal, int cus, int32_t* paired) {
-  const int64_t t64 = (M + 63) / 64, t128 = (M + 127) / 128, t256 = (M + 255) / 256;
-  // Causal: a workgroup's work grows with its rows' position.  Pairs of query tiles, the last with the first and so on,
-  // are all the same length: taken by one workgroup each where they fill the chip (two four-wave workgroups per CU or
-  // one of two groups), and where there are enough tiles that an odd one in the middle is no matter.  Otherwise the
-  // longest go first.  4 x 16 x 2048^2 59 / 50 (in order of length / pairs), 2 x 8 x 4096^2 at head dim 40 63 / 43.
-  if (causal && B <= 65535 && (t128 % 2 == 0 || t128 >= 9)) {
-    const int64_t pairs = (t128 + 1) / 2 * B;
-    *paired = pairs >= 2 * cus || (t128 >= 8 && 4 * pairs >= 3 * cus && pairs <= cus);
-    if (*paired) return pairs >= 2 * cus ? kRows128 : kGroups;
+  const int64_t tiles128 = (M + 127) / 128;
+  const int64_t t64 = (M + 63) / 64 * B, t128 = tiles128 * B, t256 = (M + 255) / 256 * B;
+  // head dims up to 64: four workgroups of kRows128 on a CU, two of larger ones
+  const bool narrow = ks <= 4 && ot <= 2, mid = !narrow && ks <= 6 && ot <= 3;
+  *paired = 0;
+  // Few keys give groups nothing to share.  48 x 28 x 28 at head dim 160: 8.9 in two groups, 7.0 in one; 12 x 316 x 77
+  // at head dim 128 8.4 / 10.2.  128 rows where they leave one workgroup per CU (48 x 390 x 77 at head dim 32: 4.7, with
+  // 64 rows 5.3) and in large grids, which are wide or K and V are read the less (272 x 3954 x 77 at head dim 40 59 / 67).
+  if (M <= 64 && (N <= 32 || ks > 2 || t64 > cus)) return kRows64;  // 992 x 34^2: 6.6, 8.2 with 128 rows
+  if (M > 64 && (N <= 96 || (ot > 4 && N <= 192)))
+    return t64 <= cus || (narrow && t128 > cus && (causal || t64 <= 8 * cus)) ? kRows64 : kRows128;
+  // Grids that leave CUs idle: 64-row workgroups whose groups share the keys.  12 x 384^2 9.5 (128 rows, one group) / 8.6
+  // (128, two) / 7.1 (64, two); 8 x 2048^2 at head dim 128 41 / 38 / 33.  A little beyond, while 128 rows still fill one
+  // half of the chip: 12 x 2048^2 32.7 / 24 / 23.4; not at head dims 128 and up (60 x 275^2 11.4 / 12.4 / 19.2).
+  if (t64 <= cus || ((narrow || mid) && N >= 256 && 16 * t64 <= 25 * cus)) return kSmall;
+  if (causal) {
+    // A workgroup's work grows with its rows' position.  Pairs of query tiles, the last with the first and so on, are all
+    // the same length: best where they fill the chip in whole rounds (of one workgroup per CU with two groups, of two or
+    // four without) and where there are enough tiles that an odd one in the middle is no matter.  Otherwise the longest
+    // go first, and until the chip is full several times over the shortest chain counts: that of kSmall.
+    // In order of length / pairs: 64 x 2048^2 59 / 50, 16 x 4096^2 at head dim 40 63 / 43, 36 x 3341^2 at 80 124 / 92;
+    // 32 x 2237^2 45 / 53, and 39 with kSmall; 16 x 2346^2 at head dim 40 35 and 23; 24 x 1741^2 at 80 40 and 29.
+    const bool pairable = B <= 65535 && (tiles128 % 2 == 0 || tiles128 >= 9);
+    const int64_t pairs = (tiles128 + 1) / 2 * B;
+    if (pairable && tiles128 >= 8 && 8 * pairs >= 7 * cus && pairs <= cus) {
+      *paired = 1;
+      return kGroups;
+    }
+    if (narrow) {
+      const bool full = pairs >= 2 * cus;
+      if (t64 <= 2 * cus || (!full && ((2 * t64 <= 9 * cus && M > 448) || M >= 1024))) return kSmall;
+      // 64 rows while a pair of 128 would be a large part of the sequence: 276 x 508^2 31 / 27, 248 x 1781^2 144 / 160
+      *paired = full && B <= 65535 && M >= 512;
+      return M < 1536 ? kRows64 : kRows128;
+    }
+    if (mid ? t64 <= 2 * cus || (t64 <= 3 * cus && M >= 1024) : 4 * t64 <= 5 * cus && N >= 512) return kSmall;
+    const int64_t rounds = (pairs + 2 * cus - 1) / (2 * cus);
+    if (pairable && pairs >= cus && 10 * pairs >= 16 * cus * rounds) {  // (a last round four fifths full at least)
+      *paired = 1;
+      return kRows128;
+    }
+    if (t128 <= cus && N >= 512) return kGroups;
+    return mid && M <= 512 ? kRows64 : kRows128;
   }
-  // Grids that leave CUs idle: 64-row workgroups whose groups share the keys; 128 rows while those do fill the chip.
-  // 1 x 12 x 384^2 8.9 (128 rows, one group) / 8.5 (128, two) / 7.1 (64, two); 1 x 12 x 2048^2 31 / 24 / 24;
-  // 1 x 8 x 2048^2 at head dim 128 41 / 38 / 33, at 512 workgroups of 64 rows (1 x 16 x 2000^2) 46 / 43 / 64.  Few
-  // keys give the groups nothing to share: 6 x 12 x 316 x 77 at head dim 128 8.4 / 10.2 / 15.6.
-  if (t64 * B <= cus || (16 * t64 * B <= 25 * cus && N >= 256)) return kSmall;
-  if (M <= 64) return kRows64;  // 62 x 16 x 34^2: 6.6, 8.2 with 128 rows
-  if (t128 * B <= cus && N >= 512) return kGroups;
-  // 64 rows per wave where K and V are read often enough to be the bound: 1 x 16 x 8192^2 288, 312 with 32 rows; even
-  // at 62 x 4 x 1472^2 and at head dim 40
-  if (!causal && ks == 4 && ot == 2 && M >= 2048 && t256 * B >= 2 * cus) return kRows256;
+  if (t128 <= cus) return N >= 512 ? kGroups : kRows128;
+  // Short sequences: smaller workgroups start and end more evenly.  816 x 135^2 20.5 (128 rows) / 17.8, 136 x 394^2 at
+  // head dim 32 13.2 / 11.1, 768 x 384^2 of mixed lengths 42.0 / 41.0; 352 x 492^2 at head dim 40 33.0 / 35.2
+  if (narrow && N <= (ks == 3 ? 256 : 512)) return kRows64;
+  // (head dim 32, where two groups' state is small: 64 x 1268^2 32.3 / 27.9)
+  if (ks <= 2 && ot == 1 && N <= 4096 && t64 <= 8 * cus) return kSmall;
+  // 64 rows per wave where K and V are read often enough to be the bound and the last round of the workgroups, two per
+  // CU, is four fifths full: 16 x 8192^2 288, 312 with 32 rows; 64 x 2209^2 (1.1 rounds) 126 / 110; even at 62 x 4 x 1472^2
+  // and at head dim 40
+  const int64_t rounds = (t256 + 2 * cus - 1) / (2 * cus);
+  if (ks == 4 && ot == 2 && M >= 2048 && 10 * t256 >= 16 * cus * rounds) return kRows256;
   return kRows128;
 }
 

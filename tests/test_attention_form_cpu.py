@@ -45,3 +45,27 @@ def test_lines_move_with_the_number_of_cus(choose):
     for _ in range(3000):
         B, M, N, d, causal = rng.randint(1, 200), rng.randint(1, 5000), rng.randint(1, 5000), rng.choice([40, 64, 128]), rng.randint(0, 1)
         assert choose(B, M, N, d, causal, 32) == choose(8 * B, M, N, d, causal, 256), (B, M, N, d, causal)
+
+
+@pytest.mark.parametrize("case,form,paired", [
+    ((48, 28, 28, 160, 0), ROWS64, 0), ((48, 28, 28, 32, 0), ROWS64, 0), ((48, 40, 40, 32, 0), SMALL, 0),     # one tile of queries
+    ((16, 285, 77, 160, 0), ROWS64, 0), ((48, 390, 77, 32, 0), ROWS128, 0), ((99, 400, 77, 64, 0), ROWS64, 0),  # few keys
+    ((64, 219, 219, 160, 0), SMALL, 0), ((64, 219, 190, 160, 0), ROWS64, 0),
+    ((60, 275, 275, 128, 0), ROWS128, 0), ((60, 275, 275, 80, 0), SMALL, 0),                                    # idle CUs
+    ((32, 2237, 2237, 64, 1), SMALL, 0), ((276, 508, 508, 64, 1), ROWS64, 0), ((276, 520, 520, 64, 1), ROWS64, 1),
+    ((248, 1781, 1781, 64, 1), ROWS128, 1), ((224, 400, 400, 40, 1), ROWS64, 0),                                # causal, narrow
+    ((24, 1741, 1741, 80, 1), SMALL, 0), ((36, 3341, 3341, 80, 1), ROWS128, 1), ((96, 639, 639, 128, 1), ROWS128, 0),
+    ((208, 397, 397, 80, 1), ROWS128, 1), ((164, 268, 268, 80, 1), ROWS64, 0), ((70000, 600, 600, 64, 1), ROWS64, 0),
+    ((768, 384, 384, 64, 0), ROWS64, 0), ((352, 492, 492, 40, 0), ROWS128, 0), ((64, 1268, 1268, 32, 0), SMALL, 0),
+    ((64, 2209, 2209, 64, 0), ROWS128, 0), ((64, 2048, 2048, 64, 0), ROWS256, 0)])                              # full grids
+def test_lines_within_a_grid_size(choose, case, form, paired):
+    assert choose(*case, 256) == (form, paired)
+
+
+def test_pairs_are_of_causal_tiles_that_the_grid_can_hold(choose):
+    rng = random.Random(1)
+    for _ in range(20000):
+        B, M, N = (int(2 ** rng.uniform(0, e)) for e in (17, 14, 14))
+        d, causal = rng.choice([8, 32, 40, 64, 80, 96, 128, 160]), rng.randint(0, 1)
+        form, paired = choose(B, M, N, d, causal, 256)
+        assert form in range(5) and (not paired or (causal and B <= 65535 and form != ROWS256 and M > 128)), (B, M, N, d, causal)

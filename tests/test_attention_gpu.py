@@ -72,6 +72,17 @@ def test_every_variant_of_the_small_head_dims(attn_variant, mode, B, M, N, K, O,
     _check(B, M, N, K, O, G, causal=causal, scale=scale, seed=mode + N)
 
 
+@pytest.mark.parametrize("B,M,N,d,causal", [
+    (48, 31, 32, 64, False), (16, 65, 77, 160, False), (16, 285, 192, 160, True),  # few keys: 64 rows
+    (72, 65, 96, 40, True), (70, 1030, 77, 64, True),
+    (260, 520, 520, 32, True),   # pairs of 64-row tiles, nine of them: the middle one by itself, the last of eight rows
+    (132, 961, 961, 64, True),   # sixteen of them, the last of one row
+    (36, 641, 641, 64, True),    # two groups of 64 rows, causal, beyond the CUs: the longest first
+    (60, 257, 300, 128, False), (136, 129, 394, 32, False), (24, 1025, 1025, 80, True)])
+def test_forms_chosen_within_a_grid_size(B, M, N, d, causal):
+    _check(B, M, N, d, d, 4 if B % 4 == 0 else 2, causal, seed=M + d)
+
+
 @pytest.mark.parametrize("B,M,N,K,O,G,causal", [
     (16, 256, 256, 160, 160, 8, False),     # the deepest attention of Stable Diffusion v1: 1280 channels, 8 heads
     (8, 100, 77, 160, 160, 8, False),       # its cross-attention over 77 text tokens
