@@ -68,7 +68,7 @@ int ptr_align(const void* p) {
 int split_factor(const GemmAlgo& a, int64_t batch, int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t tiles = ((M + a.bm - 1) / a.bm) * ((N + a.bn - 1) / a.bn) * (batch > 0 ? batch : 1);
   const int64_t k_tiles = ((a.kvec == 8 ? K : (K & ~7)) + a.bk - 1) / a.bk;
-  return split_k_rule(tiles, k_tiles, cus);
+  return split_k_rule(tiles, k_tiles, a.bk, (int64_t)a.bm * a.bn, cus);
 }
 
 // The instance with the smallest estimate of run time, from the measured figures that gemm_tiles.inc gives for each.
@@ -95,13 +95,12 @@ int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64
     double cost = a.cost.start;
     if (a.direct_lds == 4) {
       // split-K: usable with scratch memory, and worth a table entry of its own only where it does split (it is
-      // the plain instance otherwise).  Every workgroup multiplies K / s; the exchange of partial tiles through
-      // memory is three trips to it (store, count, load) and s partial tiles to add.
+      // the plain instance otherwise).  Every workgroup multiplies K / s.
       const int s_k = split_factor(a, batch, M, N, K, kNumCu);
       if (!has_workspace || s_k <= 1 || layout != 0) continue;
       slabs = (slabs + s_k - 1) / s_k;
+      cost += split_k_exchange_us(tiles, s_k, (int64_t)a.bm * a.bn);
       tiles *= s_k;
-      cost += 1.5 + (a.bm * a.bn >= 128 * 128 ? 0.65 : 0.33) * s_k;
     }
     const int per_cu = a.wgs_per_cu > 0 ? a.wgs_per_cu : 1;
     const int64_t slots = (int64_t)kNumCu * per_cu;

@@ -35,16 +35,33 @@ struct GemmAlgoTable {
   int count;
 };
 
-// Workgroups per tile of a split-K launch (the launcher and the instance choice share the rule): as many as bring
-// the grid up to about one workgroup per CU, each with at least two K-slabs, at most 16; 1 (no splitting, nothing
-// written to the scratch memory) for grids that fill the device anyway.  Measured against two and four workgroups
-// per CU and against longer minimum shares (256x1024x1024, 512x768x3072, 1x6912x8314, 64x256x8192): never slower.
-inline int split_k_rule(int64_t tiles, int64_t k_tiles, int cus) {
+// What a split-K launch pays for sharing its tiles between s workgroups each, in us: three trips to memory (store, count,
+// load), s workgroups that count and load, and the partial tiles' bytes.  Fitted, as are the slab times below,
+// on 558 problems (M 21 to 1024, N 256 to 3072, K 512 to 8192) with every number of splits.
+inline double split_k_exchange_us(int64_t tiles, int64_t s, int64_t tile_elems) {
+  const double megabytes = (double)(tiles * s * tile_elems) * 4e-6;
+  return tile_elems >= 128 * 128 ? 2.04 + 0.64 * (double)s + 0.34 * megabytes : 0.95 + 0.23 * (double)s + 0.48 * megabytes;
+}
+
+// Workgroups per tile of a split-K launch (the launcher and the instance choice share the rule): of the numbers from two
+// up to about one workgroup per CU, with at least two K-slabs each, at most 16, the one that gives the least time for a
+// workgroup's slabs and the exchange; 1 (no splitting, nothing written to the scratch memory) for grids that fill half
+// the device anyway.  Whether to split at all is the choice of the instance.  1.5 % (64 x 64 tiles) and 2.0 %
+// (128 x 128) above the best number in the geometric mean; as many as fill the CUs, the rule before, 8 % and 21 %:
+// 21 x 512 x 2048 11.5 us with 16, 7.1 with 4; 200 x 2304 x 768 in 128 x 128 tiles 17.4 with 6, 13.1 with 2.
+inline int split_k_rule(int64_t tiles, int64_t k_tiles, int bk, int64_t tile_elems, int cus) {
   if (tiles <= 0) return 1;
-  int64_t s = cus / tiles;
-  if (s > k_tiles / 2) s = k_tiles / 2;
-  if (s > 16) s = 16;
-  return (int)(s < 1 ? 1 : s);
+  const double slab_us = (tile_elems >= 128 * 128 ? 0.395 : 0.226) * bk / 64;
+  int best = 1;
+  double best_us = 0;
+  for (int64_t s = 2; s <= 16 && s * tiles <= cus && 2 * s <= k_tiles; ++s) {
+    const double us = slab_us * (double)((k_tiles + s - 1) / s) + split_k_exchange_us(tiles, s, tile_elems);
+    if (best == 1 || us < best_us) {
+      best = (int)s;
+      best_us = us;
+    }
+  }
+  return best;
 }
 
 // Defined once per (epilogue, dtype) translation unit; nullptr table when that

@@ -121,14 +121,12 @@ struct IsWide<GemmTileWide<MI, NI, KTAIL>> {
   static constexpr bool value = true;
 };
 
-// Workgroups per tile of a split-K launch: as many as bring the grid up to about one workgroup per CU, each with
-// at least two K-slabs, at most 16; 1 (no splitting, nothing written to the scratch memory) for grids that fill
-// the device anyway.
+// Workgroups per tile of a split-K launch (split_k_rule)
 template <class Tile>
 int split_k_factor(const GemmParams& p, int cus) {
   const int64_t tiles = (int64_t)((p.M + Tile::BM - 1) / Tile::BM) * ((p.N + Tile::BN - 1) / Tile::BN) * p.batch;
   const int64_t k_tiles = ((Tile::KVEC == 8 ? p.K : (p.K & ~7)) + Tile::BK - 1) / Tile::BK;
-  return split_k_rule(tiles, k_tiles, cus);
+  return split_k_rule(tiles, k_tiles, Tile::BK, (int64_t)Tile::BM * Tile::BN, cus);
 }
 template <class Tile>
 int64_t workspace_of(const GemmParams& p) {
