@@ -105,13 +105,16 @@ def _filter(instance_name, func_attrs, ab_alignment) -> bool:
 
 def _select_algo(func_attrs, exec_key) -> str:
     operands = _operands(func_attrs["op"])
-    if operands == 0:
-        return common.gemm_select_algo(func_attrs, exec_key)
     lib = _kernels.load()
     dtype = common.DTYPE_ID[func_attrs["inputs"][0]._attrs["dtype"]]
     epi = _kernels.PERMUTE_OPS[func_attrs["op"]][0]
     m, n, k = gemm_inverse_key_func(exec_key)[-3:]
-    algo = lib.aitamd_gemm_heuristic_algo_layout(epi, dtype, operands, 1, m, n, k, k, n, 16)
+    if operands == 0:
+        # (4: rcr operands, permuted store)
+        align = next(a for a in (16, 8, 4, 2) if k * 2 % a == 0)
+        algo = lib.aitamd_gemm_heuristic_algo_layout(epi, dtype, 4, 1, m, n, k, k, k, align)
+    else:
+        algo = lib.aitamd_gemm_heuristic_algo_layout(epi, dtype, operands, 1, m, n, k, k, n, 16)
     all_names = _kernels.gemm_algo_names(epi, dtype)
     if algo >= 0 and all_names[algo] in func_attrs["op_instance"]:
         return all_names[algo]

@@ -50,9 +50,7 @@ bool algo_supported(const GemmAlgo& a, int64_t M, int64_t N, int64_t K, int64_t 
   if ((b_t ? K * ldb : (int64_t)(a.direct_lds == 16 ? 256 : a.bn) * ldb) * 2 >= 0x7fffffffll) return false;
   if (M > 0x7fffffffll || K > 0x3fffffffll) return false;
   // the persistent kernels write a tile when its last K-slab has been multiplied: they need one
-  if (a.direct_lds == 2 && K < 1) return false;
-  // the four-wave kernels are built of three slab pairs at least, and store whole 16-byte pieces
-  if (a.direct_lds == 16 && ((kv == 8 ? K : (K & ~7ll)) <= 128 || N % 8 != 0)) return false;
+  if ((a.direct_lds == 2 || (a.direct_lds == 16 && kv == 8)) && K < 1) return false;
   return true;
 }
 
@@ -79,7 +77,7 @@ int split_factor(const GemmAlgo& a, int64_t batch, int64_t M, int64_t N, int64_t
 // (odd K) to 4.5 % (batched products with both operands transposed) slower than the best instance on average; the
 // differences between runs of a launch of a few us are a good part of that.
 int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
-              int align_bytes, int layout = 0, bool has_workspace = false) {
+              int align_bytes, int layout = 0, bool has_workspace = false, bool plain_store = true) {
   int best = -1;
   double best_cost = 0;
   const int kNumCu = current_device_cus();  // what the launcher sizes grids and split factors with
@@ -90,6 +88,7 @@ int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64
     if (!algo_supported(a, M, N, K, lda, ldb, align_bytes, layout)) continue;
     // (the dword-aligned twins of the direct-to-LDS tiles are for what the 16-byte ones cannot take)
     if (a.kvec == 2 && (a.direct_lds & 21) != 0 && align_bytes >= 16 && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0) continue;
+    if (a.direct_lds == 16 && !(plain_store && N % 8 == 0 && four_waves_multiply(a.kvec, K))) continue;
     int64_t slabs = ((a.kvec == 2 && a.direct_lds != 8 ? K & ~7ll : K) + a.bk - 1) / a.bk;
     int64_t tiles = ((M + a.bm - 1) / a.bm) * ((N + a.bn - 1) / a.bn) * batches;
     double cost = a.cost.start;
@@ -133,27 +132,27 @@ int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64
 struct HeuristicKey {
   const GemmAlgo* table;
   int64_t batch, M, N, K, lda, ldb;
-  int32_t align_bytes, layout, has_workspace, cus;
+  int32_t align_bytes, layout, has_workspace, plain_store, cus;
   bool operator==(const HeuristicKey& o) const {
     return table == o.table && batch == o.batch && M == o.M && N == o.N && K == o.K && lda == o.lda && ldb == o.ldb &&
-        align_bytes == o.align_bytes && layout == o.layout && has_workspace == o.has_workspace && cus == o.cus;
+        align_bytes == o.align_bytes && layout == o.layout && has_workspace == o.has_workspace && plain_store == o.plain_store && cus == o.cus;
   }
 };
 int remembered_heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t lda,
-                         int64_t ldb, int align_bytes, int layout, bool has_workspace) {
+                         int64_t ldb, int align_bytes, int layout, bool has_workspace, bool plain_store) {
   constexpr int kEntries = 256;
   struct Entry {
     HeuristicKey key{};
     int algo = -1;
   };
   static thread_local Entry entries[kEntries];
-  const HeuristicKey key{t.algos, batch, M, N, K, lda, ldb, align_bytes, layout, has_workspace ? 1 : 0, current_device_cus()};
+  const HeuristicKey key{t.algos, batch, M, N, K, lda, ldb, align_bytes, layout, has_workspace ? 1 : 0, plain_store ? 1 : 0, current_device_cus()};
   uint64_t h = reinterpret_cast<uint64_t>(t.algos);
-  for (int64_t v : {batch, M, N, K, lda, ldb, (int64_t)(align_bytes * 8 + layout * 2 + key.has_workspace)})
+  for (int64_t v : {batch, M, N, K, lda, ldb, (int64_t)(align_bytes * 16 + layout * 4 + key.has_workspace * 2 + key.plain_store)})
     h = (h ^ (uint64_t)v) * 0x9e3779b97f4a7c15ull;
   Entry& e = entries[h >> 56];
   if (!(e.key == key)) {
-    e.algo = heuristic(t, batch, M, N, K, lda, ldb, align_bytes, layout, has_workspace);
+    e.algo = heuristic(t, batch, M, N, K, lda, ldb, align_bytes, layout, has_workspace, plain_store);
     e.key = key;
   }
   return e.algo;
@@ -181,10 +180,11 @@ int run_gemm(int epilogue, int dtype, int algo, const GemmParams& p, hipStream_t
     if (a2 < align) align = a2;
   }
   if (algo < 0) {
-    algo = remembered_heuristic(t, p.batch, p.M, p.N, p.K, p.lda, p.ldb, align, p.layout, p.ws != nullptr && p.perm_on == 0);
+    const bool plain = four_waves_store(p);
+    algo = remembered_heuristic(t, p.batch, p.M, p.N, p.K, p.lda, p.ldb, align, p.layout, p.ws != nullptr && p.perm_on == 0, plain);
     // (the heuristic prices split-K with the split it would get; a buffer too small for that falls back)
     if (algo >= 0 && t.algos[algo].workspace_bytes && t.algos[algo].workspace_bytes(p) > p.ws_bytes)
-      algo = remembered_heuristic(t, p.batch, p.M, p.N, p.K, p.lda, p.ldb, align, p.layout, false);
+      algo = remembered_heuristic(t, p.batch, p.M, p.N, p.K, p.lda, p.ldb, align, p.layout, false, plain);
     if (algo < 0) return fail("aitamd_gemm: no instance supports M=%d N=%d K=%d", p.M, p.N, p.K);
   }
   if (algo >= t.count) return fail("aitamd_gemm: algo %d out of range (have %d)", algo, t.count);
@@ -244,7 +244,8 @@ int aitamd_gemm_heuristic_algo_layout(int epilogue, int dtype, int layout, int64
                                       int64_t K, int64_t lda, int64_t ldb, int align_bytes) {
   const GemmAlgoTable t = gemm_table(epilogue, dtype);
   if (t.count == 0) return -1;
-  return heuristic(t, batch, M, N, K, lda, ldb, align_bytes, layout);
+  constexpr int kPermuted = 4;  // rcr operands, an output stored permuted
+  return heuristic(t, batch, M, N, K, lda, ldb, align_bytes, layout == kPermuted ? 0 : layout, false, layout != kPermuted);
 }
 
 int aitamd_gemm_heuristic_algo(int epilogue, int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t lda,

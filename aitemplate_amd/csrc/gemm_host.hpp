@@ -35,6 +35,17 @@ struct GemmAlgoTable {
   int count;
 };
 
+// What the four-wave kernels store with their one epilogue: plain rows of whole 8-column pieces through buffer accesses.
+inline bool four_waves_store(const GemmParams& p) {
+  auto dwords = [](const void* v) { return (reinterpret_cast<uintptr_t>(v) & 3) == 0; };
+  bool ok = p.perm_on == 0 && p.layout == 0 && (p.N & 7) == 0 && (p.ldc & 1) == 0 && (p.sc & 1) == 0 && (p.sc_outer & 1) == 0 &&
+      dwords(p.c) && 256 * p.ldc * 2 < 0x7fffffffll;
+  if (p.d0 != nullptr) ok = ok && (p.ldd & 1) == 0 && (p.sd & 1) == 0 && dwords(p.d0) && dwords(p.d1) && 256 * p.ldd * 2 < 0x7fffffffll;
+  return ok;
+}
+// ... and multiply: K of three slab pairs at least
+inline bool four_waves_multiply(int kvec, int64_t K) { return (kvec == 8 ? K : (K & ~7ll)) > 128; }
+
 // What a split-K launch pays for sharing its tiles between s workgroups each, in us: three trips to memory (store, count,
 // load), s workgroups that count and load, and the partial tiles' bytes.  Fitted, as are the slab times below,
 // on 558 problems (M 21 to 1024, N 256 to 3072, K 512 to 8192) with every number of splits.

@@ -215,23 +215,15 @@ hipError_t launch_kernel(const GemmParams& p_in, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// What a four-wave kernel stores with its one epilogue: plain rows of whole 8-column pieces through buffer accesses.
-template <class Tile>
-bool wide_takes(const GemmParams& p) {
-  auto dwords = [](const void* v) { return (reinterpret_cast<uintptr_t>(v) & 3) == 0; };
-  bool ok = p.perm_on == 0 && (p.N & 7) == 0 && (p.ldc & 1) == 0 && (p.sc & 1) == 0 && (p.sc_outer & 1) == 0 && dwords(p.c) &&
-      (int64_t)Tile::BM * p.ldc * 2 < 0x7fffffffll;
-  if (Epi::kNumD >= 1) ok = ok && (p.ldd & 1) == 0 && (p.sd & 1) == 0 && dwords(p.d0) && (int64_t)Tile::BM * p.ldd * 2 < 0x7fffffffll;
-  if (Epi::kNumD >= 2) ok = ok && dwords(p.d1);
-  return ok;
-}
-
 template <class Tile>
 hipError_t launch_tile(const GemmParams& p, hipStream_t stream) {
   if constexpr (IsWide<Tile>::value) {
     if (p.layout != 0) return hipErrorInvalidValue;
-    if (wide_takes<Tile>(p)) return launch_kernel<Tile, false>(p, stream);
-    // (other stores: the instance that takes the same operands and any output)
+    const bool multiplies = four_waves_multiply(Tile::KVEC, p.K) && (p.N & 7) == 0;
+    if (multiplies && four_waves_store(p)) return launch_kernel<Tile, false>(p, stream);
+    // Asked for by name with others: an instance that takes the same operands, any K and any output.  For a permuted store
+    // the one of the same matrix instructions, whose results are those of the plain store.
+    if (multiplies && p.perm_on) return launch_tile<GemmTileDma<32, 32, 128, 2, 2, 4, 2, 0, 16, 0, Tile::KTAIL != 0 ? 2 : 0>>(p, stream);
     using Other = std::conditional_t<Tile::KTAIL != 0, GemmTileDma<128, 128, 64, 2, 4, 4, 1, 1, 32, 0, 2>,
                                      GemmTilePersist<256, 256, 32, 2, 4, 4, 16, 256>>;
     return launch_tile<Other>(p, stream);
@@ -313,10 +305,17 @@ const GemmAlgo kAlgos[] = {
 #define AITAMD_GEMM_TILE_PERSIST(BM, BN, BK, WM, WN, NS, MT, LBM, ...)                                               \
   entry<GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM>, 2, 1>(                                                     \
       AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_persist" #NS "_m" #MT, {__VA_ARGS__}),
+// (not for the bias of halves, whose sum and conversion the compiler may or may not take in one instruction: a permuted store
+// of an instance has to give the bits of its plain one, and these have none of their own)
+#if AITAMD_EPI == 1 && AITAMD_DT == 0
+#define AITAMD_GEMM_TILE_WIDE(...)
+#define AITAMD_GEMM_TILE_WIDE_K2(...)
+#else
 #define AITAMD_GEMM_TILE_WIDE(MI, NI, BM, BN, ...)                                                                   \
   entry<GemmTileWide<MI, NI, 0>, 16, 1>(AITAMD_NAME #BM "x" #BN "x32_w2x2_wide", {__VA_ARGS__}),
 #define AITAMD_GEMM_TILE_WIDE_K2(MI, NI, BM, BN, ...)                                                                \
   entry<GemmTileWide<MI, NI, 1>, 16, 1>(AITAMD_NAME #BM "x" #BN "x32_w2x2_wide_k2", {__VA_ARGS__}),
+#endif
 #define AITAMD_GEMM_TILE_DMA_SPLITK(BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, ...)                                      \
   entry<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 1>, 4, OCC>(                                           \
       AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_dma" #NS "_o" #OCC "_p" #PIPE "_m" #MT "_splitk", {__VA_ARGS__}),

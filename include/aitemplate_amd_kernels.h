@@ -209,7 +209,8 @@ AITAMD_API int aitamd_gemm_permute(int operands, int epilogue, int dtype, int al
                                    const void* a, const void* b, const void* bias, void* c,
                                    int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                    int layout, int64_t g1, int64_t g2, int64_t g3, void* stream);
-/* aitamd_gemm_algo_supported / aitamd_gemm_heuristic_algo for a given operand layout (same arguments otherwise) */
+/* aitamd_gemm_algo_supported / aitamd_gemm_heuristic_algo for a given operand layout (same arguments otherwise); layout 4
+ * of the latter: rcr operands and a permuted store */
 AITAMD_API int aitamd_gemm_algo_supported_layout(int epilogue, int dtype, int layout, int algo,
                                                  int64_t M, int64_t N, int64_t K,
                                                  int64_t lda, int64_t ldb, int align_bytes);

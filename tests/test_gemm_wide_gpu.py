@@ -9,8 +9,8 @@ from oracle import oracle
 
 pytestmark = pytest.mark.gpu
 
-ALIGNED = [n for n in _kernels.gemm_algo_names(1, 0) if n.endswith("_wide")]
-DWORDS = [n for n in _kernels.gemm_algo_names(1, 0) if n.endswith("_wide_k2")]
+ALIGNED = [n for n in _kernels.gemm_algo_names(2, 0) if n.endswith("_wide")]
+DWORDS = [n for n in _kernels.gemm_algo_names(2, 0) if n.endswith("_wide_k2")]
 
 
 def _rand(shape, seed, dtype, scale=1.0):
@@ -51,7 +51,7 @@ def _check(op, name, M, N, K, dtype=torch.float16, pitch=0, seed=0):
 ])
 def test_wide_shapes(name, M, N, K):
     seed = M + N + K
-    _check("gemm_rcr_bias", name, M, N, K, seed=seed)
+    _check("gemm_rcr_bias_relu", name, M, N, K, seed=seed)
     _check("gemm_rcr_bias_add_add", name, M, N, K, torch.bfloat16, pitch=8, seed=seed)
     _check("gemm_rcr_bias_add", name, M, N, K, pitch=24, seed=seed)
 
@@ -60,7 +60,7 @@ def test_wide_shapes(name, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(1, 8, 138), (256, 256, 196), (255, 248, 206), (257, 264, 254), (130, 216, 1030),
                                    (4100, 4200, 142), (300, 440, 8314)])
 def test_wide_dword_rows(name, M, N, K):
-    _check("gemm_rcr_bias", name, M, N, K, seed=K)
+    _check("gemm_rcr_bias_gelu", name, M, N, K, seed=K)
     _check("gemm_rcr_bias_relu", name, M, N, K, torch.bfloat16, pitch=4, seed=K)
     _check("gemm_rcr_bias_mul_add", name, M, N, K, pitch=2, seed=K)
 
@@ -68,15 +68,20 @@ def test_wide_dword_rows(name, M, N, K):
 @pytest.mark.parametrize("name", ALIGNED + DWORDS)
 @pytest.mark.parametrize("op", sorted(set(_kernels.EPILOGUE_OF_OP) - {"bmm_rcr"}))
 def test_wide_every_epilogue(name, op):
-    _check(op, name, 500, 472, 322 if name in DWORDS else 320, seed=7)
+    # (the bias of halves alone has no such instances: see the table)
+    dtype = torch.bfloat16 if _kernels.EPILOGUE_OF_OP[op] == 1 else torch.float16
+    _check(op, name, 500, 472, 322 if name in DWORDS else 320, dtype, seed=7)
 
 
 @pytest.mark.parametrize("name", ALIGNED + DWORDS)
 def test_wide_supported_problems(name):
     lib, k = _kernels.load(), 2 if name in DWORDS else 8
-    ok = lambda N, K, align: lib.aitamd_gemm_algo_supported(1, 0, _algo("gemm_rcr_bias", name, torch.float16), 64, N, K, K, K, align)
-    assert ok(64, 136, 2 * k) and not ok(64, 128, 2 * k) and not ok(60, 136, 2 * k) and not ok(64, 136 + k // 2, 2 * k)
-    assert not ok(64, 136, k)
+    ok = lambda N, K, align: lib.aitamd_gemm_algo_supported(2, 0, _algo("gemm_rcr_bias_relu", name, torch.float16), 64, N, K, K, K, align)
+    assert ok(64, 136, 2 * k) and not ok(64, 136 + k // 2, 2 * k) and not ok(64, 136, k)
+    # short K and columns that are no whole pieces: handed on to an instance that takes them
+    for M, N, K in ((64, 64, 128), (300, 60, 136), (70, 59, 48)):
+        assert ok(N, K, 2 * k)
+        _check("gemm_rcr_bias_relu", name, M, N, K, seed=8)
 
 
 @pytest.mark.parametrize("name", ALIGNED)
