@@ -59,9 +59,9 @@ struct KernelOf<GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM, PAIR>, PERM, LA
   static constexpr auto value =
       gemm_rcr_persist_kernel<Elem, GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM, PAIR>, Epi, PERM, LAYOUT == kShortK>;
 };
-template <int MT, int NW, int U, int ELEM, bool PERM, int LAYOUT>
-struct KernelOf<GemmTileRows<MT, NW, U, ELEM>, PERM, LAYOUT> {
-  static constexpr auto value = gemm_rcr_rows_kernel<Elem, GemmTileRows<MT, NW, U, ELEM>, Epi, PERM>;
+template <int NW, int NS, int ELEM, bool PERM, int LAYOUT>
+struct KernelOf<GemmTileRows<NW, NS, ELEM>, PERM, LAYOUT> {
+  static constexpr auto value = gemm_rcr_rows_kernel<Elem, GemmTileRows<NW, NS, ELEM>, Epi, PERM>;
 };
 template <int MI, int NI, int KTAIL, bool PERM, int LAYOUT>
 struct KernelOf<GemmTileWide<MI, NI, KTAIL>, PERM, LAYOUT> {
@@ -328,9 +328,10 @@ const GemmAlgo kAlgos[] = {
 #define AITAMD_GEMM_TILE_STAGED(BM, BN, BK, WM, WN, NS, OCC, MT, ...)                                                \
   entry<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, 0, MT, 0, 4>, 0, OCC>(                                              \
       AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_reg" #NS "_o" #OCC "_v1", {__VA_ARGS__}),
-#define AITAMD_GEMM_ROWS(MT, NW, U, ...)                                                                             \
-  entry<GemmTileRows<MT, NW, U, 0>, 8, 4>(AITAMD_NAME "rows" #MT "_n" #NW "_u" #U "_k2", {__VA_ARGS__}),             \
-  entry<GemmTileRows<MT, NW, U, 1>, 8, 4>(AITAMD_NAME "rows" #MT "_n" #NW "_u" #U "_v1", {__VA_ARGS__}),
+#define AITAMD_GEMM_ROWS(NW, NS, ...)                                                                                \
+  entry<GemmTileRows<NW, NS, 0>, 8, 2>(AITAMD_NAME "rows16x16_n" #NW "_s" #NS "_k2", {__VA_ARGS__}),
+#define AITAMD_GEMM_ROWS_ELEM(NW, NS, ...)                                                                           \
+  entry<GemmTileRows<NW, NS, 1>, 8, 2>(AITAMD_NAME "rows16x16_n" #NW "_s" #NS "_v1", {__VA_ARGS__}),
 #include "gemm_tiles.inc"
 #undef AITAMD_GEMM_TILE_DMA
 #undef AITAMD_GEMM_TILE_PERSIST
@@ -341,6 +342,7 @@ const GemmAlgo kAlgos[] = {
 #undef AITAMD_GEMM_TILE_DMA_SPLITK_K2
 #undef AITAMD_GEMM_TILE_STAGED
 #undef AITAMD_GEMM_ROWS
+#undef AITAMD_GEMM_ROWS_ELEM
 #undef AITAMD_NAME
 };
 
