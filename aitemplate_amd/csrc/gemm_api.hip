@@ -98,7 +98,7 @@ int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64
       const int s_k = split_factor(a, batch, M, N, K, kNumCu);
       if (!has_workspace || s_k <= 1 || layout != 0) continue;
       slabs = (slabs + s_k - 1) / s_k;
-      cost += split_k_exchange_us(tiles, s_k, (int64_t)a.bm * a.bn);
+      cost += a.bk < 64 ? 1.5 + 0.65 * s_k : split_k_exchange_us(tiles, s_k, (int64_t)a.bm * a.bn);
       tiles *= s_k;
     }
     const int per_cu = a.wgs_per_cu > 0 ? a.wgs_per_cu : 1;
