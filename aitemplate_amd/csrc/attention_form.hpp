@@ -69,8 +69,8 @@ inline Form choose_form(int64_t B, int64_t M, int64_t N, int ks, int ot, bool ca
   }
   if (t128 <= cus) return N >= 512 ? kGroups : kRows128;
   // Short sequences: smaller workgroups start and end more evenly.  816 x 135^2 20.5 (128 rows) / 17.8, 136 x 394^2 at
-  // head dim 32 13.2 / 11.1, 768 x 384^2 of mixed lengths 42.0 / 41.0; 352 x 492^2 at head dim 40 33.0 / 35.2
-  if (narrow && N <= (ks == 3 ? 256 : 512)) return kRows64;
+  // head dim 32 13.2 / 11.1; beyond, 768 x 384^2 of mixed lengths 41.2 / 41.6, 352 x 492^2 at head dim 40 33.0 / 35.2
+  if (narrow && N <= (ks <= 2 ? 512 : 256)) return kRows64;
   // (head dim 32, where two groups' state is small: 64 x 1268^2 32.3 / 27.9)
   if (ks <= 2 && ot == 1 && N <= 4096 && t64 <= 8 * cus) return kSmall;
   // 64 rows per wave where K and V are read often enough to be the bound and the last round of the workgroups, two per

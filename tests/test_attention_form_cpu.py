@@ -56,7 +56,7 @@ def test_lines_move_with_the_number_of_cus(choose):
     ((248, 1781, 1781, 64, 1), ROWS128, 1), ((224, 400, 400, 40, 1), ROWS64, 0),                                # causal, narrow
     ((24, 1741, 1741, 80, 1), SMALL, 0), ((36, 3341, 3341, 80, 1), ROWS128, 1), ((96, 639, 639, 128, 1), ROWS128, 0),
     ((208, 397, 397, 80, 1), ROWS128, 1), ((164, 268, 268, 80, 1), ROWS64, 0), ((70000, 600, 600, 64, 1), ROWS64, 0),
-    ((768, 384, 384, 64, 0), ROWS64, 0), ((352, 492, 492, 40, 0), ROWS128, 0), ((64, 1268, 1268, 32, 0), SMALL, 0),
+    ((768, 256, 256, 64, 0), ROWS64, 0), ((768, 384, 384, 64, 0), ROWS128, 0), ((768, 384, 384, 32, 0), ROWS64, 0), ((64, 1268, 1268, 32, 0), SMALL, 0),
     ((64, 2209, 2209, 64, 0), ROWS128, 0), ((64, 2048, 2048, 64, 0), ROWS256, 0)])                              # full grids
 def test_lines_within_a_grid_size(choose, case, form, paired):
     assert choose(*case, 256) == (form, paired)
