@@ -86,8 +86,9 @@ int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64
   for (int i = 0; i < t.count; ++i) {
     const GemmAlgo& a = t.algos[i];
     if (!algo_supported(a, M, N, K, lda, ldb, align_bytes, layout)) continue;
-    // (the dword-aligned twins of the direct-to-LDS tiles are for what the 16-byte ones cannot take)
+    // (the twins for dword-aligned rows, and those for rows at any element, are for what the others cannot take)
     if (a.kvec == 2 && (a.direct_lds & 21) != 0 && align_bytes >= 16 && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0) continue;
+    if (a.kvec == 1 && a.direct_lds == 8 && align_bytes >= 4 && K % 2 == 0 && lda % 2 == 0 && ldb % 2 == 0) continue;
     if (a.direct_lds == 16 && !(plain_store && N % 8 == 0 && four_waves_multiply(a.kvec, K))) continue;
     int64_t slabs = ((a.kvec == 2 && a.direct_lds != 8 ? K & ~7ll : K) + a.bk - 1) / a.bk;
     int64_t tiles = ((M + a.bm - 1) / a.bm) * ((N + a.bn - 1) / a.bn) * batches;
