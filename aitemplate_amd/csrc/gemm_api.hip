@@ -119,6 +119,8 @@ int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64
     const double last_frac = a.direct_lds == 2 && rounds > 1 && 2 * last <= kNumCu ? 0.72 : 1.0;
     const double work = (double)(rounds - 1) * round_us(per_cu) + last_frac * round_us((double)busiest);
     cost += work > memory_us ? work + 0.3 * memory_us : memory_us + 0.3 * work;
+    // (between near equals not the four-wave kernel, which has one wave per SIMD for an epilogue; the fits are of a bias alone)
+    if (a.direct_lds == 16) cost *= 1.06;
     if (best < 0 || cost < best_cost) {
       best = i;
       best_cost = cost;
