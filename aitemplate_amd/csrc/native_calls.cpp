@@ -282,6 +282,8 @@ PyObject* bmm_softmax_bmm_permute(PyObject*, PyObject* const* args, Py_ssize_t n
     if (dt < 0) return not_ordinary();
     const int64_t B = t[0]->size(0), M = t[0]->size(1), K = t[0]->size(2), N = t[2]->size(1), O = t[2]->size(2);
     const int64_t G = PyLong_AsLongLong(args[3]);
+    // (raised here: the Python path would pass on what is left of it in 64 bits)
+    if (G == -1 && PyErr_Occurred()) return nullptr;
     if (t[1]->size(0) != B || t[1]->size(1) != N || t[1]->size(2) != K || t[2]->size(0) != B || G <= 0 || B % G != 0)
       return not_ordinary();
     at::Tensor made;
@@ -350,6 +352,13 @@ bool model_dtype(at::ScalarType s, AITemplateDtype* out) {
 
 typedef std::vector<std::pair<THPObjectPtr, size_t>> Names;
 
+// A Python integer from 0 to 2^63 - 1, or -1, without an error of Python's: such calls are declined
+int64_t small_integer(PyObject* o) {
+  const int64_t v = PyLong_AsLongLong(o);
+  if (v == -1) PyErr_Clear();
+  return v < 0 ? -1 : v;
+}
+
 // The tensors of a list, or of a dict ordered by `index` (name -> position), and the names in the order of the caller's
 // dict (of `index` for a list); false where they are not ordinary.  Both are held, not borrowed: the caller's containers
 // may change while the run has given up the interpreter lock.
@@ -374,9 +383,9 @@ bool model_tensors(PyObject* params, PyObject* index, std::vector<at::Tensor>* o
   Py_ssize_t pos = 0;
   while (PyDict_Next(by_name ? params : index, &pos, &name, &value)) {
     if (!PyUnicode_CheckExact(name)) return false;
-    PyObject* at_index = PyDict_GetItemWithError(index, name);
+    PyObject* at_index = PyDict_GetItemWithError(index, name);  // (no error: strings have hashes and compare)
     if (at_index == nullptr) return false;
-    const size_t i = (size_t)PyLong_AsLong(at_index);
+    const size_t i = (size_t)small_integer(at_index);
     if (i >= (size_t)n || (by_name && !hold(i, value))) return false;
     if (names != nullptr) names->emplace_back(THPObjectPtr::dup(name), i);
   }
@@ -419,7 +428,7 @@ PyObject* model_run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     std::vector<int64_t*> shapes(n_out);
     if ((size_t)PyList_GET_SIZE(args[4]) != n_out) return not_ordinary();
     for (size_t i = 0; i < n_out; ++i) {
-      const int64_t rank = PyLong_AsLongLong(PyList_GET_ITEM(args[4], (Py_ssize_t)i));
+      const int64_t rank = small_integer(PyList_GET_ITEM(args[4], (Py_ssize_t)i));
       if (rank != (int64_t)out_data.sizes[i].size() || dims.size() + (size_t)rank > dims.capacity()) return not_ordinary();
       shapes[i] = dims.data() + dims.size();
       dims.resize(dims.size() + (size_t)rank);

@@ -216,6 +216,27 @@ def test_calls_under_a_mode_are_declined(module, mode):
     """)
 
 
+def test_declined_calls_leave_no_error_behind(module):
+    """An integer that C cannot take: raised where the call ends with it, and nothing left set where it is declined (the
+    interpreter makes a SystemError of a result with an error set)."""
+    _run(module, """
+        for heads in (2 ** 70, -2 ** 70):   # (2 ** 64 + 1 taken modulo 2 ** 64 would be one head of an empty result)
+            try:
+                native.bmm_softmax_bmm_permute(q, q, q, heads, 0.125, False, None)
+            except OverflowError:
+                pass
+            else:
+                assert False, heads
+        y = torch.zeros(6, 72).half()
+        run = lambda index, ranks: native.model_run(8, 1, {"x": index}, {"y": 0}, ranks, [x], [y], None, True, False)
+        for index, ranks in ((0, [2 ** 70]), (0, ["2"]), (0, [None]), (2 ** 70, [2]), ("0", [2]), (-1, [2])):
+            assert run(index, ranks) is NotImplemented, (index, ranks)
+            by_name = native.model_run(8, 1, {"x": index}, {"y": 0}, ranks, {"x": x}, [y], None, True, False)
+            assert by_name is NotImplemented, (index, ranks)
+        assert launches() == 0
+    """)
+
+
 def test_errors_keep_their_types(module):
     """What torch raises through its own bindings: an allocation that fails is an OutOfMemoryError, without a C++ trace."""
     _run(module, """
