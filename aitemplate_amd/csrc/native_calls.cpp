@@ -140,6 +140,10 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   return guarded([&]() -> PyObject* {
     if (nargs != 9 || !PyUnicode_Check(args[0]) || !PyLong_CheckExact(args[7])) return not_ordinary();
     const char* op = PyUnicode_AsUTF8(args[0]);
+    if (op == nullptr) {  // (a lone surrogate)
+      PyErr_Clear();
+      return not_ordinary();
+    }
     const OpInfo* info = nullptr;
     for (const OpInfo& o : kOps)
       if (strcmp(o.name, op) == 0) info = &o;

@@ -237,6 +237,14 @@ def test_declined_calls_leave_no_error_behind(module):
     """)
 
 
+def test_an_op_name_without_utf8_is_declined(module):
+    """(The Python path has no such op and says so.)"""
+    _run(module, """
+        assert native.gemm("\\ud800", x, w, None, None, None, None, -1, None) is NotImplemented
+        assert launches() == 0
+    """)
+
+
 def test_errors_keep_their_types(module):
     """What torch raises through its own bindings: an allocation that fails is an OutOfMemoryError, without a C++ trace."""
     _run(module, """
