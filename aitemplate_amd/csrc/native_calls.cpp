@@ -10,6 +10,7 @@
 // outside of torch's modes.  For anything else they return NotImplemented without having done anything, and the caller's
 // Python path, which handles the remaining cases and words the errors, takes the call.
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/PyInterpreter.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 #include <torch/headeronly/version.h>
@@ -76,13 +77,36 @@ int dtype_id(const at::Tensor& t) {
   return s == at::kHalf ? 0 : (s == at::kBFloat16 ? 1 : -1);
 }
 
+// The class of the function mode behind `with torch.device(...)` and torch.set_default_device (null where torch has none)
+PyTypeObject* device_context_type() {
+  // (not an initializer of the static: the import may give up the interpreter lock, and others would wait with it held)
+  static PyTypeObject* type = nullptr;
+  if (type == nullptr) {
+    THPObjectPtr from(PyImport_ImportModule("torch.utils._device"));
+    PyObject* found = from ? PyObject_GetAttrString(from, "DeviceContext") : nullptr;
+    if (found == nullptr)
+      PyErr_Clear();
+    else if (type == nullptr && PyType_Check(found))
+      type = reinterpret_cast<PyTypeObject*>(found);  // (kept for good)
+    else
+      Py_DECREF(found);
+  }
+  return type;
+}
+
+// Whether every function mode gives new tensors a default device and no more: what is allocated here names its device
+bool device_contexts_only() {
+  for (int64_t i = at::impl::PythonTorchFunctionTLS::stack_len(); i-- > 0;)
+    if (Py_TYPE(at::impl::PythonTorchFunctionTLS::get_stack_at(i)->ptr(getPyInterpreter())) != device_context_type()) return false;
+  return true;
+}
+
 // False under a mode that sees, changes, records or refuses what the Python path does through torch (its allocation,
-// reshapes and views): dispatch modes, fake tensors among them, function modes (torch.set_default_device is one),
+// reshapes and views): dispatch modes, fake tensors among them, function modes other than those of a default device,
 // torch.func transforms, functionalization, tracing.  All but the function modes put a key of theirs into the thread's
 // dispatch keys; autocast, no_grad and inference mode put none.
 bool ordinary_context() {
-  return (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() &&
-      at::impl::PythonTorchFunctionTLS::stack_len() == 0;
+  return (c10::impl::tls_local_dispatch_key_set().included_ - c10::default_included_set).empty() && device_contexts_only();
 }
 
 // results of torch.empty that torch would have to fill are not ordinary

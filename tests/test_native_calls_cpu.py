@@ -245,6 +245,38 @@ def test_an_op_name_without_utf8_is_declined(module):
     """)
 
 
+@pytest.mark.parametrize("first", ["context", "default"])
+def test_a_default_device_changes_nothing(module, first):
+    """`with torch.device(...)` and torch.set_default_device say where tensors go whose device is not named: the calls name
+    it.  A class of that mode's that does more, or a mode beside it, is as any other mode."""
+    _run(module, f"""
+        from torch.overrides import TorchFunctionMode
+        from torch.utils._device import DeviceContext
+        class Derived(DeviceContext):
+            pass
+        class Function(TorchFunctionMode):
+            def __torch_function__(self, func, types, args=(), kwargs=None):
+                return func(*args, **(kwargs or {{}}))
+        call = lambda: native.gemm("gemm_rcr", x, w, None, None, None, None, -1, None)
+        def within():
+            out = call()
+            assert out is not NotImplemented and out.device == x.device
+            with Function():
+                assert call() is NotImplemented
+        if "{first}" == "context":
+            with torch.device("meta"):
+                within()
+        else:
+            torch.set_default_device("meta")
+            within()
+            torch.set_default_device(None)
+        assert launches() == 1
+        with Derived("meta"):
+            assert call() is NotImplemented
+        assert call() is not NotImplemented
+    """)
+
+
 def test_errors_keep_their_types(module):
     """What torch raises through its own bindings: an allocation that fails is an OutOfMemoryError, without a C++ trace."""
     _run(module, """
