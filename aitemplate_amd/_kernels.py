@@ -191,8 +191,9 @@ def load_native():
     try:
         from . import _native
 
-        built_for = getattr(_native, "torch_version", "unknown")
-        if built_for == torch.__version__.split("+")[0]:
+        # (the headers' version has no pre-release part: a module built for one of those names it beside that)
+        built_for = getattr(_native, "torch_build", getattr(_native, "torch_version", "unknown"))
+        if built_for.split("+")[0] == torch.__version__.split("+")[0]:
             return _native
         why = f"it was built for torch {built_for}, this is {torch.__version__}"
     except ImportError as e:

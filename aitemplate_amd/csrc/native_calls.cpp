@@ -30,6 +30,11 @@
 #include "../../include/model_interface.h"
 #include "native_device.h"
 
+// torch's own version string, pre-release part and all (the Makefile reads it from torch/version.py)
+#ifndef AITAMD_TORCH_BUILD
+#define AITAMD_TORCH_BUILD TORCH_VERSION
+#endif
+
 namespace {
 
 struct OpInfo {
@@ -504,6 +509,8 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "Eager calls and model 
 PyMODINIT_FUNC PyInit__native() {
   THPObjectPtr module(PyModule_Create(&kModule));
   // (the loader compares it with the torch that is there)
-  if (!module || PyModule_AddStringConstant(module.get(), "torch_version", TORCH_VERSION) != 0) return nullptr;
+  if (!module || PyModule_AddStringConstant(module.get(), "torch_version", TORCH_VERSION) != 0 ||
+      PyModule_AddStringConstant(module.get(), "torch_build", AITAMD_TORCH_BUILD) != 0)
+    return nullptr;
   return module.release();
 }

@@ -334,10 +334,35 @@ def test_without_the_extension_module_the_python_path_takes_every_call(why):
     assert done.returncode == 0, done.stdout
 
 
+@pytest.mark.parametrize("built,here,used", [
+    ("2.10.0", "2.10.0", True), ("2.10.0+rocm7.0", "2.10.0+rocm7.0", True), ("2.10.0+rocm7.0", "2.10.0+local", True),
+    ("2.10.0", "2.11.0", False), ("2.11.0a0+git0123abc", "2.11.0a0+git0123abc", True), ("2.11.0a0", "2.11.0", False),
+    ("2.11.0.dev20260101", "2.11.0.dev20260101+rocm7.0", True), ("2.11.0.dev20260101", "2.11.0.dev20260102", False)])
+def test_the_module_is_used_with_the_torch_it_was_built_for(monkeypatch, built, here, used):
+    """Pre-releases too: the version that torch names at run time, not the three numbers of its headers."""
+    import types
+    import warnings
+
+    import aitemplate_amd
+    from aitemplate_amd import _kernels
+
+    there = types.ModuleType("aitemplate_amd._native")
+    there.torch_version, there.torch_build = built.split("a0")[0].split(".dev")[0].split("+")[0], built
+    monkeypatch.setitem(sys.modules, "aitemplate_amd._native", there)
+    monkeypatch.setattr(aitemplate_amd, "_native", there, raising=False)
+    monkeypatch.setattr(torch, "__version__", here)
+    with warnings.catch_warnings(record=True) as seen:
+        warnings.simplefilter("always")
+        assert (_kernels.load_native() is there) is used
+    assert bool(seen) is not used
+
+
 def test_the_built_module_fits_this_torch():
     from aitemplate_amd import _kernels
 
-    assert _kernels.load_native().torch_version == torch.__version__.split("+")[0]
+    native = _kernels.load_native()
+    assert native.torch_version == torch.__version__.split("+")[0]
+    assert native.torch_build == torch.__version__
 
 
 def test_the_kernel_library_builds_without_torch(tmp_path):
