@@ -431,20 +431,22 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_wide_kernel(const GemmPa
         const int rows_b = (p.N - cur.n0) < BN ? (p.N - cur.n0) : BN;
         const __amdgpu_buffer_rsrc_t ra = make_rsrc(Ab, clamp_records((((int64_t)rows_a - 1) * p.lda + p.K) * 2));
         const __amdgpu_buffer_rsrc_t rb = make_rsrc(Bb, clamp_records((((int64_t)rows_b - 1) * p.ldb + p.K) * 2));
-        auto tail = [&](const __amdgpu_buffer_rsrc_t& r, int row, int64_t ld) __attribute__((always_inline)) {
-          uint32_t w[3];
+        // (opaque: offsets computed once for all tiles would be spilled, while the first tile's fragments are on their way)
+        auto tail = [&](auto n_c, vec8* t, const __amdgpu_buffer_rsrc_t& r, int row, int64_t ld) __attribute__((always_inline)) {
+          uint32_t at = (uint32_t)((row * (int)ld + k_main) * 2), zero = 0;
+          asm volatile("" : "+v"(at), "+v"(zero));
+          uint32_t off[3];
 #pragma unroll
-          for (int d = 0; d < 3; ++d) {
-            const int k = k_main + 2 * d;
-            w[d] = buffer_load_4B(r, fq == 0 && k < p.K ? (uint32_t)(((int64_t)row * ld + k) * 2) : kOobOffset);
+          for (int d = 0; d < 3; ++d) off[d] = fq == 0 && k_main + 2 * d < p.K ? at + 4 * d : kOobOffset;
+#pragma unroll
+          for (int i = 0; i < decltype(n_c)::value; ++i) {
+            const uint32_t rows = (uint32_t)(i * 16 * (int)ld * 2);
+            t[i] = __builtin_bit_cast(vec8, u32x4{buffer_load_4B(r, off[0] + rows), buffer_load_4B(r, off[1] + rows), buffer_load_4B(r, off[2] + rows), zero});
           }
-          return __builtin_bit_cast(vec8, u32x4{w[0], w[1], w[2], 0u});
         };
         vec8 ta[MI], tb[NI];
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi) ta[mi] = tail(ra, wm * Tile::WTM + mi * 16 + fr, p.lda);
-#pragma unroll
-        for (int ni = 0; ni < NI; ++ni) tb[ni] = tail(rb, wn * Tile::WTN + ni * 16 + fr, p.ldb);
+        tail(std::integral_constant<int, MI>{}, ta, ra, wm * Tile::WTM + fr, p.lda);
+        tail(std::integral_constant<int, NI>{}, tb, rb, wn * Tile::WTN + fr, p.ldb);
         asm volatile("s_nop 7" ::: "memory");
         static_for<0, MI * NI>([&](auto x_c) __attribute__((always_inline)) {
           constexpr int x = decltype(x_c)::value;
