@@ -28,11 +28,18 @@ inline Form choose_form(int64_t B, int64_t M, int64_t N, int ks, int ot, bool ca
   // head dims up to 64: four workgroups of kRows128 on a CU, two of larger ones
   const bool narrow = ks <= 4 && ot <= 2, mid = !narrow && ks <= 6 && ot <= 3;
   *paired = 0;
-  // Few keys give groups nothing to share.  48 x 28 x 28 at head dim 160: 8.9 in two groups, 7.0 in one; 12 x 316 x 77
-  // at head dim 128 8.4 / 10.2.  128 rows where they leave one workgroup per CU (48 x 390 x 77 at head dim 32: 4.7, with
-  // 64 rows 5.3) and in large grids, which are wide or K and V are read the less (272 x 3954 x 77 at head dim 40 59 / 67).
-  if (M <= 64 && (N <= 32 || ks > 2 || t64 > cus)) return kRows64;  // 992 x 34^2: 6.6, 8.2 with 128 rows
-  if (M > 64 && (N <= 96 || (ot > 4 && N <= 192)))
+  // Few queries: two groups halve the chain over the keys while all workgroups fit the chip at once (of kSmall one per CU at
+  // head dims 128 and up, two below, three at 32).  64 x 1 x 4096 55 in one group, 32 in two; 554 x 21 x 1180 27.7 / 30.6.
+  // Few keys give the second group nothing to share, three tiles of 32 too little: 48 x 28 x 28 at head dim 160 7.0 / 8.9.
+  if (M <= 64) {
+    const int64_t keys = causal && N > 64 ? 64 : N;  // (a causal tile stops behind its last row)
+    const bool share = narrow || mid ? keys > 32 && (keys <= 64 || keys > 96) : keys > 192;
+    return share && t64 <= cus * (ks <= 2 ? 3 : (narrow || mid ? 2 : 1)) ? kSmall : kRows64;  // 992 x 34^2: 6.6, 8.2 with 128 rows
+  }
+  // Few keys for more queries: 12 x 316 x 77 at head dim 128 8.4 in one group, 10.2 in two.  128 rows where they leave one
+  // workgroup per CU (48 x 390 x 77 at head dim 32: 4.7, with 64 rows 5.3) and in large grids, which are wide or K and V are
+  // read the less (272 x 3954 x 77 at head dim 40 59 / 67).
+  if (N <= 96 || (ot > 4 && N <= 192))
     return t64 <= cus || (narrow && t128 > cus && (causal || t64 <= 8 * cus)) ? kRows64 : kRows128;
   // Grids that leave CUs idle: 64-row workgroups whose groups share the keys.  12 x 384^2 9.5 (128 rows, one group) / 8.6
   // (128, two) / 7.1 (64, two); 8 x 2048^2 at head dim 128 41 / 38 / 33.  A little beyond, while 128 rows still fill one

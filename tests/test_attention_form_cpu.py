@@ -62,6 +62,20 @@ def test_lines_within_a_grid_size(choose, case, form, paired):
     assert choose(*case, 256) == (form, paired)
 
 
+@pytest.mark.parametrize("d", [32, 40, 64, 80, 128, 160])
+@pytest.mark.parametrize("M", [1, 16, 64])
+def test_few_queries_over_many_keys_share_them(choose, d, M):
+    """Two groups halve the chain over the keys as long as all workgroups fit the chip at once; no chain under a causal mask."""
+    resident = 256 * (3 if d <= 32 else 2 if d <= 96 else 1)
+    for N in (256, 1024, 4096):
+        for B in (1, 8, 64, resident):
+            assert choose(B, M, N, d, 0, 256) == (SMALL, 0), (B, N)
+        assert choose(resident + 1, M, N, d, 0, 256) == (ROWS64, 0), N
+    for N in (1, 32, 96 if d > 32 else 32, 192 if d > 96 else 32):
+        assert choose(8, M, N, d, 0, 256) == (ROWS64, 0), N
+    assert choose(8, M, 4096, d, 1, 256) == choose(8, M, 64, d, 1, 256) == choose(8, M, 64, d, 0, 256)
+
+
 def test_pairs_are_of_causal_tiles_that_the_grid_can_hold(choose):
     rng = random.Random(1)
     for _ in range(20000):

@@ -83,6 +83,13 @@ def test_forms_chosen_within_a_grid_size(B, M, N, d, causal):
     _check(B, M, N, d, d, 4 if B % 4 == 0 else 2, causal, seed=M + d)
 
 
+@pytest.mark.parametrize("B,M,N,d,causal", [
+    (8, 1, 1000, 64, False), (16, 16, 4096, 40, False), (512, 64, 257, 80, False), (768, 5, 130, 32, False),
+    (256, 33, 193, 160, False), (8, 64, 700, 128, True), (520, 7, 600, 64, False)])
+def test_few_queries_over_many_keys(B, M, N, d, causal):
+    _check(B, M, N, d, d, 4, causal, seed=N + d)
+
+
 @pytest.mark.parametrize("B,M,N,K,O,G,causal", [
     (16, 256, 256, 160, 160, 8, False),     # the deepest attention of Stable Diffusion v1: 1280 channels, 8 heads
     (8, 100, 77, 160, 160, 8, False),       # its cross-attention over 77 text tokens
