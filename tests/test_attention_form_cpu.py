@@ -56,9 +56,27 @@ def test_lines_move_with_the_number_of_cus(choose):
     ((248, 1781, 1781, 64, 1), ROWS128, 1), ((224, 400, 400, 40, 1), ROWS64, 0),                                # causal, narrow
     ((24, 1741, 1741, 80, 1), SMALL, 0), ((36, 3341, 3341, 80, 1), ROWS128, 1), ((96, 639, 639, 128, 1), ROWS128, 0),
     ((208, 397, 397, 80, 1), ROWS128, 1), ((164, 268, 268, 80, 1), ROWS64, 0), ((70000, 600, 600, 64, 1), ROWS64, 0),
-    ((768, 256, 256, 64, 0), ROWS64, 0), ((768, 384, 384, 64, 0), ROWS128, 0), ((768, 384, 384, 32, 0), ROWS64, 0), ((64, 1268, 1268, 32, 0), SMALL, 0),
+    ((768, 256, 256, 64, 0), ROWS128, 0), ((768, 384, 384, 64, 0), ROWS128, 0), ((768, 384, 384, 32, 0), ROWS64, 0), ((64, 1268, 1268, 32, 0), SMALL, 0),
     ((64, 2209, 2209, 64, 0), ROWS128, 0), ((64, 2048, 2048, 64, 0), ROWS256, 0)])                              # full grids
 def test_lines_within_a_grid_size(choose, case, form, paired):
+    assert choose(*case, 256) == (form, paired)
+
+
+# where the lines are drawn differently from before: us, and those of the form on the line's other side
+@pytest.mark.parametrize("case,form,paired", [
+    ((768, 256, 256, 64, 0), ROWS128, 0), ((768, 200, 200, 40, 0), ROWS128, 0),       # 27.0, 29.4 with 64 rows; 17.7, 20.7
+    ((768, 135, 135, 64, 0), ROWS64, 0), ((192, 256, 256, 64, 0), ROWS64, 0),         # (half of 128 rows empty; few workgroups)
+    ((244, 381, 381, 32, 0), ROWS128, 0),                                             # 12.7, 14.7 with 64 rows
+    ((168, 748, 77, 64, 0), ROWS128, 0), ((256, 3234, 77, 40, 1), ROWS128, 0),        # 12.0, 14.2; 41.8, 47.7
+    ((32, 3290, 328, 40, 1), ROWS128, 0),                                             # 17.1, 21.8 with two groups of 64 rows
+    ((8, 6164, 6164, 128, 1), GROUPS, 1), ((24, 2161, 2161, 40, 1), GROUPS, 1),       # 107, 132 unpaired; 27, 36
+    ((8, 2563, 2563, 160, 1), SMALL, 0), ((32, 703, 703, 160, 1), GROUPS, 0),         # 50, 58 in groups of 128 rows
+    ((128, 474, 474, 40, 1), ROWS64, 0), ((96, 1154, 1154, 40, 1), ROWS128, 1),       # 12.9, 15.5 in two groups; 31.4, 33.2
+    ((112, 629, 629, 32, 1), SMALL, 0), ((880, 135, 77, 64, 1), ROWS64, 0),           # 12.4, 15.9 with 64 rows; 14.7, 17.8 with 128
+    ((180, 1274, 1274, 64, 1), ROWS128, 1), ((240, 993, 993, 64, 1), ROWS128, 1),     # 65.9, 73.8 with 64 rows; 58, 65
+    ((156, 1143, 1143, 64, 1), ROWS64, 1), ((200, 702, 702, 64, 1), ROWS64, 1),       # 49, 57 with 128 rows; 31, 35
+    ((64, 4811, 4811, 64, 0), ROWS256, 0), ((60, 3092, 3092, 64, 0), ROWS128, 0)])    # 429, 460 with 128 rows; 188, 215 with 256
+def test_lines_between_forms_on_256_cus(choose, case, form, paired):
     assert choose(*case, 256) == (form, paired)
 
 

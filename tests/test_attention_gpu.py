@@ -78,6 +78,7 @@ def test_every_variant_of_the_small_head_dims(attn_variant, mode, B, M, N, K, O,
     (260, 520, 520, 32, True),   # pairs of 64-row tiles, nine of them: the middle one by itself, the last of eight rows
     (132, 961, 961, 64, True),   # sixteen of them, the last of one row
     (36, 641, 641, 64, True),    # two groups of 64 rows, causal, beyond the CUs: the longest first
+    (40, 1100, 500, 40, True), (260, 135, 77, 64, True),  # half as many keys as queries, and few
     (60, 257, 300, 128, False), (136, 129, 394, 32, False), (24, 1025, 1025, 80, True)])
 def test_forms_chosen_within_a_grid_size(B, M, N, d, causal):
     _check(B, M, N, d, d, 4 if B % 4 == 0 else 2, causal, seed=M + d)
