@@ -11,6 +11,8 @@
 // fp32, which differs from it by at most a few fp16 ulps.
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace aitamd {
@@ -116,6 +118,49 @@ AITAMD_DEVICE float apply_folded(float xb, T d0, T d1, float one) {
   const float f0 = Epi::kLeadingAdds >= 1 ? -0.0f : (Epi::kNumD >= 1 ? Tr::to_float(d0) : 0.0f);
   const float f1 = Epi::kLeadingAdds >= 2 ? -0.0f : (Epi::kNumD >= 2 ? Tr::to_float(d1) : 0.0f);
   return Epi::apply(xb, -0.0f, f0, f1);
+}
+
+// acc + b to a half, rounded once, in the instruction that adds (v_fma_mixlo_f16).  Each by itself, opaque to the optimizer: it
+// would take two of eight neighbours so and round the others to 32 bits first, and the last bit of a sum next to a tie would
+// depend on its column and on the kernel (a permuted store could differ from a plain one).
+AITAMD_DEVICE f16 half_sum(float acc, f16 b, float one) {
+  f16 h = (f16)__builtin_fmaf((float)b, one, acc);
+  asm("" : "+v"(h));
+  return h;
+}
+
+// Eight results of a row: accumulators, bias and residuals to elements
+template <class Epi, class T>
+AITAMD_DEVICE typename ElemTraits<T>::vec8 epilogue8(const float (&v)[8], typename ElemTraits<T>::vec8 b, typename ElemTraits<T>::vec8 d0,
+                                                     typename ElemTraits<T>::vec8 d1, float one) {
+  using Tr = ElemTraits<T>;
+  using vec8 = typename Tr::vec8;
+  if constexpr (Epi::kId == kEpiBias && std::is_same_v<T, f16>) {
+    vec8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = half_sum(v[j], b[j], one);
+    return o;
+  } else {
+    vec8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      // bias conversion and add as one instruction where the type has one; -0.0 is the bias that adds nothing
+      const float xb = Epi::kHasBias ? Tr::to_float_plus(b[j], one, v[j]) : v[j];
+      o[j] = Tr::from_float(apply_folded<Epi, T>(xb, d0[j], d1[j], one));
+    }
+    return o;
+  }
+}
+// ... and one
+template <class Epi, class T>
+AITAMD_DEVICE T epilogue1(float v, T b, T d0, T d1, float one) {
+  using Tr = ElemTraits<T>;
+  if constexpr (Epi::kId == kEpiBias && std::is_same_v<T, f16>) {
+    return half_sum(v, b, one);
+  } else {
+    return Tr::from_float(Epi::apply(v, Epi::kHasBias ? Tr::to_float(b) : 0.0f, Epi::kNumD >= 1 ? Tr::to_float(d0) : 0.0f,
+                                     Epi::kNumD >= 2 ? Tr::to_float(d1) : 0.0f));
+  }
 }
 
 }  // namespace aitamd

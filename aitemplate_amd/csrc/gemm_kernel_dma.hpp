@@ -695,23 +695,17 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
             if constexpr (Epi::kHasBias && !kEarlyBias) bv = load_vec<vec8>(bias + n);
             if constexpr (Epi::kNumD >= 1 && kEarlyD == 0) d0v = load_vec<vec8>(D0b + d_idx);
             if constexpr (Epi::kNumD >= 2 && kEarlyD == 0) d1v = load_vec<vec8>(D1b + d_idx);
-            vec8 o;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              // bias conversion and add as one instruction where the type has one; -0.0 is the bias that adds nothing
-              const float xb = Epi::kHasBias ? Tr::to_float_plus(bv[j], one, v[j]) : v[j];
-              o[j] = Tr::from_float(apply_folded<Epi, T>(xb, d0v[j], d1v[j], one));
-            }
+            const vec8 o = epilogue8<Epi, T>(v, bv, d0v, d1v, one);
             store_out(Cb, c_idx, o, stream_ok, rc);
           } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
               if (n + j < p.N) {
-                float bj = 0.f, d0j = 0.f, d1j = 0.f;
-                if constexpr (Epi::kHasBias) bj = Tr::to_float(bias[n + j]);
-                if constexpr (Epi::kNumD >= 1) d0j = Tr::to_float(D0b[d_idx + j]);
-                if constexpr (Epi::kNumD >= 2) d1j = Tr::to_float(D1b[d_idx + j]);
-                Cb[out_index<PERM>(p, m, n + j)] = Tr::from_float(Epi::apply(v[j], bj, d0j, d1j));
+                T bj = T{}, d0j = T{}, d1j = T{};
+                if constexpr (Epi::kHasBias) bj = bias[n + j];
+                if constexpr (Epi::kNumD >= 1) d0j = D0b[d_idx + j];
+                if constexpr (Epi::kNumD >= 2) d1j = D1b[d_idx + j];
+                Cb[out_index<PERM>(p, m, n + j)] = epilogue1<Epi, T>(v[j], bj, d0j, d1j, one);
               }
             }
           }

@@ -208,6 +208,8 @@ __global__ void __launch_bounds__(Tile::NT) gemm_rcr_rows_kernel(const GemmParam
   float* const part = reinterpret_cast<float*>(smem_raw);  // [NW][16 rows of A][16 columns]
   *reinterpret_cast<f32x4*>(part + (wave * BM + fr) * BN + fq * 4) = acc;
   __syncthreads();
+  float one = 1.0f;
+  asm volatile("" : "+s"(one));  // (opaque to the optimizer: see to_float_plus)
   T* Cb = reinterpret_cast<T*>(p.c) + out_batch_offset(p, batch);
 #pragma unroll
   for (int o = 0; o < OUTS; ++o) {
@@ -216,8 +218,7 @@ __global__ void __launch_bounds__(Tile::NT) gemm_rcr_rows_kernel(const GemmParam
       float v = 0.0f;
 #pragma unroll
       for (int w = 0; w < NW; ++w) v += part[(w * BM + m) * BN + out_n];
-      Cb[out_index<PERM>(p, m0 + m, n0 + out_n)] =
-          Tr::from_float(Epi::apply(v, Tr::to_float(bias_v[o]), Tr::to_float(d0_v[o]), Tr::to_float(d1_v[o])));
+      Cb[out_index<PERM>(p, m0 + m, n0 + out_n)] = epilogue1<Epi, T>(v, bias_v[o], d0_v[o], d1_v[o], one);
     }
   }
 }

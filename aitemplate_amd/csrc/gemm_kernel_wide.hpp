@@ -341,12 +341,7 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_wide_kernel(const GemmPa
           v[4 + j] = y[j];
           swap_rows16(v[j], v[4 + j]);
         }
-        vec8 o;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float xb = Epi::kHasBias ? Tr::to_float_plus(bv[u][j], one, v[j]) : v[j];
-          o[j] = Tr::from_float(apply_folded<Epi, T>(xb, d0v[s][j], d1v[s][j], one));
-        }
+        const vec8 o = epilogue8<Epi, T>(v, bv[u], d0v[s], d1v[s], one);
         auto store = [&](u32x4 v, uint32_t off) __attribute__((always_inline)) {
           __builtin_amdgcn_raw_buffer_store_b128(v, rc, off + (uint32_t)(row * (int)p.ldc * 2), 0, NT_BITS);
         };

@@ -79,6 +79,28 @@ def test_every_instance_stores_permuted(algo, name):
         _case(op, M, N, K, shape, algo=algo, seed=algo)
 
 
+@pytest.mark.parametrize("K", [192, 194])
+def test_a_sum_next_to_a_tie_is_rounded_once_in_every_column(K):
+    """1 + 2^-11, half way between two halves, + a bias of 2^-24: above the tie, on it when rounded to 32 bits first.  Every
+    instance that keeps its accumulators in 32 bits up to the bias gives 1 + 2^-10, in whole pieces and at the ragged end."""
+    M, N = 70, 133 * 4
+    x, w, b = torch.zeros(M, K), torch.zeros(N, K), torch.full((N,), 2.0 ** -24)
+    x[:, :2], w[:, 0], w[:, 1] = 1.0, 1.0, 2.0 ** -11
+    x, b = x.half().cuda(), b.half().cuda()
+    lib, seen = _kernels.load(), 0
+    for algo, name in _algos():
+        if "_persist" in name or not lib.aitamd_gemm_algo_supported(1, 0, algo, M, N, K, K, K, 16 if K % 8 == 0 else 4):
+            continue
+        print(f"case sum next to a tie K={K} instance={name}", flush=True)
+        for n in (N, N - 1):
+            plain = eager.gemm("gemm_rcr_bias", x, w[:n].half().cuda(), b[:n], algo=algo)
+            assert bool((plain == 1.0 + 2.0 ** -10).all()), (name, n)
+        got = eager.gemm_permute("gemm_rcr_bias_permute_m2n3", x, w.half().cuda(), b, (70, 4, 7), algo=algo)
+        assert bool((got == 1.0 + 2.0 ** -10).all()), name
+        seen += 1
+    assert seen > 5
+
+
 def test_argument_errors():
     x = torch.zeros(12, 8, dtype=torch.float16, device="cuda:0")
     w = torch.zeros(24, 8, dtype=torch.float16, device="cuda:0")
