@@ -136,10 +136,17 @@ AITAMD_DEVICE typename ElemTraits<T>::vec8 epilogue8(const float (&v)[8], typena
   using Tr = ElemTraits<T>;
   using vec8 = typename Tr::vec8;
   if constexpr (Epi::kId == kEpiBias && std::is_same_v<T, f16>) {
-    vec8 o;
+    u32x4 o;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = half_sum(v[j], b[j], one);
-    return o;
+    for (int q = 0; q < 4; ++q) {
+      typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+      // (the second one written to the upper half in place, v_fma_mixhi_f16)
+      const f16x2 pair = {half_sum(v[2 * q], b[2 * q], one), (f16)__builtin_fmaf((float)b[2 * q + 1], one, v[2 * q + 1])};
+      uint32_t w = __builtin_bit_cast(uint32_t, pair);
+      asm("" : "+v"(w));
+      o[q] = w;
+    }
+    return __builtin_bit_cast(vec8, o);
   } else {
     vec8 o;
 #pragma unroll
