@@ -305,17 +305,10 @@ const GemmAlgo kAlgos[] = {
 #define AITAMD_GEMM_TILE_PERSIST(BM, BN, BK, WM, WN, NS, MT, LBM, ...)                                               \
   entry<GemmTilePersist<BM, BN, BK, WM, WN, NS, MT, LBM>, 2, 1>(                                                     \
       AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_persist" #NS "_m" #MT, {__VA_ARGS__}),
-// (not for the bias of halves, whose sum and conversion the compiler may or may not take in one instruction: a permuted store
-// of an instance has to give the bits of its plain one, and these have none of their own)
-#if AITAMD_EPI == 1 && AITAMD_DT == 0
-#define AITAMD_GEMM_TILE_WIDE(...)
-#define AITAMD_GEMM_TILE_WIDE_K2(...)
-#else
 #define AITAMD_GEMM_TILE_WIDE(MI, NI, BM, BN, ...)                                                                   \
   entry<GemmTileWide<MI, NI, 0>, 16, 1>(AITAMD_NAME #BM "x" #BN "x32_w2x2_wide", {__VA_ARGS__}),
 #define AITAMD_GEMM_TILE_WIDE_K2(MI, NI, BM, BN, ...)                                                                \
   entry<GemmTileWide<MI, NI, 1>, 16, 1>(AITAMD_NAME #BM "x" #BN "x32_w2x2_wide_k2", {__VA_ARGS__}),
-#endif
 #define AITAMD_GEMM_TILE_DMA_SPLITK(BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, ...)                                      \
   entry<GemmTileDma<BM, BN, BK, WM, WN, NS, OCC, PIPE, MT, 0, 1>, 4, OCC>(                                           \
       AITAMD_NAME #BM "x" #BN "x" #BK "_w" #WM "x" #WN "_dma" #NS "_o" #OCC "_p" #PIPE "_m" #MT "_splitk", {__VA_ARGS__}),

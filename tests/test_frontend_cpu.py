@@ -1122,3 +1122,15 @@ def test_non_finite_constant_operands_are_spelled_as_cmath_macros(tmp_path):
                         f"-I{os.path.join(ROOT, 'include')}", f"-I{os.path.join(ROOT, 'aitemplate_amd', 'static', 'include')}",
                         str(f)], capture_output=True, text=True)
     assert r.returncode == 0, r.stderr[-2000:]
+
+
+def test_every_linear_layer_has_the_same_instances():
+    """An epilogue or a type without an instance that the others have would run its large products on a slower one."""
+    from aitemplate_amd import _kernels
+
+    want = _kernels.gemm_algo_names(2, 0)
+    assert any(n.endswith("_wide") for n in want) and any(n.endswith("_wide_k2") for n in want)
+    for epilogue in sorted(set(_kernels.EPILOGUE_OF_OP.values())):
+        for dtype in (0, 1):
+            names = [n.replace("_bf16_", "_f16_") for n in _kernels.gemm_algo_names(epilogue, dtype)]
+            assert names == want, (epilogue, dtype)

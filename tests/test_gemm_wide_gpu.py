@@ -68,9 +68,15 @@ def test_wide_dword_rows(name, M, N, K):
 @pytest.mark.parametrize("name", ALIGNED + DWORDS)
 @pytest.mark.parametrize("op", sorted(set(_kernels.EPILOGUE_OF_OP) - {"bmm_rcr"}))
 def test_wide_every_epilogue(name, op):
-    # (the bias of halves alone has no such instances: see the table)
+    # (the bias alone: of halves below)
     dtype = torch.bfloat16 if _kernels.EPILOGUE_OF_OP[op] == 1 else torch.float16
     _check(op, name, 500, 472, 322 if name in DWORDS else 320, dtype, seed=7)
+
+
+@pytest.mark.parametrize("name", ALIGNED + DWORDS)
+def test_wide_bias_of_halves(name):
+    for M, N, K in ((500, 472, 320), (257, 264, 136), (4100, 4200, 200)):
+        _check("gemm_rcr_bias", name, M, N, K + 2 if name in DWORDS else K, pitch=8, seed=K)
 
 
 @pytest.mark.parametrize("name", ALIGNED + DWORDS)
