@@ -53,6 +53,7 @@ DTYPE_ID = {"float16": 0, "bfloat16": 1}
 # python/aitemplate/compiler/ops/gemm_universal/).
 PERMUTE_M2N3, PERMUTE_M3N2 = 1, 2
 LAYOUT_ID = {"rcr": 0, "rrr": 1, "ccr": 2, "crr": 3}
+LAYOUT_RCR_PERMUTED = 4  # of the questions about instances: rcr operands and a permuted store
 # plain-epilogue ops launched through aitamd_bmm / aitamd_bmm_rcr_permute
 LAYOUT_OPS = ("bmm_rcr_permute", "bmm_rrr", "bmm_rrr_permute", "bmm_ccr", "bmm_crr", "gemm_rrr",
               "bmm_rrr_add", "bmm_ccr_add", "bmm_crr_add")

@@ -32,6 +32,11 @@ def _layout(func_attrs):
     return lay, lay[0] == "c", lay[1] == "r"
 
 
+def _layout_asked(func_attrs) -> int:
+    """The layout to ask the library's instances about."""
+    return _kernels.LAYOUT_RCR_PERMUTED if func_attrs["op"] == "bmm_rcr_permute" else _kernels.LAYOUT_ID[_layout(func_attrs)[0]]
+
+
 def _pitches(func_attrs, m, n, k):
     _, a_col, b_row = _layout(func_attrs)
     return (m if a_col else k), (n if b_row else k)
@@ -49,7 +54,7 @@ def _filter(instance_name, func_attrs, ab_alignment) -> bool:
     """True when the instance has a kernel for the op's layout and can run every profiled workload."""
     lib = _kernels.load()
     dtype = common.DTYPE_ID[func_attrs["inputs"][0]._attrs["dtype"]]
-    lay = _kernels.LAYOUT_ID[_layout(func_attrs)[0]]
+    lay = _layout_asked(func_attrs)
     algo = func_attrs["op_instance"][instance_name]
     dyn_a, dyn_b = _dynamic_pitch(func_attrs)
     for key in func_attrs["exec_path"]:
@@ -75,7 +80,7 @@ def _dynamic_pitch(func_attrs):
 def _select_algo(func_attrs, exec_key) -> str:
     lib = _kernels.load()
     dtype = common.DTYPE_ID[func_attrs["inputs"][0]._attrs["dtype"]]
-    lay = _kernels.LAYOUT_ID[_layout(func_attrs)[0]]
+    lay = _layout_asked(func_attrs)
     dims = gemm_inverse_key_func(exec_key)
     m, n, k = dims[-3:]
     batch = dims[0] if len(dims) == 4 else 1

@@ -87,34 +87,32 @@ def _config(func_attrs, dtype="float16"):
     common.gemm_config(func_attrs, dtype, "gemm_permute")
 
 
-def _filter(instance_name, func_attrs, ab_alignment) -> bool:
+def _problem(func_attrs, key):
+    """(layout to ask the library about, m, n, k, ldb)"""
+    m, n, k = gemm_inverse_key_func(key)[-3:]
     operands = _operands(func_attrs["op"])
-    if operands == 0:
-        return common.gemm_filter(instance_name, func_attrs, ab_alignment)
+    return (operands, m, n, k, n) if operands else (_kernels.LAYOUT_RCR_PERMUTED, m, n, k, k)
+
+
+def _filter(instance_name, func_attrs, ab_alignment) -> bool:
     lib = _kernels.load()
     dtype = common.DTYPE_ID[func_attrs["inputs"][0]._attrs["dtype"]]
     epi = _kernels.PERMUTE_OPS[func_attrs["op"]][0]
     algo = func_attrs["op_instance"][instance_name]
     for key in func_attrs["exec_path"]:
-        m, n, k = gemm_inverse_key_func(key)[-3:]
-        if not lib.aitamd_gemm_algo_supported_layout(epi, dtype, operands, algo, m, n, k, k, n,
-                                                     max(2, min(16, ab_alignment * 2))):
+        layout, m, n, k, ldb = _problem(func_attrs, key)
+        if not lib.aitamd_gemm_algo_supported_layout(epi, dtype, layout, algo, m, n, k, k, ldb, max(2, min(16, ab_alignment * 2))):
             return False
     return True
 
 
 def _select_algo(func_attrs, exec_key) -> str:
-    operands = _operands(func_attrs["op"])
     lib = _kernels.load()
     dtype = common.DTYPE_ID[func_attrs["inputs"][0]._attrs["dtype"]]
     epi = _kernels.PERMUTE_OPS[func_attrs["op"]][0]
-    m, n, k = gemm_inverse_key_func(exec_key)[-3:]
-    if operands == 0:
-        # (4: rcr operands, permuted store)
-        align = next(a for a in (16, 8, 4, 2) if k * 2 % a == 0)
-        algo = lib.aitamd_gemm_heuristic_algo_layout(epi, dtype, 4, 1, m, n, k, k, k, align)
-    else:
-        algo = lib.aitamd_gemm_heuristic_algo_layout(epi, dtype, operands, 1, m, n, k, k, n, 16)
+    layout, m, n, k, ldb = _problem(func_attrs, exec_key)
+    align = 16 if layout != _kernels.LAYOUT_RCR_PERMUTED else next(a for a in (16, 8, 4, 2) if k * 2 % a == 0)
+    algo = lib.aitamd_gemm_heuristic_algo_layout(epi, dtype, layout, 1, m, n, k, k, ldb, align)
     all_names = _kernels.gemm_algo_names(epi, dtype)
     if algo >= 0 and all_names[algo] in func_attrs["op_instance"]:
         return all_names[algo]

@@ -240,15 +240,16 @@ int aitamd_gemm_algo_supported_layout(int epilogue, int dtype, int layout, int a
                                       int64_t lda, int64_t ldb, int align_bytes) {
   const GemmAlgoTable t = gemm_table(epilogue, dtype);
   if (algo < 0 || algo >= t.count) return 0;
-  return algo_supported(t.algos[algo], M, N, K, lda, ldb, align_bytes, layout) ? 1 : 0;
+  // (the four-wave instances hand a permuted store on to a small tile: no candidates for one)
+  if (layout == AITAMD_LAYOUT_RCR_PERMUTED && t.algos[algo].direct_lds == 16) return 0;
+  return algo_supported(t.algos[algo], M, N, K, lda, ldb, align_bytes, layout == AITAMD_LAYOUT_RCR_PERMUTED ? 0 : layout) ? 1 : 0;
 }
 
 int aitamd_gemm_heuristic_algo_layout(int epilogue, int dtype, int layout, int64_t batch, int64_t M, int64_t N,
                                       int64_t K, int64_t lda, int64_t ldb, int align_bytes) {
   const GemmAlgoTable t = gemm_table(epilogue, dtype);
   if (t.count == 0) return -1;
-  constexpr int kPermuted = 4;  // rcr operands, an output stored permuted
-  return heuristic(t, batch, M, N, K, lda, ldb, align_bytes, layout == kPermuted ? 0 : layout, false, layout != kPermuted);
+  return heuristic(t, batch, M, N, K, lda, ldb, align_bytes, layout == AITAMD_LAYOUT_RCR_PERMUTED ? 0 : layout, false, layout != AITAMD_LAYOUT_RCR_PERMUTED);
 }
 
 int aitamd_gemm_heuristic_algo(int epilogue, int dtype, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t lda,

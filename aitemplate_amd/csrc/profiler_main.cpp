@@ -257,6 +257,8 @@ int profile_gemm_like(const std::string& op, int dtype, int64_t B, int64_t M, in
       if (!aitamd_gemm_algo_supported_layout(epi, dtype, perm.operands, algo, M, N, K, lda, ldb, 16)) continue;
     } else if (!aitamd_gemm_algo_supported(epi, dtype, algo, M, N, K, K, K, 16)) {
       continue;
+    } else if (perm.layout && !(only && *only) && !aitamd_gemm_algo_supported_layout(epi, dtype, AITAMD_LAYOUT_RCR_PERMUTED, algo, M, N, K, K, K, 16)) {
+      continue;  // (it would run on another instance's tile)
     }
     // what other instances do better on every problem of the kind is not timed unless it is asked for: loads in dwords
     // where whole 16-byte pieces fit, the few-rows kernel for many rows

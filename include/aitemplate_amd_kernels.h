@@ -189,7 +189,8 @@ AITAMD_API int aitamd_bmm_rcr(int dtype, int algo,
  * Replaces the DeviceBatchedGemmXdl / DeviceGemm instances behind bmm_rrr, bmm_ccr, bmm_crr, gemm_rrr and
  * bmm_rrr_permute (python/aitemplate/backend/rocm/gemm/bmm_rrr.py, bmm_ccr.py, bmm_crr.py, gemm_rrr.py,
  * bmm_rrr_permute.py; layouts in backend/rocm/gemm/layout.py). */
-enum { AITAMD_LAYOUT_RCR = 0, AITAMD_LAYOUT_RRR = 1, AITAMD_LAYOUT_CCR = 2, AITAMD_LAYOUT_CRR = 3 };
+enum { AITAMD_LAYOUT_RCR = 0, AITAMD_LAYOUT_RRR = 1, AITAMD_LAYOUT_CCR = 2, AITAMD_LAYOUT_CRR = 3,
+       AITAMD_LAYOUT_RCR_PERMUTED = 4 /* for aitamd_gemm_{algo_supported,heuristic_algo}_layout only */ };
 AITAMD_API int aitamd_bmm(int layout, int dtype, int algo, const void* a, const void* b, void* c,
                           int64_t batch, int64_t M, int64_t N, int64_t K,
                           int64_t lda, int64_t ldb, int64_t ldc,
@@ -209,8 +210,9 @@ AITAMD_API int aitamd_gemm_permute(int operands, int epilogue, int dtype, int al
                                    const void* a, const void* b, const void* bias, void* c,
                                    int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                    int layout, int64_t g1, int64_t g2, int64_t g3, void* stream);
-/* aitamd_gemm_algo_supported / aitamd_gemm_heuristic_algo for a given operand layout (same arguments otherwise); layout 4
- * of the latter: rcr operands and a permuted store */
+/* aitamd_gemm_algo_supported / aitamd_gemm_heuristic_algo for a given operand layout (same arguments otherwise);
+ * AITAMD_LAYOUT_RCR_PERMUTED: rcr operands and a permuted store (an instance that would hand it to another's tile does not
+ * count as supporting it) */
 AITAMD_API int aitamd_gemm_algo_supported_layout(int epilogue, int dtype, int layout, int algo,
                                                  int64_t M, int64_t N, int64_t K,
                                                  int64_t lda, int64_t ldb, int align_bytes);

@@ -1134,3 +1134,26 @@ def test_every_linear_layer_has_the_same_instances():
         for dtype in (0, 1):
             names = [n.replace("_bf16_", "_f16_") for n in _kernels.gemm_algo_names(epilogue, dtype)]
             assert names == want, (epilogue, dtype)
+
+
+@pytest.mark.parametrize("op", ["gemm_rcr_permute_m2n3", "gemm_rcr_bias_permute_m2n3", "bmm_rcr_permute"])
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+def test_permuted_stores_are_not_given_to_the_four_wave_instances(op, dtype):
+    """Which would hand them on to a 32 x 32 tile: neither candidates to be timed nor chosen without timing."""
+    from types import SimpleNamespace
+
+    from aitemplate_amd import _kernels
+    from aitemplate_amd.backend import registry
+
+    names = _kernels.gemm_algo_names(1 if "bias" in op else 0, int(dtype == "bfloat16"))
+    dim = SimpleNamespace(_attrs={"values": [64]})
+    operand = SimpleNamespace(_attrs={"dtype": dtype, "shape": [dim, dim]})
+    attrs = {"op": op, "inputs": [operand, operand], "op_instance": {n: i for i, n in enumerate(names)}}
+    for m, n, k in ((8192, 8192, 8192), (2048, 6912, 8314), (12608, 1024, 4096), (2136, 344, 2320)):
+        key = f"{'12,' if op.startswith('bmm') else ''}{m},{n},{k}"
+        attrs["exec_path"] = {key: None}
+        align = 8 if k % 8 == 0 else 2
+        left = [name for name in names if registry.get(f"rocm.{op}.filter")(name, attrs, align)]
+        assert len(left) > 5 and not any("_wide" in name for name in left)
+        if align == 8 or not op.startswith("bmm"):
+            assert registry.get(f"rocm.{op}.select_algo")(attrs, key) in left
