@@ -28,8 +28,8 @@ def _inputs(M, N, K, nres, dtype, seed):
 @pytest.mark.parametrize("op,nres", [("gemm_rcr", 0), ("gemm_rcr_bias", 0), ("gemm_rcr_bias_gelu", 0),
                                      ("gemm_rcr_bias_add", 1), ("gemm_rcr_bias_add_add", 2)])
 @pytest.mark.parametrize("M,N,K", [
-    (256, 1024, 1024),   # the plumbing configuration: 64 tiles of 64 x 64, four workgroups each
-    (100, 200, 4096),    # ragged tiles, sixteen workgroups per tile
+    (256, 1024, 1024),   # the plumbing configuration: 64 tiles of 64 x 64
+    (100, 200, 4096),    # ragged tiles, long K
     (64, 64, 264),       # K tail in the last workgroup's share
     (300, 72, 136),      # three K-slabs: one workgroup per tile only (no partial tiles written)
     (512, 768, 3072),    # small-batch BERT down-projection
@@ -51,6 +51,41 @@ def test_splitk_matches_oracle(op, nres, M, N, K):
             torch.testing.assert_close(out.cpu().float(), want, atol=1e-2, rtol=1e-2)
         counter_bytes = min(need, 4096)
         assert int(scratch[:counter_bytes].to(torch.int32).sum()) == 0
+
+
+def _splits(name, op, algo, M, N, K):
+    """Workgroups per tile, from the scratch memory: a page of counters and an fp32 tile for each."""
+    bm, bn = (int(v) for v in name.split("_")[3].split("x")[:2])
+    need = eager.gemm_workspace_bytes(op, algo, M, N, K)
+    return (need - 4096) / (-(-M // bm) * -(-N // bn) * bm * bn * 4) if need else 1
+
+
+# the partial tiles are read two or four at a time: numbers of them with every remainder
+@pytest.mark.parametrize("part,M,N,K,splits", [
+    ("_64x64x64_", 60, 56, 768, 3), ("_64x64x64_", 1000, 72, 4096, 5), ("_64x64x64_", 50, 64, 3072, 6),
+    ("_64x64x64_", 1090, 72, 8192, 7), ("_64x64x64_", 64, 40, 4096, 8),
+    ("_128x128x64_", 100, 64, 768, 3), ("_128x128x64_", 128, 128, 1000, 4), ("_128x128x64_", 1000, 64, 4096, 5),
+    ("_128x128x64_", 64, 64, 3072, 6),
+    ("_128x128x32_", 1000, 1096, 384, 3), ("_128x128x32_", 640, 1096, 384, 5), ("_128x128x32_", 64, 64, 384, 6),
+    ("_128x128x32_", 700, 768, 512, 7)])
+def test_every_number_of_splits(part, M, N, K, splits):
+    """Whole numbers, whose sums of 32 bits are exact: every bit of the result."""
+    op = "gemm_rcr_bias"
+    algos = [(i, n) for i, n in _splitk_algos(op) if part in n]
+    assert algos, f"no split-K instance of {part}"
+    for algo, name in algos:
+        k = K + 2 if "_k2_" in name else K
+        assert _splits(name, op, algo, M, N, k) == splits, name
+        print(f"case {name} M={M} N={N} K={k} splits={splits}", flush=True)
+        g = torch.Generator().manual_seed(splits)
+        x, w, b = (torch.randint(-2, 3, s, generator=g).double() for s in ((M, k), (N, k), (N,)))
+        want = (x @ w.T + b).half()
+        scratch = eager.new_workspace(eager.gemm_workspace_bytes(op, algo, M, N, k))
+        scratch[4096:].view(torch.float32).fill_(float("nan"))
+        for rep in range(2):
+            out = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+            eager.gemm(op, x.half().cuda(), w.half().cuda(), b.half().cuda(), out=out, algo=algo, workspace=scratch)
+            assert torch.equal(out.cpu(), want), name
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 6912, 8314), (100, 200, 4102), (64, 64, 270), (48, 136, 12)])

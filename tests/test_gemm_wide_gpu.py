@@ -11,6 +11,7 @@ pytestmark = pytest.mark.gpu
 
 ALIGNED = [n for n in _kernels.gemm_algo_names(2, 0) if n.endswith("_wide")]
 DWORDS = [n for n in _kernels.gemm_algo_names(2, 0) if n.endswith("_wide_k2")]
+assert ALIGNED and DWORDS
 
 
 def _rand(shape, seed, dtype, scale=1.0):
@@ -19,7 +20,9 @@ def _rand(shape, seed, dtype, scale=1.0):
 
 def _algo(op, name, dtype):
     name = name.replace("_f16_", "_bf16_") if dtype == torch.bfloat16 else name
-    return _kernels.load().aitamd_gemm_find_algo(_kernels.EPILOGUE_OF_OP[op], int(dtype == torch.bfloat16), name.encode())
+    algo = _kernels.load().aitamd_gemm_find_algo(_kernels.EPILOGUE_OF_OP[op], int(dtype == torch.bfloat16), name.encode())
+    assert algo >= 0, f"{op} has no instance {name}"  # (-1 would be the automatic choice)
+    return algo
 
 
 def _check(op, name, M, N, K, dtype=torch.float16, pitch=0, seed=0):
