@@ -57,8 +57,8 @@ inline double split_k_exchange_us(int64_t tiles, int64_t s, int64_t tile_elems) 
 // Workgroups per tile of a split-K launch (the launcher and the instance choice share the rule): of the numbers from two
 // up to about one workgroup per CU, with at least two K-slabs each, at most 16, the one that gives the least time for a
 // workgroup's slabs and the exchange; 1 (no splitting, nothing written to the scratch memory) for grids that fill half
-// the device anyway.  (The 32-deep slabs of 128 x 128 are not among the fitted: as many as fill the CUs.)  Whether to split
-// at all is the choice of the instance.  1.5 % (64 x 64 tiles) and 2.0 %
+// the device anyway.  (The 32-deep slabs of 128 x 128 take as many as fill the CUs, a third more time than the best number: an
+// instance that is never ahead of the others, for those who name it.)  Whether to split at all is the choice of the instance.  1.5 % (64 x 64 tiles) and 2.0 %
 // (128 x 128) above the best number in the geometric mean; as many as fill the CUs, the rule before, 8 % and 21 %:
 // 21 x 512 x 2048 11.5 us with 16, 7.1 with 4; 200 x 2304 x 768 in 128 x 128 tiles 17.4 with 6, 13.1 with 2.
 inline int split_k_rule(int64_t tiles, int64_t k_tiles, int bk, int64_t tile_elems, int cus) {

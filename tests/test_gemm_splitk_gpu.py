@@ -214,3 +214,21 @@ def test_splitk_on_two_streams_with_separate_scratch_buffers():
     torch.cuda.synchronize()
     for case in cases:
         assert int(case[-1]) == 0
+
+
+@pytest.mark.parametrize("M,N,K", [(180, 6048, 7056), (1616, 640, 4752), (660, 2016, 7792)])
+def test_automatic_choice_shares_a_long_k_between_workgroups(M, N, K):
+    """64 to 128 tiles of 128 x 128 over a long K, with scratch memory: the split-K instance of 64-deep slabs is ahead of all others
+    (39 us against 48 of the next at the first).  Its bits, and partial tiles in the scratch memory, say that it was taken."""
+    op = "gemm_rcr_bias"
+    x, w, b, _ = (t.cuda() if isinstance(t, torch.Tensor) else t for t in _inputs(M, N, K, 0, torch.float16, seed=K))
+    algo = next(i for i, n in _splitk_algos(op) if "_128x128x64_" in n)
+    need = eager.gemm_workspace_bytes(op, algo, M, N, K)
+    assert need > 4096
+    named = eager.gemm(op, x, w, b, algo=algo, workspace=eager.new_workspace(need))
+    scratch = eager.new_workspace(need)
+    slots = scratch[4096:].view(torch.float32)
+    slots.fill_(float("nan"))
+    got = eager.gemm(op, x, w, b, workspace=scratch)
+    assert torch.equal(got, named) and not bool(slots.isnan().any())
+    assert int(scratch[:4096].to(torch.int32).sum()) == 0
