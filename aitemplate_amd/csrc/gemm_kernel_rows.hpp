@@ -16,8 +16,8 @@
 // 31 x 1232 x 5504 14.0 / 9.5, 41 x 158 x 3879 9.3 / 6.8.  Tiles of 16 x 32, 32 x 16 and 32 x 32: slower at all of these.
 // Groups past a wave's last are not requested - though out of range, their loads and the wait for them took 0.2 us of every launch -
 // and the loop over all groups but the last ones has nothing to cut.  Before / after, on average over 40 to 70 problems each:
-// M 5 to 16, K 65 to 128 2.97 / 2.70, K 513 to 1024 3.38 / 3.02, K above 4096 6.42 / 5.89; M to 4 at an odd K of 65 to 128 3.05 / 2.94,
-// where the register form, without a pass through LDS, took 2.77.
+// M 5 to 16, K 65 to 128 2.97 / 2.70, K 513 to 1024 3.38 / 3.02, K above 4096 6.42 / 5.89; M to 4 at an odd K of 65 to 128 3.01 / 2.95,
+// where the register form, without a pass through LDS, took 2.72.
 // Four waves with two groups each on their way, or eight with one: two workgroups fit a CU (one, with twice as much on its
 // way: as fast or up to a quarter slower).  Eight for odd elements, whose shifts a lone wave on its SIMD waits for.
 //
@@ -156,10 +156,11 @@ __global__ void __launch_bounds__(Tile::NT) gemm_rcr_rows_kernel(const GemmParam
       if (i < mine) issue(i, i * Tile::STAGE);
     read_epilogue();  // (the first wait, which counts them, takes in as many loads of the next group)
     uint32_t at = 0;
-    // MORE: group i + NS is requested as soon as group i has been read
+    // MORE: group i + NS is requested as soon as group i has been read (kAsk: if there is one)
+    constexpr int kNo = 0, kYes = 1, kAsk = 2;
     auto multiply = [&](auto more, int i) __attribute__((always_inline)) {
-      constexpr bool MORE = decltype(more)::value;
-      if (MORE || i + NS - 1 < mine)
+      constexpr int MORE = decltype(more)::value;
+      if (NS == 1 || MORE == kYes || i + NS - 1 < mine)
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * (LOADS_A + 4)) : "memory");
       else  // (fewer than NS - 1 groups behind it)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -180,7 +181,7 @@ __global__ void __launch_bounds__(Tile::NT) gemm_rcr_rows_kernel(const GemmParam
       for (int j = 0; j < 4; ++j)
 #pragma unroll
         for (int x = 0; x < 2; ++x) rows_arrived(f[x][j], behind[x][j]);
-      if constexpr (MORE) issue(i + NS, at);
+      if (MORE == kYes || (MORE == kAsk && i + NS < mine)) issue(i + NS, at);
       at = at + Tile::STAGE == NS * Tile::STAGE ? 0 : at + Tile::STAGE;
       if constexpr (ELEM != 0) {
 #pragma unroll
@@ -195,7 +196,7 @@ __global__ void __launch_bounds__(Tile::NT) gemm_rcr_rows_kernel(const GemmParam
       }
       // past the end of K: nothing of either operand
       const int g = wave + i * NW;
-      if (!MORE && g == groups - 1) {
+      if (MORE != kYes && g == groups - 1) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const int left = p.K - g * GROUP - (j * 4 + fq) * 8;
@@ -209,8 +210,13 @@ __global__ void __launch_bounds__(Tile::NT) gemm_rcr_rows_kernel(const GemmParam
       for (int j = 0; j < 4; ++j) acc = Tr::mfma16(__builtin_bit_cast(vec8, f[1][j]), __builtin_bit_cast(vec8, f[0][j]), acc);
     };
     int i = 0;
-    for (; i + NS < mine; ++i) multiply(std::true_type{}, i);
-    for (; i < mine; ++i) multiply(std::false_type{}, i);
+    // (at odd elements in one loop: the shifts bound it and not the instructions of the cut, and two loops were 4 % slower above K = 4096)
+    if constexpr (ELEM != 0) {
+      for (; i < mine; ++i) multiply(std::integral_constant<int, kAsk>{}, i);
+    } else {
+      for (; i + NS < mine; ++i) multiply(std::integral_constant<int, kYes>{}, i);
+      for (; i < mine; ++i) multiply(std::integral_constant<int, kNo>{}, i);
+    }
   };
   if (rows_a <= 4)
     multiply_all(std::integral_constant<int, 1>{});
