@@ -17,7 +17,7 @@
 // What bounds it: the board's power on operands with random bits, the latency of lines from beyond the L2 on constant
 // ones (where all come from the L2: 537 us).  A slab's loads over one K-step instead of two: 837 us against 715 (before
 // the above); one slab at a time: 870; lines touched ahead of their loads, to bring them into the L2: no gain on random
-// operands.  8192^3 bf16, normally distributed operands: 814 us (eight waves) -> 727.
+// operands.  8192^3 bf16, normally distributed operands: 813 us (eight waves) -> 721.
 //
 // The epilogue needs no LDS: v_permlane16_swap between two column blocks gives a lane 8 consecutive columns of a row,
 // in fp32.  It stores 16-byte pieces through buffer descriptors only; the launcher sends other outputs elsewhere.
