@@ -7,6 +7,13 @@
 //    fetches, so the ds_read side stays bank-conflict free.
 //  * NS slabs are resident: the slab for step k+NS-1 is issued while step k is
 //    multiplied, and one s_waitcnt vmcnt + one barrier per step orders them.
+//    The last NS-1 steps request nothing, and wait for ever fewer loads: a slab
+//    past the end of K, all of it out of range, takes as long on its way to LDS as
+//    any other (0.11 us for 16 KiB), and there were NS-1 of them in every tile's
+//    time.  us before -> now: 70 x 1024 x 256 2.93 -> 2.77, 312 x 768 x 256
+//    3.33 -> 3.08, 4096 x 4096 x 64 10.9 -> 10.2, 384 x 768 x 3072 shared along K
+//    10.1 -> 9.2; 64 x 64 x 128 and 32 x 32 x 128 tiles 6 and 7 % on average over 23
+//    problems, the others 1 to 4 %.
 //  * MT selects the MFMA: 32 -> v_mfma_f32_32x32x16, 16 -> v_mfma_f32_16x16x32.
 //  * the accumulator tile goes registers -> LDS (row-major, padded) -> registers
 //    so that each lane owns 8 consecutive output columns: bias / residual loads
@@ -293,11 +300,9 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
     const __amdgpu_buffer_rsrc_t rb = make_rsrc(reinterpret_cast<const char*>(Bb) - odd_b,
                                                 clamp_records(Tile::STAGED ? (bytes_b + odd_b + 3) & ~3ll : bytes_b));
 
-    // Issue the wave-loads of K-slab `kt` into ring slot `stage`.  Slabs past
-    // the end of K are still issued (every chunk out of range -> zero fill) so
-    // the number of loads in flight per step stays constant for s_waitcnt.
+    // Issue the wave-loads of K-slab `kt` into ring slot `stage`: only slabs of this workgroup's range.
     auto issue_loads = [&](int kt, int stage, int i0, int i1) {
-      const int k0 = (Tile::SPLITK && kt >= k_tiles) ? k_main : (k_lo + kt) * BK;  // (past the own range: nothing to fetch)
+      const int k0 = (k_lo + kt) * BK;
       T* sbase = smem + stage * Tile::STAGE_ELEMS;
 #pragma unroll
       for (int i = 0; i < L_IT; ++i) {
@@ -377,16 +382,13 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
     // the L_IT wave-loads of a slab are issued in KK equal portions, one per MFMA step
     constexpr int L_PER = (L_IT + KK - 1) / KK;
     constexpr int L_P0 = L_PER < L_IT ? L_PER : L_IT;  // size of portion 0
-    if constexpr (Tile::STAGED != 0) {
-      // (the staged loop fills its own pipeline)
-    } else if constexpr (Tile::PIPE == 0) {
+    if constexpr (Tile::STAGED == 0) {
+      // whole slabs: NS - 1, or (PIPE 1) NS - 2 and portion 0 of the next
+      constexpr int kWhole = Tile::PIPE == 0 ? NS - 1 : NS - 2;
 #pragma unroll
-      for (int s = 0; s < NS - 1; ++s) issue_loads(s, s, 0, L_IT);
-    } else {
-      // steady state at the top of slab 0: slabs 0..NS-3 whole, slab NS-2 up to portion 0
-#pragma unroll
-      for (int s = 0; s < NS - 2; ++s) issue_loads(s, s, 0, L_IT);
-      issue_loads(NS - 2, NS - 2, 0, L_P0);
+      for (int s = 0; s < kWhole; ++s)
+        if (s < k_tiles) issue_loads(s, s, 0, L_IT);
+      if (Tile::PIPE == 1 && kWhole < k_tiles) issue_loads(kWhole, kWhole, 0, L_P0);
     }
 
     auto load_frags = [&](const T* st, int kk, vec8* af, vec8* bf) {
@@ -493,9 +495,12 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
         });
       }
     } else if constexpr (Tile::PIPE == 0) {
-      for (int kt = 0; kt < k_tiles; ++kt) {
-        // slab kt has landed once at most the (NS-2) younger slabs are in flight
-        wait_vmcnt<(NS - 2) * Tile::LOADS_PER_STEP>();
+      // LEFT: slabs behind slab kt that are on their way or to come, NS - 1 standing for any number from there on
+      auto slab = [&](int kt, auto left_c) {
+        constexpr int LEFT = decltype(left_c)::value;
+        constexpr bool kFetch = LEFT >= NS - 1;
+        // slab kt has landed once at most the younger slabs, NS - 2 unless fewer are left, are in flight
+        wait_vmcnt<(kFetch ? NS - 2 : LEFT) * Tile::LOADS_PER_STEP>();
         __builtin_amdgcn_s_barrier();
         const T* cur = smem + (kt % NS) * Tile::STAGE_ELEMS;
         load_frags(cur, 0, af[0], bf[0]);
@@ -503,57 +508,69 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
         for (int kk = 0; kk < KK; ++kk) {
           const int cb = kk & 1, nb = cb ^ 1;
           const int i0 = kk * L_PER, i1 = (kk + 1) * L_PER < L_IT ? (kk + 1) * L_PER : L_IT;
-          issue_loads(kt + NS - 1, (kt + NS - 1) % NS, i0, i1);
+          if constexpr (kFetch) issue_loads(kt + NS - 1, (kt + NS - 1) % NS, i0, i1);
           if (kk + 1 < KK) load_frags(cur, kk + 1, af[nb], bf[nb]);
           mfmas(af[cb], bf[cb]);
           if (kk + 1 < KK)
-            sched_step<MI * NI, kFragReads, L_PER>();
+            sched_step<MI * NI, kFragReads, kFetch ? L_PER : 0>();
           else
-            sched_step<MI * NI, 0, L_PER>();
+            sched_step<MI * NI, 0, kFetch ? L_PER : 0>();
         }
-      }
+      };
+      int kt = 0;
+      for (; kt + NS - 1 < k_tiles; ++kt) slab(kt, std::integral_constant<int, NS - 1>{});
+      // the last NS - 1 slabs (or all, where there are fewer): nothing more is requested
+      static_for<0, NS - 1>([&](auto i) {
+        constexpr int left = NS - 2 - decltype(i)::value;
+        if (left < k_tiles) slab(k_tiles - 1 - left, std::integral_constant<int, left>{});
+      });
     } else {
-      wait_vmcnt<(NS - 3) * Tile::LOADS_PER_STEP + L_P0>();
+      static_assert(KK % 2 == 0, "the register buffers alternate inside a slab");
+      if (NS - 2 < k_tiles)
+        wait_vmcnt<(NS - 3) * Tile::LOADS_PER_STEP + L_P0>();
+      else
+        wait_vmcnt<0>();
       __builtin_amdgcn_s_barrier();
       load_frags(smem, 0, af[0], bf[0]);
-      // with a single MFMA step per slab the register buffers alternate per slab
-      constexpr int KT_UNROLL = (KK % 2 == 0) ? 1 : 2;
-      for (int kt0 = 0; kt0 < k_tiles; kt0 += KT_UNROLL) {
+      auto slab = [&](int kt, auto left_c) {
+        constexpr int LEFT = decltype(left_c)::value;  // as above
+        const T* cur = smem + (kt % NS) * Tile::STAGE_ELEMS;
 #pragma unroll
-        for (int u = 0; u < KT_UNROLL; ++u) {
-          const int kt = kt0 + u;
-          if (KT_UNROLL > 1 && kt >= k_tiles) break;
-          const T* cur = smem + (kt % NS) * Tile::STAGE_ELEMS;
-#pragma unroll
-          for (int kk = 0; kk < KK; ++kk) {
-            const int cb = (u * KK + kk) & 1, nb = cb ^ 1;
-            // portion `pi` of the slab being loaded during this period: the period
-            // starts at the barrier in a slab's last step and covers the next KK-1 steps
-            if (kk + 1 < KK) {
-              const int pi = kk + 1;
-              const int i0 = pi * L_PER, i1 = (pi + 1) * L_PER < L_IT ? (pi + 1) * L_PER : L_IT;
-              issue_loads(kt + NS - 2, (kt + NS - 2) % NS, i0, i1);
-              load_frags(cur, kk + 1, af[nb], bf[nb]);
-              mfmas(af[cb], bf[cb]);
-              sched_step<MI * NI, kFragReads, L_PER>();
-            } else {
-              // slab kt+1 has landed once at most (NS-3) younger slabs are in flight;
-              // past the barrier nobody reads slab kt-1 any more, so its ring slot
-              // starts taking slab kt+NS-1, and the next slab's first fragments are
-              // fetched under this slab's last MFMAs.
-              wait_vmcnt<(NS - 3) * Tile::LOADS_PER_STEP>();
-              __builtin_amdgcn_s_barrier();
-              const int i1 = L_P0;
-              issue_loads(kt + NS - 1, (kt + NS - 1) % NS, 0, i1);
-              load_frags(smem + ((kt + 1) % NS) * Tile::STAGE_ELEMS, 0, af[nb], bf[nb]);
-              mfmas(af[cb], bf[cb]);
-              sched_step<MI * NI, kFragReads, L_P0>();
-            }
+        for (int kk = 0; kk < KK; ++kk) {
+          const int cb = kk & 1, nb = cb ^ 1;
+          // portion `pi` of the slab being loaded during this period: the period
+          // starts at the barrier in a slab's last step and covers the next KK-1 steps
+          if (kk + 1 < KK) {
+            const int pi = kk + 1;
+            const int i0 = pi * L_PER, i1 = (pi + 1) * L_PER < L_IT ? (pi + 1) * L_PER : L_IT;
+            if constexpr (LEFT >= NS - 2) issue_loads(kt + NS - 2, (kt + NS - 2) % NS, i0, i1);
+            load_frags(cur, kk + 1, af[nb], bf[nb]);
+            mfmas(af[cb], bf[cb]);
+            sched_step<MI * NI, kFragReads, LEFT >= NS - 2 ? L_PER : 0>();
+          } else if constexpr (LEFT > 0) {
+            // slab kt+1 has landed once at most (NS-3) younger slabs are in flight;
+            // past the barrier nobody reads slab kt-1 any more, so its ring slot
+            // starts taking slab kt+NS-1, and the next slab's first fragments are
+            // fetched under this slab's last MFMAs.
+            wait_vmcnt<(LEFT >= NS - 2 ? NS - 3 : LEFT - 1) * Tile::LOADS_PER_STEP>();
+            __builtin_amdgcn_s_barrier();
+            if constexpr (LEFT >= NS - 1) issue_loads(kt + NS - 1, (kt + NS - 1) % NS, 0, L_P0);
+            load_frags(smem + ((kt + 1) % NS) * Tile::STAGE_ELEMS, 0, af[nb], bf[nb]);
+            mfmas(af[cb], bf[cb]);
+            sched_step<MI * NI, kFragReads, LEFT >= NS - 1 ? L_P0 : 0>();
+          } else {
+            mfmas(af[cb], bf[cb]);
           }
         }
-      }
+      };
+      int kt = 0;
+      for (; kt + NS - 1 < k_tiles; ++kt) slab(kt, std::integral_constant<int, NS - 1>{});
+      static_for<0, NS - 1>([&](auto i) {
+        constexpr int left = NS - 2 - decltype(i)::value;
+        if (left < k_tiles) slab(k_tiles - 1 - left, std::integral_constant<int, left>{});
+      });
     }
-    // drain the zero-fill slabs still in flight before LDS is reused
+    // every wave has read its last slab before LDS is reused
     wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
     if constexpr (Tile::KTAIL != 0) {

@@ -227,3 +227,23 @@ def test_config_c4_full_size():
     got = eager.bmm_rcr(inp["q"].cuda(), inp["k"].cuda())
     torch.cuda.synchronize()
     torch.testing.assert_close(got.cpu().float(), want, atol=ATOL, rtol=RTOL)
+
+
+@pytest.mark.parametrize("name", [n for n in _kernels.gemm_algo_names(4, 0) if "_dma" in n])
+def test_slab_counts(name):
+    """Direct-to-LDS instances request no slab past the end of K: as many slabs as fill a part of the ring, all of it, and
+    a few more, the last whole or cut."""
+    bm, bn, bk = (int(v) for v in name.split("f16_")[1].split("_")[0].split("x"))
+    M, N = bm + 9, bn + 24
+    algo = _kernels.load().aitamd_gemm_find_algo(4, 0, name.encode())
+    assert algo >= 0, name
+    for slabs in range(1, 8):
+        for cut in (0, 2) if "_k2" in name else (0, 8):
+            K = slabs * bk - cut
+            print(f"case instance={name} M={M} N={N} K={K}", flush=True)
+            x, w = _rand((M, K), torch.float16, K), _rand((N, K), torch.float16, K + 1, scale=K ** -0.5)
+            b, d = _rand((N,), torch.float16, K + 2), _rand((M, N), torch.float16, K + 3)
+            got = eager.gemm("gemm_rcr_bias_add", x.cuda(), w.cuda(), b.cuda(), d.cuda(), algo=algo)
+            want = oracle.torch_gemm("gemm_rcr_bias_add", x, w, b, d).float()
+            # one rounding of a 32-bit result, and sums of K products of N(0, 1) x N(0, 1/K) in another order
+            torch.testing.assert_close(got.cpu().float(), want, rtol=2.0 ** -10, atol=2.0 ** -10)
