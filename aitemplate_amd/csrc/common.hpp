@@ -145,53 +145,34 @@ AITAMD_DEVICE uint32_t clamp_records(int64_t bytes) {
 }
 
 // ---------------------------------------------------------------------------
-// Workgroup -> tile mapping.  The hardware deals consecutive workgroup ids
-// round-robin over the 8 XCDs; tiles that share an A row-panel or a B
-// column-panel should land on the same XCD so the panel is fetched into one
-// L2 only.  Step 1 gives every XCD a contiguous range of logical (batch, tile) ids,
-// step 2 walks the tiles of a batch in groups of kGroupM tile-rows, column by column.
+// Division by a number the host knows: the quotient by a multiplication with its scaled reciprocal (Granlund and
+// Montgomery, "Division by invariant integers using multiplication", 1994), three scalar instructions.  The compiler's own
+// division of two values in registers is a chain of 35, through the vector unit and back, and a tile's coordinates took
+// three of them ahead of its first load.
 // ---------------------------------------------------------------------------
-AITAMD_DEVICE void map_tile_grouped(int wg, int tiles_m, int tiles_n, int batch, int kGroupM, int& b, int& tm, int& tn);
-template <int kGroupM>
-AITAMD_DEVICE void map_tile(int wg, int tiles_m, int tiles_n, int batch, int& b, int& tm, int& tn) {
-  map_tile_grouped(wg, tiles_m, tiles_n, batch, kGroupM, b, tm, tn);
+struct Divisor {
+  uint32_t mul, shift;
+};
+// d of 1 to 2^31 - 1
+constexpr Divisor make_divisor(int64_t d) {
+  uint32_t shift = 0;
+  while ((1ll << shift) < d) ++shift;
+  return {(uint32_t)((((1ull << shift) - (uint64_t)d) << 32) / (uint64_t)d + 1), shift};
 }
-// (the group height as a value: the persistent kernels take it from the launcher)
-AITAMD_DEVICE void map_tile_grouped(int wg, int tiles_m, int tiles_n, int batch, int kGroupM, int& b, int& tm, int& tn) {
-  // wg runs over batch * tiles_m * tiles_n workgroups; logical ids are batch-major, so an XCD's
-  // contiguous id range is a run of whole batches (plus at most two partial ones at its ends):
-  // the tiles of one batch share its operands through one L2 and fill its output rows together.
-  const int per_batch = tiles_m * tiles_n;
-  const int total = per_batch * batch;
-  const int xcd = wg % kNumXcd;
-  const int local = wg / kNumXcd;
-  const int q = total / kNumXcd;
-  const int r = total % kNumXcd;
-  const int flat = xcd * q + (xcd < r ? xcd : r) + local;
-  b = flat / per_batch;
-  const int id = flat - b * per_batch;
-  const int group_sz = kGroupM * tiles_n;
-  const int g = id / group_sz;
-  const int first_m = g * kGroupM;
-  const int gm = (tiles_m - first_m) < kGroupM ? (tiles_m - first_m) : kGroupM;
-  const int in_group = id - g * group_sz;
-  tm = first_m + in_group % gm;
-  tn = in_group / gm;
+// n / d for n of 0 to 2^31 - 1 (mulhi(n, mul) <= n: the sum stays below 2^32)
+constexpr __host__ __device__ __forceinline__ int quotient(int n, Divisor d) {
+  const uint32_t hi = (uint32_t)(((uint64_t)(uint32_t)n * d.mul) >> 32);
+  return (int)((hi + (uint32_t)n) >> d.shift);
 }
-
-// Block form of the mapping for one batch whose tile grid divides over the XCDs as xcd_cols column blocks times
-// 8 / xcd_cols row blocks: XCD x works through its own block row by row, so the B panels of the block's few
-// columns are fetched into its L2 once and stay there for every row (the tiles that need an A panel are adjacent
-// in the walk and run at the same time).  Same workgroup -> XCD deal as above: wg % 8 is the XCD.
-AITAMD_DEVICE void map_tile_block(int wg, int tiles_m, int tiles_n, int xcd_cols, int& tm, int& tn) {
-  const int xcd = wg % kNumXcd;
-  const int local = wg / kNumXcd;
-  const int cols = tiles_n / xcd_cols;
-  const int rows = tiles_m / (kNumXcd / xcd_cols);
-  const int cb = xcd % xcd_cols, rb = xcd / xcd_cols;
-  const int r = local / cols;
-  tm = rb * rows + r;
-  tn = cb * cols + (local - r * cols);
+constexpr bool divides_right(long long d) {
+  const Divisor r = make_divisor(d);
+  for (long long q : {0ll, 1ll, 2ll, 3ll, 0x7fffffffll / d - 1, 0x7fffffffll / d})
+    for (long long n : {q * d - 1, q * d, q * d + 1, q * d + d - 1})
+      if (n >= 0 && n <= 0x7fffffffll && quotient((int)n, r) != n / d) return false;
+  return quotient(0x7fffffff, r) == 0x7fffffffll / d;
 }
+static_assert(divides_right(1) && divides_right(2) && divides_right(3) && divides_right(7) && divides_right(8) && divides_right(641) &&
+              divides_right(65535) && divides_right(65536) && divides_right(65537) && divides_right(0x3fffffff) &&
+              divides_right(0x40000000) && divides_right(0x40000001) && divides_right(0x7ffffffe) && divides_right(0x7fffffff));
 
 }  // namespace aitamd

@@ -121,6 +121,15 @@ struct IsWide<GemmTileWide<MI, NI, KTAIL>> {
   static constexpr bool value = true;
 };
 
+template <class Tile>
+struct IsRows {
+  static constexpr bool value = false;
+};
+template <int NW, int NS, int ELEM>
+struct IsRows<GemmTileRows<NW, NS, ELEM>> {
+  static constexpr bool value = true;
+};
+
 // Workgroups per tile of a split-K launch (split_k_rule)
 template <class Tile>
 int split_k_factor(const GemmParams& p, int cus) {
@@ -140,8 +149,8 @@ int64_t workspace_of(const GemmParams& p) {
   return 0;
 }
 
-// Column blocks of the per-XCD block mapping of the persistent kernels (GemmParams::xcd_cols; 0: the grouped
-// mapping).  The grid of one batch is cut into xcd_cols column blocks times 8 / xcd_cols row blocks, one per XCD,
+// The per-XCD block mapping of the persistent kernels (GemmParams::xcd_shift; -1: the grouped mapping).  The grid of
+// one batch is cut into 2^xcd_shift column blocks times 8 / 2^xcd_shift row blocks, one per XCD,
 // where it divides so and the B panels of a block's columns take at most 2.5 MiB; the fewest column blocks that fit
 // are taken, which share an A panel among the most tiles.  An XCD then reads few B panels over and over and every
 // A panel once.  Measured on M=24576 N=3072 K=768 (two column blocks of six tile columns): 158 MB fetched per launch
@@ -149,14 +158,14 @@ int64_t workspace_of(const GemmParams& p) {
 // The B panels do not stay in the 4 MiB L2 from one block row to the next all the same: a round of 32 tiles streams
 // 4.4 MB of distinct panel data between two uses of a B line (loading A with the non-temporal policy to protect B
 // loses the sharing of A among the tiles of a row: 0.159 against 0.123 ms).
-inline int xcd_column_blocks(const GemmParams& p, int bn, int grid) {
-  if (p.batch != 1 || grid % 8 != 0 || p.tiles_m <= 0 || p.tiles_n <= 0) return 0;
-  for (int a = 1; a <= 8; a *= 2) {
-    if (p.tiles_n % a != 0 || p.tiles_m % (8 / a) != 0) continue;
-    const int64_t b_bytes = (int64_t)(p.tiles_n / a) * bn * p.K * 2;
-    if (b_bytes <= (5ll << 19)) return a;
+inline int xcd_block_shift(const GemmParams& p, int64_t tiles_m, int64_t tiles_n, int bn, int64_t grid) {
+  if (p.batch != 1 || grid % 8 != 0 || tiles_m <= 0 || tiles_n <= 0) return -1;
+  for (int shift = 0; shift <= 3; ++shift) {
+    if (tiles_n % (1 << shift) != 0 || tiles_m % (8 >> shift) != 0) continue;
+    const int64_t b_bytes = (tiles_n >> shift) * bn * p.K * 2;
+    if (b_bytes <= (5ll << 19)) return shift;
   }
-  return 0;
+  return -1;
 }
 
 template <class Tile, bool PERM, int LAYOUT = 0>
@@ -184,24 +193,30 @@ hipError_t launch_kernel(const GemmParams& p_in, hipStream_t stream) {
     const long long span = p.perm_on ? (long long)p.M * p.N * 2 : ((long long)(p.M - 1) * p.ldc + p.N) * 2;
     p.nt_store = (long long)p.M * p.N * p.batch * 2 >= nt_min && span < 0x7fffffffll;
   }
-  p.tiles_m = (p.M + Tile::BM - 1) / Tile::BM;
-  p.tiles_n = (p.N + Tile::BN - 1) / Tile::BN;
-  const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-  if (tiles <= 0 || p.batch <= 0) return hipSuccess;
+  const int64_t tiles_m = ((int64_t)p.M + Tile::BM - 1) / Tile::BM, tiles_n = ((int64_t)p.N + Tile::BN - 1) / Tile::BN;
+  if (tiles_m <= 0 || tiles_n <= 0 || p.batch <= 0) return hipSuccess;
   // one workgroup per (batch, tile) pair, or, for the persistent kernels, one per CU walking them
-  const int64_t total = tiles * p.batch;
-  if (total > 0x7fffffffll) return hipErrorInvalidValue;
+  if (tiles_m * tiles_n > 0x7fffffffll / p.batch) return hipErrorInvalidValue;
+  const int64_t total = tiles_m * tiles_n * p.batch;
   dim3 grid((unsigned)total, 1, 1);
   if constexpr (IsPersistent<Tile>::value || IsWide<Tile>::value) {
     const int cus = device_cus(dev);
     grid = dim3((unsigned)(total < cus ? total : cus), 1, 1);
-    p.xcd_cols = xcd_column_blocks(p, Tile::BN, (int)grid.x);
     // few tile columns: the grouped walk goes row by row, so that the run of tiles of an XCD ends inside at most
     // one row of tiles whose A panel a second XCD then fetches too (eight rows with the default group height;
     // measured on M=24576 N=768 K=3072 and M=12608 N=1024 K=4096: 1 % less time)
     // (the four-wave tiles: groups of four rows, so that more XCDs work on the same columns at a time; 8192^3 on the
     // metric's kind of operands 712 us against 731 with eight)
-    p.group_m = p.tiles_n <= 4 ? 1 : (IsWide<Tile>::value ? 4 : 8);
+    set_tiles(p, Tile::BM, Tile::BN, tiles_n <= 4 ? 0 : (IsWide<Tile>::value ? 2 : 3),
+              xcd_block_shift(p, tiles_m, tiles_n, Tile::BN, grid.x));
+  } else {
+    set_tiles(p, Tile::BM, Tile::BN, IsRows<Tile>::value ? 0 : 3, -1);
+  }
+  if constexpr (PERM) {
+    p.by_perm_m1 = make_divisor(p.perm_m1);
+    p.by_perm_m2 = make_divisor(p.perm_m2);
+    p.by_perm_n1 = make_divisor(p.perm_n1);
+    p.by_perm_n2 = make_divisor(p.perm_n2);
   }
   if constexpr (IsSplitK<Tile>::value) {
     // tiles are shared along K only with enough scratch memory to hold the partial tiles; without it the

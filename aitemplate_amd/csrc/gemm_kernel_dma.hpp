@@ -207,12 +207,13 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
   const int fr = lane % MT;  // row of the MFMA operand / column of the transposed result
   const int fq = lane / MT;  // which 8-wide k chunk of the MFMA step this lane feeds
 
+  fetch_arguments(p);
   // split-K: the workgroups of one split form one full grid of tiles (split s = workgroups [s * tiles, (s + 1) * tiles))
   const int grid_tiles = p.tiles_m * p.tiles_n * p.batch;
   const int split = Tile::SPLITK ? (int)blockIdx.x / grid_tiles : 0;
   const int tile_wg = Tile::SPLITK ? (int)blockIdx.x - split * grid_tiles : (int)blockIdx.x;
   int batch, tm, tn;
-  map_tile<8>(tile_wg, p.tiles_m, p.tiles_n, p.batch, batch, tm, tn);
+  map_tile(p, tile_wg, batch, tm, tn);
   const int m0 = tm * BM;
   const int n0 = tn * BN;
   const int rows_a = (p.M - m0) < BM ? (p.M - m0) : BM;
@@ -232,20 +233,20 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
     const int j = wave + i * Tile::NW;
     // (with A_LOADS a multiple of the wave count, whether load i fetches A or B is the same for every wave)
     const bool is_a = Tile::A_LOADS % Tile::NW == 0 ? i * Tile::NW < Tile::A_LOADS : j < Tile::A_LOADS;
-    const int64_t ld = is_a ? p.lda : p.ldb;
+    const uint32_t ld = (uint32_t)(is_a ? p.lda : p.ldb);
     if ((is_a && A_T) || (!is_a && B_T)) {
       // 1 KiB of the operand's slab = 512 / BX whole k-rows of BX elements
       const int bx = is_a ? BM : BN;
       const int cpr = bx / 8;
       const int k_row = (is_a ? j : j - Tile::A_LOADS) * (512 / bx) + lane / cpr;
       const int chunk = (lane % cpr) ^ (2 * (k_row & 3));
-      l_off[i] = (uint32_t)(((int64_t)k_row * ld + chunk * 8) * 2);
+      l_off[i] = ((uint32_t)k_row * ld + (uint32_t)chunk * 8u) * 2u;
       l_chunk_k[i] = k_row;
-      l_kbytes[i] = (uint32_t)(ld * 2);
+      l_kbytes[i] = ld * 2u;
     } else {
       const int row = (is_a ? j : j - Tile::A_LOADS) * Tile::ROWS_PER_LOAD + l_row;
       const int chunk = l_slot ^ ((row / Tile::RPW) % Tile::CPR);
-      l_off[i] = (uint32_t)(((int64_t)row * ld + chunk * 8) * 2);
+      l_off[i] = ((uint32_t)row * ld + (uint32_t)chunk * 8u) * 2u;
       l_chunk_k[i] = chunk * 8;
       l_kbytes[i] = 2;
     }
@@ -288,17 +289,23 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
 
   {
     // a transposed operand starts at its first column of the tile and ends with the tile's columns of row K-1
-    const T* Ab = reinterpret_cast<const T*>(p.a) + (int64_t)batch * p.sa + (A_T ? (int64_t)m0 : (int64_t)m0 * p.lda);
-    const T* Bb = reinterpret_cast<const T*>(p.b) + (int64_t)batch * p.sb + (B_T ? (int64_t)n0 : (int64_t)n0 * p.ldb);
-    const int64_t bytes_a = A_T ? (((int64_t)p.K - 1) * p.lda + rows_a) * 2 : (((int64_t)rows_a - 1) * p.lda + p.K) * 2;
-    const int64_t bytes_b = B_T ? (((int64_t)p.K - 1) * p.ldb + rows_b) * 2 : (((int64_t)rows_b - 1) * p.ldb + p.K) * 2;
+    const T* Ab = reinterpret_cast<const T*>(p.a) + (A_T ? (int64_t)m0 : (int64_t)m0 * p.lda);
+    const T* Bb = reinterpret_cast<const T*>(p.b) + (B_T ? (int64_t)n0 : (int64_t)n0 * p.ldb);
+    if (p.batch > 1) {
+      Ab += (int64_t)batch * p.sa;
+      Bb += (int64_t)batch * p.sb;
+    }
+    // (less than 2 GiB each: algo_supported; no rows of K at all where K is 0)
+    const uint32_t lda = (uint32_t)p.lda, ldb = (uint32_t)p.ldb, k_rows = p.K > 0 ? (uint32_t)p.K - 1u : 0u;
+    const uint32_t bytes_a = (A_T ? k_rows * lda + (uint32_t)rows_a : ((uint32_t)rows_a - 1u) * lda + (uint32_t)p.K) * 2u;
+    const uint32_t bytes_b = (B_T ? k_rows * ldb + (uint32_t)rows_b : ((uint32_t)rows_b - 1u) * ldb + (uint32_t)p.K) * 2u;
     // (staged: descriptors start at a dword and end with one, so that no element of an operand at an odd place is cut off)
     const uint32_t odd_a = Tile::STAGED ? (uint32_t)(reinterpret_cast<uintptr_t>(Ab) & 3) : 0u;
     const uint32_t odd_b = Tile::STAGED ? (uint32_t)(reinterpret_cast<uintptr_t>(Bb) & 3) : 0u;
-    const __amdgpu_buffer_rsrc_t ra = make_rsrc(reinterpret_cast<const char*>(Ab) - odd_a,
-                                                clamp_records(Tile::STAGED ? (bytes_a + odd_a + 3) & ~3ll : bytes_a));
-    const __amdgpu_buffer_rsrc_t rb = make_rsrc(reinterpret_cast<const char*>(Bb) - odd_b,
-                                                clamp_records(Tile::STAGED ? (bytes_b + odd_b + 3) & ~3ll : bytes_b));
+    const __amdgpu_buffer_rsrc_t ra =
+        make_rsrc(reinterpret_cast<const char*>(Ab) - odd_a, Tile::STAGED ? (bytes_a + odd_a + 3u) & ~3u : bytes_a);
+    const __amdgpu_buffer_rsrc_t rb =
+        make_rsrc(reinterpret_cast<const char*>(Bb) - odd_b, Tile::STAGED ? (bytes_b + odd_b + 3u) & ~3u : bytes_b);
 
     // Issue the wave-loads of K-slab `kt` into ring slot `stage`: only slabs of this workgroup's range.
     auto issue_loads = [&](int kt, int stage, int i0, int i1) {

@@ -192,12 +192,7 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_persist_kernel(const Gem
     int b, tm, tn;
     const bool half = split && i == full_rounds;
     const int vwg = half ? full_rounds * G + split_tile : g + i * G;
-    if (p.xcd_cols > 0) {
-      b = 0;
-      map_tile_block(vwg, p.tiles_m, p.tiles_n, p.xcd_cols, tm, tn);
-    } else {
-      map_tile_grouped(vwg, p.tiles_m, p.tiles_n, p.batch, p.group_m > 0 ? p.group_m : 8, b, tm, tn);
-    }
+    map_tile<true>(p, vwg, b, tm, tn);
     c.m0 = tm * BM + (half ? split_half * (BM / 2) : 0);
     c.n0 = tn * BN;
     c.batch = b;

@@ -68,14 +68,11 @@ __global__ void __launch_bounds__(Tile::NT) gemm_rcr_rows_kernel(const GemmParam
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fq = lane >> 4;
-  // (a division is a tenth of a microsecond of a launch that takes three)
-  int batch = 0, id = (int)blockIdx.x, tm = 0;
-  if (p.batch > 1) {
-    const int per_batch = p.tiles_m * p.tiles_n;
-    batch = id / per_batch;
-    id -= batch * per_batch;
-  }
-  if (p.tiles_m > 1) tm = id / p.tiles_n;
+  fetch_arguments(p);
+  // tiles in rows: by_group divides by tiles_n
+  const int batch = p.batch > 1 ? quotient((int)blockIdx.x, p.by_batch) : 0;
+  const int id = (int)blockIdx.x - batch * (p.tiles_m * p.tiles_n);
+  const int tm = quotient(id, p.by_group);
   const int m0 = tm * BM, n0 = (id - tm * p.tiles_n) * BN;
   const int rows_a = (p.M - m0) < BM ? (p.M - m0) : BM;
   const int rows_b = (p.N - n0) < BN ? (p.N - n0) : BN;

@@ -119,12 +119,7 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_wide_kernel(const GemmPa
   auto tile_coord = [&](int i) __attribute__((always_inline)) {
     TileCoord c;
     int b, tm, tn;
-    if (p.xcd_cols > 0) {
-      b = 0;
-      map_tile_block(g + i * G, p.tiles_m, p.tiles_n, p.xcd_cols, tm, tn);
-    } else {
-      map_tile_grouped(g + i * G, p.tiles_m, p.tiles_n, p.batch, p.group_m > 0 ? p.group_m : 8, b, tm, tn);
-    }
+    map_tile<true>(p, g + i * G, b, tm, tn);
     c.m0 = tm * BM;
     c.n0 = tn * BN;
     c.batch = b;
