@@ -59,15 +59,21 @@ struct LdsOptIn {
 };
 
 template <class T, int KS, int OT, int FORM>
-hipError_t launch_pipe(const AttnParams& p, hipStream_t stream) {
+hipError_t launch_pipe(const AttnParams& p_in, hipStream_t stream) {
   using Tile = typename PipeOf<KS, OT, FORM>::type;
   auto kernel = attention_pipe_kernel<T, Tile>;
   static LdsOptIn opt_in;
   const hipError_t e = opt_in(reinterpret_cast<const void*>(kernel), Tile::kLdsBytes);
   if (e != hipSuccess) return e;
-  int64_t m_tiles = (p.M + Tile::BM - 1) / Tile::BM;
+  AttnParams p = p_in;
+  int64_t m_tiles = ((int64_t)p.M + Tile::BM - 1) / Tile::BM;
   if (p.paired) m_tiles = (m_tiles + 1) / 2;
-  dim3 grid((unsigned)m_tiles, (unsigned)(p.B < 65535 ? p.B : 65535), 1);
+  p.tiles = (int32_t)m_tiles;
+  p.entries = p.B < 65535 ? p.B : 65535;
+  p.dealt = p.entries == p.B && m_tiles * p.B <= 0x7fffffffll;
+  p.by_tiles = make_divisor(m_tiles);
+  p.by_heads = make_divisor(p.G);
+  dim3 grid((unsigned)p.tiles, (unsigned)p.entries, 1);
   hipLaunchKernelGGL(kernel, grid, dim3(Tile::NT), Tile::kLdsBytes, stream, p);
   return hipGetLastError();
 }

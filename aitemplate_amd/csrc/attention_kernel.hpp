@@ -52,6 +52,10 @@ struct AttnParams {
   int32_t nan_reset;
   // Non-zero (causal): the grid has half the query tiles, and a workgroup takes the i-th from the end and then the i-th.
   int32_t paired;
+  // Set by the launcher of the pipelined kernel: the grid's extents (query tiles, batch entries), whether the entries are
+  // dealt round the XCDs (a workgroup for every entry, fewer than 2^31), and the reciprocals of the tiles and of G.
+  int32_t tiles, entries, dealt;
+  Divisor by_tiles, by_heads;
 };
 
 // NW waves (32 query rows each) share the K / V tiles in two LDS stages

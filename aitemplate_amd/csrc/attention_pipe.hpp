@@ -22,9 +22,14 @@
 //   4 x 8 x 4096^2, d 80           229 -> 212    2 x 16 x 4096^2, d 128, bf16, causal   176 -> 142
 //   2 x 8 x 1024^2, d 160           43 -> 31     64 x 12 x 384^2, d 64, mixed lengths    45 -> 40
 //   and short calls (a few heads of up to 128 keys), that a launch and one tile's latency bound: 7 to 13 -> 4 to 8.
+// What comes ahead of the first tile counts for those: 345 instructions and four trips to memory one after the other
+// (arguments, grid, lengths, Q) until coordinates came without divisions and Q was asked for ahead of the lengths, 227 and
+// two: 768 x 64^2 with lengths 7.8 -> 7.3, 88 x 195^2 at d 128 10.3 -> 9.9, 144 x 41^2 4.2 -> 4.0, 16 x 200^2 4.9 -> 4.7.
 // Tried and not kept: the scores one tile further ahead (S twice in registers: slower at every head dim), one more
-// stage in both rings (nothing), three or four workgroups per CU at head dim 80 and above (spills), 8 waves on one
-// K / V tile (head dim 80 5 % faster, 128 even, 64 slower).
+// stage in both rings (nothing), no tile asked for past the last (a branch in the loop: 2 % slower), row sums by a 4x4x4
+// matrix instruction (3 % slower; no sums at all are 2 % faster), K fragments read a tile ahead (even, spills at 128), three
+// or four workgroups per CU at head dim 80 and above (spills), 8 waves on one K / V tile (head dim 80 5 % faster, 128
+// even, 64 slower).
 #pragma once
 
 #include "attention_kernel.hpp"
@@ -78,19 +83,22 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) attention_pipe_kernel(con
   // 8 XCDs, each with its own L2; XCD x works through the batch entries x, x + 8, x + 16, ... one after the other, so
   // the workgroups that stream the same K / V share one L2 and long and short sequences are spread over the XCDs.  The
   // up to seven entries that are left over go round the XCDs tile by tile.  Causal: the longest rows first.
+  // (the arguments with one wait and coordinates without divisions: see fetch_arguments and Divisor)
+  asm volatile("" ::"s"(p.q), "s"(p.k), "s"(p.v), "s"(p.B), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.O), "s"(p.G), "s"(p.causal), "s"(p.kv_len),
+               "s"(p.q_len), "s"(p.tiles), "s"(p.dealt), "s"(p.by_tiles.mul), "s"(p.by_tiles.shift), "s"(p.by_heads.mul), "s"(p.by_heads.shift));
   int bx = blockIdx.x, by = blockIdx.y;
-  if ((int)gridDim.y == p.B) {
-    const int id = blockIdx.x + gridDim.x * blockIdx.y;
-    const int tiles = gridDim.x, even = p.B & ~(kNumXcd - 1);
-    if (id < even * tiles) {
-      const int slot = id / kNumXcd, entry = slot / tiles;
-      by = entry * kNumXcd + id % kNumXcd;
-      bx = slot - entry * tiles;
+  if (p.dealt) {
+    const int id = bx + p.tiles * by;
+    const int even = p.B & ~(kNumXcd - 1);
+    if (id < even * p.tiles) {
+      const int slot = (int)((uint32_t)id / kNumXcd), entry = quotient(slot, p.by_tiles);
+      by = entry * kNumXcd + (int)((uint32_t)id % kNumXcd);
+      bx = slot - entry * p.tiles;
     }
-    if (p.causal) bx = tiles - 1 - bx;
+    if (p.causal) bx = p.tiles - 1 - bx;
   }
   const int m_tiles = (p.M + Tile::BM - 1) / Tile::BM;
-  const int first_tile = p.paired ? m_tiles - 1 - ((int)gridDim.x - 1 - bx) : bx;
+  const int first_tile = p.paired ? m_tiles - 1 - (p.tiles - 1 - bx) : bx;
   const int passes = p.paired && 2 * first_tile != m_tiles - 1 ? 2 : 1;
 
   // lane offsets of the tile loads: load i of a wave fills 1 KiB block wave_all + NWT * i of the K (V) stage
@@ -119,17 +127,38 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) attention_pipe_kernel(con
   const float c = fmaxf(__builtin_fabsf(p.scale_log2e), 1e-37f);
   const uint32_t flip = p.scale_log2e < 0.0f ? 0x80008000u : 0u;  // a negative scale changes sides: (-Q) K^T, exact
 
-  for (int b = by, pass = 0; b < p.B; pass = pass + 1 < passes ? pass + 1 : 0, b += pass == 0 ? gridDim.y : 0) {
+  for (int b = by, pass = 0; b < p.B; pass = pass + 1 < passes ? pass + 1 : 0, b += pass == 0 ? p.entries : 0) {
     const int m0 = (pass == 0 ? first_tile : m_tiles - 1 - first_tile) * Tile::BM;
     const int w0 = m0 + wave * 32 * QB;  // first row of this wave
+    // Q fragments (B operand of S^T = K Q^T): lane (q = r32, k = 16 ks + 8 h + j).  Asked for first: nothing about them
+    // depends on the entry's lengths, which are a trip to memory of their own.
+    u32x4 raw[QB][KS];
+    {
+      const int rows = p.M - m0 < Tile::BM ? p.M - m0 : Tile::BM;
+      const __amdgpu_buffer_rsrc_t rq = make_rsrc(
+          reinterpret_cast<const T*>(p.q) + ((int64_t)b * p.M + m0) * p.K, rows > 0 ? (uint32_t)(rows * p.K * 2) : 0u);
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const int k0 = ks * 16 + h * 8;
+          raw[qb][ks] = buffer_load_16B(rq, k0 < p.K ? (uint32_t)((((wave * QB + qb) * 32 + r32) * p.K + k0) * 2) : kOobOffset);
+        }
+    }
+    const int seq = quotient(b, p.by_heads);
+    // (through the scalar cache: nothing writes them while this runs)
+    auto lengths = [&](const int32_t* of) __attribute__((always_inline)) {
+      typedef const __attribute__((address_space(4))) int32_t* scalar_ptr;
+      return __builtin_amdgcn_readfirstlane(((scalar_ptr)(uintptr_t)of)[seq]);
+    };
     int N = p.N;
     if (p.kv_len != nullptr) {
-      const int len = __builtin_amdgcn_readfirstlane(p.kv_len[b / p.G]);
+      const int len = lengths(p.kv_len);
       N = len < 0 ? 0 : (len < N ? len : N);
     }
     int m_rows = p.M;
     if (p.q_len != nullptr) {
-      const int len = __builtin_amdgcn_readfirstlane(p.q_len[b / p.G]);
+      const int len = lengths(p.q_len);
       m_rows = len < 0 ? 0 : (len < m_rows ? len : m_rows);
       if (m0 >= m_rows) N = 0;  // nothing but padding rows here: no keys, zeros out
     }
@@ -166,34 +195,20 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) attention_pipe_kernel(con
       k_in = k_in + 1 == NK ? 0 : k_in + 1;
       v_in = v_in + 1 == NV ? 0 : v_in + 1;
     };
-    // Q fragments (B operand of S^T = K Q^T): lane (q = r32, k = 16 ks + 8 h + j)
-    vec8 qf[QB][KS];
-    {
-      const int rows = p.M - m0 < Tile::BM ? p.M - m0 : Tile::BM;
-      const __amdgpu_buffer_rsrc_t rq = make_rsrc(
-          reinterpret_cast<const T*>(p.q) + ((int64_t)b * p.M + m0) * p.K, rows > 0 ? (uint32_t)(rows * p.K * 2) : 0u);
-      u32x4 raw[QB][KS];
+    if (n_tiles > 0) {
 #pragma unroll
-      for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const int k0 = ks * 16 + h * 8;
-          raw[qb][ks] = buffer_load_16B(rq, k0 < p.K ? (uint32_t)((((wave * QB + qb) * 32 + r32) * p.K + k0) * 2) : kOobOffset);
-        }
-      if (n_tiles > 0) {
-#pragma unroll
-        for (int t = 0; t < D; ++t) issue(t);
-      }
-      // (used here, so that Q is waited for ahead of the loop and the tiles behind it are not)
-#pragma unroll
-      for (int qb = 0; qb < QB; ++qb)
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-#pragma unroll
-          for (int d = 0; d < 4; ++d) raw[qb][ks][d] ^= flip;
-          qf[qb][ks] = __builtin_bit_cast(vec8, raw[qb][ks]);
-        }
+      for (int t = 0; t < D; ++t) issue(t);
     }
+    // (used here, so that Q is waited for ahead of the loop and the tiles behind it are not)
+    vec8 qf[QB][KS];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) raw[qb][ks][d] ^= flip;
+        qf[qb][ks] = __builtin_bit_cast(vec8, raw[qb][ks]);
+      }
 
     f32x16 oacc[QB][OT];
     float m_run[QB], l_run[QB];
@@ -394,7 +409,7 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) attention_pipe_kernel(con
     // 16-byte pieces instead of 8 bytes of 64 rows at a time
     if (grp == 0) {
       T* const strip = reinterpret_cast<T*>(smem_raw) + wave * 32 * Tile::O_PITCH;
-      T* const ob = reinterpret_cast<T*>(p.out) + ((int64_t)(b / p.G) * p.M * p.G + b % p.G) * p.O;
+      T* const ob = reinterpret_cast<T*>(p.out) + ((int64_t)seq * p.M * p.G + (b - seq * p.G)) * p.O;
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
         const int q_row = w0 + qb * 32 + r32;
@@ -425,7 +440,7 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) attention_pipe_kernel(con
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
     }
-    if (passes > 1 || (int)gridDim.y < p.B) __syncthreads();  // the strips lie where the next tiles land
+    if (passes > 1 || p.entries < p.B) __syncthreads();  // the strips lie where the next tiles land
   }
 }
 
