@@ -247,3 +247,26 @@ def test_slab_counts(name):
             want = oracle.torch_gemm("gemm_rcr_bias_add", x, w, b, d).float()
             # one rounding of a 32-bit result, and sums of K products of N(0, 1) x N(0, 1/K) in another order
             torch.testing.assert_close(got.cpu().float(), want, rtol=2.0 ** -10, atol=2.0 ** -10)
+
+
+def _many_wave_names():
+    return [n for n in _kernels.gemm_algo_names(4, 0) if any(t in n for t in ("_w4x4_", "_96x64x", "_128x64x", "_64x128x", "_32x64x"))]
+
+
+@pytest.mark.parametrize("name", _many_wave_names())
+def test_edges_of_the_tiles(name):
+    """Instances whose waves own parts of 16 or 32 rows: a row and a column less than a tile, exactly one, one more, and
+    rows and columns that end inside the first and the last wave's part; K ending inside a slab, odd where the instance
+    takes any."""
+    bm, bn, bk = (int(v) for v in name.split("f16_")[1].split("_")[0].split("x"))
+    algo = _kernels.load().aitamd_gemm_find_algo(4, 0, name.encode())
+    assert algo >= 0, name
+    K = 3 * bk + (5 if name.endswith("_v1") else 6 if "_k2" in name else 8)
+    for M, N in ((bm - 1, bn - 1), (bm, bn), (bm + 1, bn + 1), (1, 7), (bm - 17, 2 * bn - 9)):
+        print(f"case instance={name} M={M} N={N} K={K}", flush=True)
+        x, w = _rand((M, K), torch.float16, M), _rand((N, K), torch.float16, N + 1, scale=K ** -0.5)
+        b, d = _rand((N,), torch.float16, K + 2), _rand((M, N), torch.float16, K + 3)
+        got = eager.gemm("gemm_rcr_bias_add", x.cuda(), w.cuda(), b.cuda(), d.cuda(), algo=algo)
+        want = oracle.torch_gemm("gemm_rcr_bias_add", x, w, b, d).float()
+        # one rounding of a 32-bit result, and sums of K products of N(0, 1) x N(0, 1/K) in another order
+        torch.testing.assert_close(got.cpu().float(), want, rtol=2.0 ** -10, atol=2.0 ** -10)
