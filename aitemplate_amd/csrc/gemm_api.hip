@@ -73,9 +73,9 @@ int split_factor(const GemmAlgo& a, int64_t batch, int64_t M, int64_t N, int64_t
 // Work is dealt in rounds of (CUs x workgroups per CU) tiles.  A CU with n workgroups takes n times an instance's
 // slab time for a slab of each, but no less than the slab takes a workgroup that is alone there (it is then waiting
 // for memory); a tile adds its fill and its epilogue.  The time that memory takes for the operands and the result goes on
-// beside that: the longer of the two counts, and three tenths of the shorter.  Over 500 linear layers of halves with a bias
-// (M 1 to 24576, N and K 64 to 8400, a third of them ragged) the choice is 1.5 % slower than the best instance on average, at 22 of
-// them more than 10 %; the differences between runs of a launch of a few us are a good part of that.
+// beside that: the longer of the two counts, and three tenths of the shorter.  Over 2100 linear layers and batched
+// products of halves (gemm_tiles.inc) the choice is 1.3 % slower than the best instance on average, at 104 of them more than
+// 10 %; the differences between runs of a launch of a few us are a good part of that.
 int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
               int align_bytes, int layout = 0, bool has_workspace = false, bool plain_store = true) {
   int best = -1;

@@ -245,6 +245,9 @@ int profile_gemm_like(const std::string& op, int dtype, int64_t B, int64_t M, in
                               scratch, (int64_t)scratch_bytes, stream);
   };
 
+  int dev = 0, cus = 0;
+  HIP_OK(hipGetDevice(&dev));
+  HIP_OK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   int printed = 0;
   for (int algo = 0; algo < n_algos; ++algo) {
     const char* name = aitamd_gemm_algo_name(epi, dtype, algo);
@@ -261,8 +264,14 @@ int profile_gemm_like(const std::string& op, int dtype, int64_t B, int64_t M, in
       continue;  // (it would run on another instance's tile)
     }
     // what other instances do better on every problem of the kind is not timed unless it is asked for: loads in dwords
-    // where whole 16-byte pieces fit, the few-rows kernel for many rows
+    // where whole 16-byte pieces fit, the few-rows kernel for many rows, tiles of 192 x 128 and up that are fewer than a
+    // sixth of the CUs (never less than 1.39 times the best instance's time over 1240 problems)
     if (!(only && *only)) {
+      int bm = 0, bn = 0;
+      const char* size = strstr(name, "f16_");
+      if (size != nullptr && sscanf(size + 4, "%dx%d", &bm, &bn) == 2 && bm * bn >= 192 * 128 &&
+          ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * B < cus / 6)
+        continue;
       if (K % 8 == 0 && strstr(name, "_k2") && !strstr(name, "_rows")) continue;
       if (M > 64 && strstr(name, "_rows")) continue;
     }
