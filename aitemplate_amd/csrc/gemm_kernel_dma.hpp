@@ -307,6 +307,14 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
     const __amdgpu_buffer_rsrc_t rb =
         make_rsrc(reinterpret_cast<const char*>(Bb) - odd_b, Tile::STAGED ? (bytes_b + odd_b + 3u) & ~3u : bytes_b);
 
+    // One block per matrix instruction step, one wave per SIMD, operands that are gathered: a slab is the chain of its reads and
+    // its four (eight) instructions, and whatever stands in between shows.  A step's load and the next one's reads go ahead of
+    // its instruction, in one basic block: the compiler makes a branch of a choice that a multiplication can be put behind, so
+    // the out-of-range bit is set instead of one of two offsets taken.  24 x 64 x 64 x K rrr / ccr / crr, us, instruction first and
+    // with the branches -> now: 64 x 64 x 64, K 1024 6.32 / 6.27 / 6.10 -> 5.83 / 5.73 / 5.60; 64 x 64 x 128, K 2048 9.31 / 8.87 /
+    // 8.58 -> 8.42 / 8.30 / 8.19; full grids even.  On eight waves and more it is within 4 % on either side: as it was there.
+    constexpr bool kLoadsFirst = LAYOUT != 0 && Tile::PIPE == 0 && MI * NI == 1 && Tile::NW == 4;
+
     // Issue the wave-loads of K-slab `kt` into ring slot `stage`: only slabs of this workgroup's range.
     auto issue_loads = [&](int kt, int stage, int i0, int i1) {
       const int k0 = (k_lo + kt) * BK;
@@ -316,7 +324,8 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
         if (i < i0 || i >= i1) continue;
         const int j = wave + i * Tile::NW;
         const uint32_t step = (A_T || B_T) ? (uint32_t)k0 * l_kbytes[i] : (uint32_t)(k0 * 2);
-        const uint32_t off = (k0 + l_chunk_k[i] < k_main) ? l_off[i] + step : kOobOffset;
+        const bool in_k = k0 + l_chunk_k[i] < k_main;
+        const uint32_t off = kLoadsFirst ? (l_off[i] + step) | (in_k ? 0u : kOobOffset) : (in_k ? l_off[i] + step : kOobOffset);
         T* dst = sbase + j * 512;  // 1 KiB = 512 elements per wave-load; A blocks then B blocks
         const bool is_a = Tile::A_LOADS % Tile::NW == 0 ? i * Tile::NW < Tile::A_LOADS : j < Tile::A_LOADS;
         if (is_a)
@@ -518,10 +527,16 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) gemm_rcr_dma_kernel(const
           if constexpr (kFetch) issue_loads(kt + NS - 1, (kt + NS - 1) % NS, i0, i1);
           if (kk + 1 < KK) load_frags(cur, kk + 1, af[nb], bf[nb]);
           mfmas(af[cb], bf[cb]);
-          if (kk + 1 < KK)
+          if constexpr (kLoadsFirst) {
+            if (kk == 0) __builtin_amdgcn_sched_group_barrier(0x100, kFragReads, 0);
+            if constexpr (kFetch) __builtin_amdgcn_sched_group_barrier(0x020, L_PER, 0);
+            if (kk + 1 < KK) __builtin_amdgcn_sched_group_barrier(0x100, kFragReads, 0);
+            sched_mfma<1>();
+          } else if (kk + 1 < KK) {
             sched_step<MI * NI, kFragReads, kFetch ? L_PER : 0>();
-          else
+          } else {
             sched_step<MI * NI, 0, kFetch ? L_PER : 0>();
+          }
         }
       };
       int kt = 0;
