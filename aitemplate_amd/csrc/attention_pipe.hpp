@@ -146,10 +146,15 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) attention_pipe_kernel(con
         }
     }
     const int seq = quotient(b, p.by_heads);
-    // (through the scalar cache: nothing writes them while this runs)
+    // Through the scalar cache: nothing writes them while this runs.  A scalar load takes an address without its low two
+    // bits, and the lengths may lie at any byte: the dwords of the first and the last byte of one, which are the same where
+    // it is whole.  (Behind the asm, so that nothing of the address is held in registers from one entry to the next.)
     auto lengths = [&](const int32_t* of) __attribute__((always_inline)) {
-      typedef const __attribute__((address_space(4))) int32_t* scalar_ptr;
-      return __builtin_amdgcn_readfirstlane(((scalar_ptr)(uintptr_t)of)[seq]);
+      typedef const __attribute__((address_space(4))) uint32_t* scalar_ptr;
+      uintptr_t at = reinterpret_cast<uintptr_t>(of) + 4 * (uintptr_t)(uint32_t)seq;
+      asm("" : "+s"(at));
+      const uint64_t lo = *(scalar_ptr)(at & ~(uintptr_t)3), hi = *(scalar_ptr)((at + 3) & ~(uintptr_t)3);
+      return __builtin_amdgcn_readfirstlane((int)((hi << 32 | lo) >> (8 * (at & 3))));
     };
     int N = p.N;
     if (p.kv_len != nullptr) {

@@ -3,7 +3,7 @@ Tolerance atol = rtol = 2e-2 (softmax path, fp16 out / fp32 accumulate)."""
 import pytest
 import torch
 
-from aitemplate_amd import eager
+from aitemplate_amd import _kernels, eager
 from oracle import oracle
 
 pytestmark = pytest.mark.gpu
@@ -198,6 +198,34 @@ def test_mem_eff_attention_query_lengths(attn_variant, mode, causal):
         attn_variant(mode)
     _check_mem_eff(5, 2, 700, 640, 40, 40, [640, 300, 640, 1, 640], causal=causal, seed=mode or 9,
                    lens_q=[700, 130, 0, 257, 9000])
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("d", [40, 36])   # 36: the form for unaligned operands
+def test_lengths_at_any_byte(attn_variant, mode, d):
+    """The C entry takes lengths at any address: the bits of the result are those of lengths at a whole dword."""
+    attn_variant(mode)
+    batch, heads, S, Skv = 5, 2, 300, 1000
+    q, k, v = (_rand((batch, heads, n, d), torch.float16, n + i).cuda() for i, n in enumerate((S, Skv, Skv)))
+    values = {"kv": [1000, 259, 0, 515, 77], "q": [300, 257, 300, 1, 256]}   # (several bytes of each count)
+
+    def run(off):
+        print(f"case lengths mode={mode} d={d} {off} bytes behind a dword", flush=True)
+        lengths = {}
+        for name, of in values.items():
+            lengths[name] = torch.zeros(4 * batch + 4, dtype=torch.uint8)
+            lengths[name][off:off + 4 * batch] = torch.tensor(of, dtype=torch.int32).view(torch.uint8)
+            lengths[name] = lengths[name].cuda()
+        out = torch.full((batch, S, heads, d), 3.0, dtype=torch.float16, device="cuda")
+        rc = _kernels.load().aitamd_mem_eff_attention(
+            0, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), batch, heads, S, Skv, d, d, d ** -0.5, 0,
+            lengths["kv"].data_ptr() + off, lengths["q"].data_ptr() + off, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0
+        return out.cpu()
+
+    want = run(0)
+    for off in (1, 2, 3):
+        assert torch.equal(run(off), want)
 
 
 def test_mem_eff_attention_argument_checks():
