@@ -187,7 +187,7 @@ int attention_entry(const char* who, int dtype, const void* q, const void* k, co
   p.B = (int32_t)B;
   p.M = (int32_t)M;
   p.N = (int32_t)N;
-  p.K = (int32_t)K;
+  p.K = N > 0 ? (int32_t)K : 0;  // (no keys: q, which may be null then, is not read)
   p.O = (int32_t)O;
   p.G = (int32_t)G;
   // the reference hands alpha to its kernel in the element type

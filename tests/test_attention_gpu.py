@@ -142,6 +142,17 @@ def test_empty_keys_give_zero_and_empty_batch_is_noop():
         eager.bmm_softmax_bmm_permute(q, k, v, (3,))  # batch 2 is not a multiple of 3 heads
 
 
+@pytest.mark.parametrize("K,O", [(64, 64), (40, 40), (20, 12)])   # (20, 12): the form for unaligned operands
+def test_no_keys_and_no_operands(K, O):
+    """Without keys the C entry takes null operands: the result is zeros, and nothing is read."""
+    print(f"case null operands K={K} O={O}", flush=True)
+    out = torch.full((3, 70, 2, O), 7.0, dtype=torch.float16, device="cuda")
+    rc = _kernels.load().aitamd_bmm_softmax_bmm_permute(0, None, None, None, out.data_ptr(), 6, 70, 0, K, O, 2, 0.1, 0,
+                                                        torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert float(out.abs().max()) == 0.0
+
+
 def _check_mem_eff(batch, heads, S, Skv, d, dv, lens, causal=False, dtype=torch.float16, seed=0, lens_q=None):
     print(f"case mem_eff_attention batch={batch} heads={heads} S={S} Skv={Skv} d={d} dv={dv} lens={lens} "
           f"causal={causal} {dtype}", flush=True)
