@@ -22,10 +22,10 @@ namespace aitamd {
 
 GemmAlgoTable gemm_table(int epilogue, int dtype) {
 #define AITAMD_TABLE(E, D) \
-  if (epilogue == E && dtype == D) return &aitamd_gemm_table_##E##_##D ? aitamd_gemm_table_##E##_##D() : GemmAlgoTable{nullptr, 0};
+  if (epilogue == E && dtype == D) return &aitamd_gemm_table_##E##_##D ? aitamd_gemm_table_##E##_##D() : GemmAlgoTable{nullptr, 0, 0};
 #include "gemm_tables.inc"
 #undef AITAMD_TABLE
-  return {nullptr, 0};
+  return {nullptr, 0, 0};
 }
 
 namespace {
@@ -90,8 +90,14 @@ int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64
     if (a.kvec == 2 && (a.direct_lds & 21) != 0 && align_bytes >= 16 && K % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0) continue;
     if (a.kvec == 1 && a.direct_lds == 8 && align_bytes >= 4 && K % 2 == 0 && lda % 2 == 0 && ldb % 2 == 0) continue;
     if (a.direct_lds == 16 && !(plain_store && N % 8 == 0 && four_waves_multiply(a.kvec, K))) continue;
+    const int64_t whole = ((M + a.bm - 1) / a.bm) * ((N + a.bn - 1) / a.bn) * batches;
+    // 128 x 128 through registers on sixteen waves has a CU to itself, its twin on eight shares one with a second workgroup,
+    // which goes on while the first waits for its residuals or gathers a transposed B.  Over 2000 problems of odd K and layouts
+    // that only these take, eight waves to sixteen: 1.04 to 1.12 the time up to one tile per CU; beyond that 1.00 to 1.04, but
+    // 0.82 to 0.95 with residuals and 0.8 to 0.86 with B [K, N] (0.98 with both operands transposed).
+    if (a.direct_lds == 0 && a.threads == 1024 && a.bm == 128 && whole > kNumCu && (t.residuals > 0 || (layout & 1))) continue;
     int64_t slabs = ((a.kvec == 2 && a.direct_lds != 8 ? K & ~7ll : K) + a.bk - 1) / a.bk;
-    int64_t tiles = ((M + a.bm - 1) / a.bm) * ((N + a.bn - 1) / a.bn) * batches;
+    int64_t tiles = whole;
     double cost = a.cost.start;
     if (a.direct_lds == 4) {
       // split-K: usable with scratch memory, and worth a table entry of its own only where it does split (it is

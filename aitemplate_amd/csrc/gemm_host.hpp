@@ -33,6 +33,7 @@ struct GemmAlgo {
 struct GemmAlgoTable {
   const GemmAlgo* algos;
   int count;
+  int residuals;  // operands of the result's size that the epilogue reads
 };
 
 // What the four-wave kernels store with their one epilogue: plain rows of whole 8-column pieces through buffer accesses.

@@ -361,5 +361,5 @@ const GemmAlgo kAlgos[] = {
 #define AITAMD_TABLE_SYM(e, d) AITAMD_CAT3(aitamd_gemm_table_, e, d)
 
 extern "C" __attribute__((visibility("hidden"))) aitamd::GemmAlgoTable AITAMD_TABLE_SYM(AITAMD_EPI, AITAMD_DT)() {
-  return {aitamd::kAlgos, (int)(sizeof(aitamd::kAlgos) / sizeof(aitamd::kAlgos[0]))};
+  return {aitamd::kAlgos, (int)(sizeof(aitamd::kAlgos) / sizeof(aitamd::kAlgos[0])), aitamd::Epi::kNumD};
 }

@@ -1,0 +1,25 @@
+"""What the library takes for a product when nothing was timed (heuristic, csrc/gemm_api.hip).  Without a device it reckons for
+256 CUs."""
+import pytest
+
+from aitemplate_amd import _kernels
+
+
+def _choice(epi, layout, batch, M, N, K, align):
+    lda, ldb = (M if layout & 2 else K), (N if layout & 1 else K)
+    algo = _kernels.load().aitamd_gemm_heuristic_algo_layout(epi, 0, layout, batch, M, N, K, lda, ldb, align)
+    assert algo >= 0
+    return _kernels.gemm_algo_names(epi, 0)[algo]
+
+
+@pytest.mark.parametrize("epi,layout,batch,M,N,K", [
+    (4, 0, 1, 6029, 3143, 3123), (5, 0, 1, 6674, 1079, 1091), (4, 0, 1, 5796, 2898, 511), (0, 1, 19, 536, 553, 995),
+    (0, 1, 59, 452, 219, 109), (17, 1, 59, 452, 219, 109)])
+def test_sixteen_waves_through_registers_only_with_a_cu_for_every_tile(epi, layout, batch, M, N, K):
+    """A grid of more 128 x 128 tiles than CUs whose epilogue or operands a second workgroup per CU hides."""
+    assert "128x128x64_w4x4_reg2" not in _choice(epi, layout, batch, M, N, K, 2)
+
+
+@pytest.mark.parametrize("epi,layout,batch,M,N,K", [(4, 0, 1, 1900, 2039, 2049), (1, 0, 1, 1900, 2039, 2049)])
+def test_sixteen_waves_through_registers_with_a_cu_for_every_tile(epi, layout, batch, M, N, K):
+    assert "128x128x64_w4x4_reg2" in _choice(epi, layout, batch, M, N, K, 2)
