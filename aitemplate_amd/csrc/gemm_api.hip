@@ -127,6 +127,11 @@ int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64
     cost += work > memory_us ? work + 0.3 * memory_us : memory_us + 0.3 * work;
     // (between near equals not the four-wave kernel, which has one wave per SIMD for an epilogue; the fits are of a bias alone)
     if (a.direct_lds == 16) cost *= 1.06;
+    // 256 x 256 through registers has one workgroup per CU and two slabs on their way: with K-contiguous rows at any element and
+    // up to eight slabs a tile is mostly its fill and its store.  Over 300 problems of odd K it takes 1.04 to 1.2 times the better
+    // 128 x 128 form's time there (2 to 8 slabs, 128 to 1024 tiles; 0.80 to 0.93 with more slabs), which its figures, fitted over
+    // all K and layouts, do not say; transposed operands come in whole rows: 0.86 to 1.0.
+    if (a.direct_lds == 0 && a.bm == 256 && layout == 0 && K <= 512) cost *= 1.14;
     if (best < 0 || cost < best_cost) {
       best = i;
       best_cost = cost;

@@ -23,3 +23,14 @@ def test_sixteen_waves_through_registers_only_with_a_cu_for_every_tile(epi, layo
 @pytest.mark.parametrize("epi,layout,batch,M,N,K", [(4, 0, 1, 1900, 2039, 2049), (1, 0, 1, 1900, 2039, 2049)])
 def test_sixteen_waves_through_registers_with_a_cu_for_every_tile(epi, layout, batch, M, N, K):
     assert "128x128x64_w4x4_reg2" in _choice(epi, layout, batch, M, N, K, 2)
+
+
+@pytest.mark.parametrize("M,N,K", [(9419, 1124, 115), (9737, 3454, 217), (5900, 1527, 105), (6592, 1286, 76)])
+def test_no_large_tiles_through_registers_for_few_slabs(M, N, K):
+    """The fill and the store of a 256 x 256 tile have nothing beside them."""
+    assert "256x256x64_w4x4_reg2" not in _choice(1, 0, 1, M, N, K, 4 if K % 2 == 0 else 2)
+
+
+@pytest.mark.parametrize("M,N,K", [(8192, 4097, 2049), (4096, 4095, 6001)])
+def test_large_tiles_through_registers_for_many_slabs(M, N, K):
+    assert "256x256x64_w4x4_reg2" in _choice(1, 0, 1, M, N, K, 2)
