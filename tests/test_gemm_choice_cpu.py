@@ -34,3 +34,14 @@ def test_no_large_tiles_through_registers_for_few_slabs(M, N, K):
 @pytest.mark.parametrize("M,N,K", [(8192, 4097, 2049), (4096, 4095, 6001)])
 def test_large_tiles_through_registers_for_many_slabs(M, N, K):
     assert "256x256x64_w4x4_reg2" in _choice(1, 0, 1, M, N, K, 2)
+
+
+@pytest.mark.parametrize("M,N,K,align", [(79, 1625, 6950, 4), (1596, 76, 4274, 4), (84, 1192, 2314, 4), (51, 1389, 7242, 4)])
+def test_few_outputs_kernel_not_for_several_tiles_per_cu(M, N, K, align):
+    """16 x 16 tiles of more than a few hundred fetch every row of the operands many times over."""
+    assert "rows16x16" not in _choice(1, 0, 1, M, N, K, align)
+
+
+@pytest.mark.parametrize("M,N,K,align", [(1, 768, 768, 16), (1, 6912, 8314, 4), (8, 4096, 4096, 16), (16, 1001, 3001, 2)])
+def test_few_outputs_kernel_for_one_tile_of_rows(M, N, K, align):
+    assert "rows16x16" in _choice(1, 0, 1, M, N, K, align)
