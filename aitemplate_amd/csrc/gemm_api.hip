@@ -131,7 +131,8 @@ int heuristic(const GemmAlgoTable& t, int64_t batch, int64_t M, int64_t N, int64
     // up to eight slabs a tile is mostly its fill and its store.  Over 300 problems of odd K it takes 1.04 to 1.2 times the better
     // 128 x 128 form's time there (2 to 8 slabs, 128 to 1024 tiles; 0.80 to 0.93 with more slabs), which its figures, fitted over
     // all K and layouts, do not say; transposed operands come in whole rows: 0.86 to 1.0.
-    if (a.direct_lds == 0 && a.bm == 256 && layout == 0 && K <= 512) cost *= 1.14;
+    // (more than four rounds of tiles: 0.97 to 1.04, by the figures)
+    if (a.direct_lds == 0 && a.bm == 256 && layout == 0 && K <= 512 && whole <= 4 * kNumCu) cost *= 1.14;
     if (best < 0 || cost < best_cost) {
       best = i;
       best_cost = cost;

@@ -36,6 +36,10 @@ def test_large_tiles_through_registers_for_many_slabs(M, N, K):
     assert "256x256x64_w4x4_reg2" in _choice(1, 0, 1, M, N, K, 2)
 
 
+def test_large_tiles_through_registers_for_many_rounds():
+    assert "256x256x64_w4x4_reg2" in _choice(0, 0, 321, 684, 403, 42, 4)
+
+
 @pytest.mark.parametrize("M,N,K,align", [(79, 1625, 6950, 4), (1596, 76, 4274, 4), (84, 1192, 2314, 4), (51, 1389, 7242, 4)])
 def test_few_outputs_kernel_not_for_several_tiles_per_cu(M, N, K, align):
     """16 x 16 tiles of more than a few hundred fetch every row of the operands many times over."""
