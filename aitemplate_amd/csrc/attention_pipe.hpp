@@ -414,7 +414,15 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) attention_pipe_kernel(con
     // 16-byte pieces instead of 8 bytes of 64 rows at a time
     if (grp == 0) {
       T* const strip = reinterpret_cast<T*>(smem_raw) + wave * 32 * Tile::O_PITCH;
-      T* const ob = reinterpret_cast<T*>(p.out) + ((int64_t)seq * p.M * p.G + (b - seq * p.G)) * p.O;
+      // The arguments of the store are fetched here and not held over the loop, which has no registers for them: held, they and
+      // by_heads had 18 scalar and 6 vector registers spilled at head dim 64 with four workgroups per CU (3 and 5 where by_heads
+      // was no argument), 4 and none so.  us, held -> fetched: 64 x 12 x 384^2, d 64, mixed lengths 32.3 -> 29.6, 64 x 12 x 512^2
+      // 73.2 -> 69.9, 4 x 8 x 2048^2, d 80 57.1 -> 55.4.  Held are M and O with four workgroups per CU (fetched: 9 vector registers)
+      // and all at head dims to 128 (2 x 16 x 4096^2 277.2, fetched 278.6).
+      const AttnParams& w = KS == 8 ? p : arguments_anew<AttnParams>();
+      const AttnParams& extent = Tile::OCC >= 4 ? p : w;
+      const int out_seq = quotient(b, w.by_heads);
+      T* const ob = reinterpret_cast<T*>(w.out) + ((int64_t)out_seq * w.M * w.G + (b - out_seq * w.G)) * w.O;
 #pragma unroll
       for (int qb = 0; qb < QB; ++qb) {
         const int q_row = w0 + qb * 32 + r32;
@@ -437,8 +445,8 @@ __global__ void __launch_bounds__(Tile::NT, Tile::OCC) attention_pipe_kernel(con
         for (int i = 0; i < OC / 2; ++i) {
           const int idx = i * 64 + lane, row = idx / OC, ch = idx - row * OC;
           const int m = w0 + qb * 32 + row;
-          if (m < p.M && ch * 8 < p.O)
-            store_vec(ob + (int64_t)m * p.G * p.O + ch * 8, *reinterpret_cast<const vec8*>(strip + row * Tile::O_PITCH + ch * 8));
+          if (m < extent.M && ch * 8 < extent.O)
+            store_vec(ob + (int64_t)m * w.G * w.O + ch * 8, *reinterpret_cast<const vec8*>(strip + row * Tile::O_PITCH + ch * 8));
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();

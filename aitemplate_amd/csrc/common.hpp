@@ -175,4 +175,15 @@ static_assert(divides_right(1) && divides_right(2) && divides_right(3) && divide
               divides_right(65535) && divides_right(65536) && divides_right(65537) && divides_right(0x3fffffff) &&
               divides_right(0x40000000) && divides_right(0x40000001) && divides_right(0x7ffffffe) && divides_right(0x7fffffff));
 
+// The arguments of a kernel whose one parameter is a P, as memory that nothing is known of: what is read through this is
+// fetched where it is used.  The compiler fetches an argument at the kernel's start and holds it in registers to its last
+// use; where that is behind a long loop, it stands in the loop's way, and what does not fit is spilled.
+template <class P>
+AITAMD_DEVICE const P& arguments_anew() {
+  typedef const __attribute__((address_space(4))) P* scalar_ptr;
+  uintptr_t at = (uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(at));
+  return *(const P*)(scalar_ptr)at;
+}
+
 }  // namespace aitamd
