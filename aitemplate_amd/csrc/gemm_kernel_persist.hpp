@@ -450,6 +450,12 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_persist_kernel(const Gem
         epilogue_fast(c, std::integral_constant<int, 0>{});
       return;
     }
+    // The permuted store's thirteen arguments (the reciprocals of its divisors among them): 320 rows, which have no registers
+    // left, fetch them anew.  Held over the K loop they spill 260 bytes a lane, and 248 for short K (232 and 152 where nothing
+    // but the divisors was held), fetched 152 and 76.  us, held -> fetched: 24576 x 2304 x 768, m3n2 125.5 -> 117.2, x 96
+    // 104.0 -> 83.6, 24576 x 768 x 3072 130.8 -> 128.1.  The other tiles hold them: fetched, 24576 x 2304 x 768 on 256 rows takes
+    // 110.1 for 106.2, 12608 x 3072 x 1024 on 224 rows 96.5 for 92.7.
+    const GemmParams& perm = PERM && XTRA > 0 ? arguments_anew<GemmParams>() : p;
     T* Cb = reinterpret_cast<T*>(p.c) + out_batch_offset(p, c.batch);
     const __amdgpu_buffer_rsrc_t rc = make_rsrc(Cb, kStoreRecords);
     const T* D0b = Epi::kNumD >= 1 ? reinterpret_cast<const T*>(p.d0) + (int64_t)c.batch * p.sd : nullptr;
@@ -477,7 +483,7 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_persist_kernel(const Gem
             *reinterpret_cast<const vec8*>(strip + row * Tile::STRIP_PITCH + ((r_c ^ (row & (SC - 1))) << 4));
         const int m = c.m0 + wm * Tile::WTM + sb * SB + row;
         if (m < p.M && n < p.N) {
-          const int64_t c_idx = out_index<PERM>(p, m, n);
+          const int64_t c_idx = out_index<PERM>(perm, m, n);
           const int64_t d_idx = (int64_t)m * p.ldd + n;
           if (vec_ok && n + 8 <= p.N) {
             vec8 d0v = {}, d1v = {};
@@ -496,7 +502,7 @@ __global__ void __launch_bounds__(Tile::NT, 1) gemm_rcr_persist_kernel(const Gem
                 if constexpr (Epi::kHasBias) bj = Tr::to_float(bias[n + j]);
                 if constexpr (Epi::kNumD >= 1) d0j = Tr::to_float(D0b[d_idx + j]);
                 if constexpr (Epi::kNumD >= 2) d1j = Tr::to_float(D1b[d_idx + j]);
-                Cb[out_index<PERM>(p, m, n + j)] = Tr::from_float(Epi::apply(Tr::to_float(raw[j]), bj, d0j, d1j));
+                Cb[out_index<PERM>(perm, m, n + j)] = Tr::from_float(Epi::apply(Tr::to_float(raw[j]), bj, d0j, d1j));
               }
             }
           }

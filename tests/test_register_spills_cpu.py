@@ -1,6 +1,6 @@
 """Registers that the compiled kernels spill: an argument held in registers over a kernel's main loop, for a use behind it, is
 paid for with lane writes and scratch memory around the loop.  The limits are what the kernels had before their coordinates
-came from reciprocals, which are arguments too."""
+came from reciprocals, which are arguments too (320 rows: in scratch memory and vector registers)."""
 import os
 import re
 import subprocess
@@ -12,6 +12,8 @@ from aitemplate_amd import _kernels
 LLVM = os.environ.get("ROCM_LLVM_BIN", "/opt/rocm/llvm/bin")
 TYPES = r"(?:DF16_|DF16b)"
 ATTENTION = r"_ZN6aitamd21attention_pipe_kernelI" + TYPES + r"NS_8AttnPipeI{0}EEEEvNS_10AttnParamsE"
+PERSISTENT = r"_ZN6aitamd23gemm_rcr_persist_kernelI" + TYPES + r"NS_15GemmTilePersistI{0}EEENS_8EpilogueILi{1}EEE{2}EEvNS_10GemmParamsE"
+ROWS_320 = "Li320ELi256ELi32ELi2ELi4ELi4ELi16ELi320ELi0"
 
 # kernels (regular expression), and the most scratch bytes, scalar and vector registers that one of them may spill
 LIMITS = [
@@ -21,6 +23,9 @@ LIMITS = [
     pytest.param(ATTENTION.format("Li4ELi2ELi2ELi4ELi1ELi2ELi1ELi2E"), 0, 4, 0, id="attention-d64-groups"),
     pytest.param(ATTENTION.format("Li4ELi2ELi1ELi4ELi2ELi1ELi1ELi2E"), 0, 11, 0, id="attention-d64-rows256"),
     pytest.param(ATTENTION.format("Li4ELi2ELi1ELi2ELi1ELi1ELi1ELi2E"), 0, 12, 0, id="attention-d64-rows64"),
+    # 320 x 256, permuted store: K of fewer slabs than the ring has, and more
+    pytest.param(PERSISTENT.format(ROWS_320, "[01]", "Lb1ELb1E"), 152, 44, 45, id="gemm-320-rows-permuted-short-k"),
+    pytest.param(PERSISTENT.format(ROWS_320, "[01]", "Lb1ELb0E"), 232, 41, 57, id="gemm-320-rows-permuted"),
 ]
 
 
