@@ -239,7 +239,7 @@ hipError_t launch_tile(const GemmParams& p, hipStream_t stream) {
     // Asked for by name with others: an instance that takes the same operands, any K and any output.  For a permuted store
     // the one of the same matrix instructions, whose results are those of the plain store.
     if (multiplies && p.perm_on) return launch_tile<GemmTileDma<32, 32, 128, 2, 2, 4, 2, 0, 16, 0, Tile::KTAIL != 0 ? 2 : 0>>(p, stream);
-    using Other = std::conditional_t<Tile::KTAIL != 0, GemmTileDma<128, 128, 64, 4, 4, 4, 4, 0, 32, 0, 2>,
+    using Other = std::conditional_t<Tile::KTAIL != 0, GemmTileDma<128, 128, 64, 2, 4, 4, 1, 1, 32, 0, 2>,
                                      GemmTilePersist<256, 256, 32, 2, 4, 4, 16, 256>>;
     return launch_tile<Other>(p, stream);
   } else {

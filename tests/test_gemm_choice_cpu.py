@@ -49,3 +49,10 @@ def test_few_outputs_kernel_not_for_several_tiles_per_cu(M, N, K, align):
 @pytest.mark.parametrize("M,N,K,align", [(1, 768, 768, 16), (1, 6912, 8314, 4), (8, 4096, 4096, 16), (16, 1001, 3001, 2)])
 def test_few_outputs_kernel_for_one_tile_of_rows(M, N, K, align):
     assert "rows16x16" in _choice(1, 0, 1, M, N, K, align)
+
+
+@pytest.mark.parametrize("M,N,K,align", [(2048, 2048, 2048, 16), (2164, 1592, 864, 16), (3785, 856, 4576, 16),
+                                         (1511, 2456, 3378, 4)])
+def test_a_ring_of_128_x_128_runs_on_eight_waves(M, N, K, align):
+    """One 128 x 128 tile per CU at most: sixteen waves take up to 1.06 times as long."""
+    assert "128x128x64_w2x4_dma4" in _choice(1, 0, 1, M, N, K, align)
