@@ -7,7 +7,8 @@
 //    fetches, so the ds_read side stays bank-conflict free.
 //  * NS slabs are resident: the slab for step k+NS-1 is issued while step k is
 //    multiplied, and one s_waitcnt vmcnt + one barrier per step orders them.
-//    The last NS-1 steps request nothing, and wait for ever fewer loads: a slab
+//    (Direct to LDS.  Slabs through registers are asked for past the end of K as
+//    before.)  The last NS-1 steps request nothing, and wait for ever fewer loads: a slab
 //    past the end of K, all of it out of range, takes as long on its way to LDS as
 //    any other (0.11 us for 16 KiB), and there were NS-1 of them in every tile's
 //    time.  us before -> now: 70 x 1024 x 256 2.93 -> 2.77, 312 x 768 x 256
