@@ -62,8 +62,8 @@ inline double split_k_exchange_us(int64_t tiles, int64_t s, int64_t tile_elems) 
 // instance that is never ahead of the others, for those who name it.)  Whether to split at all is the choice of the instance.  1.5 % (64 x 64 tiles) and 2.0 %
 // (128 x 128) above the best number in the geometric mean; as many as fill the CUs, the rule before, 8 % and 21 %:
 // 21 x 512 x 2048 11.5 us with 16, 7.1 with 4; 200 x 2304 x 768 in 128 x 128 tiles 17.4 with 6, 13.1 with 2.
-// (128 x 128: measured on eight waves, the 0.395 us of a slab too.  On sixteen, which came after, a product takes 1.05 times
-// less time in the mean with the numbers of this rule, which were not timed against others again.)
+// (128 x 128: measured on eight waves, the 0.395 us of a slab too.  On sixteen, which came after and take 0.96 to 1.03 times the
+// time with the numbers of this rule, other numbers were not timed again.)
 inline int split_k_rule(int64_t tiles, int64_t k_tiles, int bk, int64_t tile_elems, int cus) {
   if (tiles <= 0) return 1;
   if (bk < 64) {
